@@ -320,12 +320,13 @@ bool fit_atan(double zmax, int nc, float *coef);
 // s, the table holds kRampSkew = 8 copies shifted by one tap each:
 //     table[pl][r][u] = plane pl (hi, lo, ll) of h[u - r + dlo],   u < lg,
 // zero where |u - r + dlo| > nC - 1; h[s .. s + 7] is row r = (-s) mod 8 from u = s - dlo + r
-// (a multiple of 8).  dlo = -(np + 8) and lg = np + kp + 64 cover every offset an np x kp
-// tiling reads, with the slack of the 8-aligned windows.
+// (a multiple of 8).  dlo = -(np + 8) and lg = np + kp + 160 cover every offset an np x kp
+// tiling reads, with the slack of the 8-aligned windows and of K steps of up to 128 (kp is
+// a multiple of 32).
 constexpr int kRampSkew = 8;
 constexpr int kRampTileN = 256;  // np: a multiple of the widest column tile of the filter
 constexpr int ramp_table_dlo(int np) { return -(np + 8); }
-constexpr int ramp_table_len(int np, int kp) { return np + kp + 64; }
+constexpr int ramp_table_len(int np, int kp) { return np + kp + 160; }
 void ramp_tap_table(const std::vector<double> &taps, int nC, int np, int kp, std::vector<uint16_t> &table, int &lg);
 
 // hipMalloc + copy of a host vector (at least one element is allocated).

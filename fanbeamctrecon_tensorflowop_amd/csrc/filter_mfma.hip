@@ -12,12 +12,11 @@
 // registers as it is loaded (optionally multiplied by a per-sample weight first, the
 // cone-beam pre-weight; a BF16 input needs no split).
 //
-// Tiling: a workgroup of 4 waves computes 128 rows x 128 (or 256) columns; per K step of 32 it
+// Tiling: a workgroup of 4 waves computes a tile of rows x columns; per K step it
 // stages the BF16 planes of its P rows (split once per element) and the window of split
 // taps its H columns read (H is Toeplitz and symmetric: the B fragment of column c at k is
 // h[k - c .. k - c + 7], read from skewed copies of the taps so that every fragment is one
-// aligned 16-byte LDS read) in LDS, and each wave multiplies its part, 64 rows x 64 (or
-// 128) columns of 16 x 16 MFMA tiles.
+// aligned 16-byte LDS read) in LDS, and each wave multiplies its part in 16 x 16 MFMA tiles.
 // Lane layout of v_mfma_f32_16x16x32_bf16: A lane l holds row l%16, k = 8*(l/16)+j;
 // B lane l holds column l%16, k = 8*(l/16)+j; D lane l holds rows 4*(l/16)+j, column l%16.
 
@@ -54,47 +53,57 @@ __device__ __forceinline__ void split3(float x, __bf16 &hi, __bf16 &lo, __bf16 &
 __device__ __forceinline__ float widen(float x) { return x; }
 __device__ __forceinline__ float widen(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
 
-// A workgroup (4 waves) computes 128 rows x BN columns; per K step of 32 it stages the
-// BF16 planes of its P rows (split once per element, weights applied first) and the tap
-// window of its H columns in LDS, then each wave multiplies its 64 x BN/2 part from LDS.
-// Rows of the P planes are padded to 40 BF16 so the 16 rows a fragment read touches fall
-// in distinct banks.
-constexpr int kBM = 128, kBK = 32, kKS = 40;
+// 16 consecutive elements of a row, at the alignment of an element: rows of any length and
+// base take 16-byte loads (a row length that is no multiple of 16 bytes took scalar loads
+// before: 300 columns of BF16, 17280 rows, 55 us, now 33 us).
+template <typename TI>
+struct __attribute__((packed, aligned(sizeof(TI)))) Run {
+    TI v[16];
+};
 
-// BN output columns per workgroup (128 or 256; each wave takes BN / 2 of them, NT tiles of
-// 16).  Staged taps per plane and copy and K step: the fragments of a K step reach offsets
-// s in [k0 - c0 - BN + 1, k0 - c0 + 31], plus 7 for the copies' shift and 7 for the
-// window's 8-alignment: BN + 48 BF16 per row, 88 or 152 dwords (an odd multiple of 8, so
-// the 16 lanes of a fragment read, 8 copies x 2 windows 16 bytes apart, fall in distinct
-// bank groups).
-template <typename TI, bool kW, int BN>
-__global__ __launch_bounds__(256) void ramp_gemm_kernel(MfmaArgs A)
+constexpr int kGemmThreads = 256;
+
+// A workgroup (4 waves) computes BM rows x BN columns; per K step of BK it stages the BF16
+// planes of its P rows (split once per element, weights applied first; 16 consecutive values
+// per thread) and the tap window of its H columns in LDS, then each wave multiplies its part
+// (MT x NT tiles of 16 x 16) from LDS.  Rows of the P planes are padded by 8 BF16, so the 16
+// rows a fragment read touches start in distinct bank groups.  Staged taps per plane and
+// copy and K step: the fragments reach offsets s in [k0 - c0 - BN + 1, k0 - c0 + BK - 1], plus
+// 7 for the copies' shift and 7 for the window's 8-alignment: BN + BK + 16 BF16 per row, an
+// odd multiple of 8 dwords (so the 16 lanes of a fragment read, 8 copies x 2 windows 16 bytes
+// apart, fall in distinct bank groups).
+//
+// What bounds it: a workgroup's K steps are a serial chain of load, split, barrier, multiply,
+// barrier (about 3.5 us a step at two waves per SIMD), hidden only by other workgroups.  Three
+// tile shapes, see launch_ramp_gemm.
+template <typename TI, bool kW, int BM, int BN, int BK>
+__global__ __launch_bounds__(kGemmThreads) void ramp_gemm_kernel(MfmaArgs A)
 {
-    constexpr int kTW = BN + 48, NT = BN / 32;
+    constexpr int kTW = BN + BK + 16;
+    constexpr int kKS = BK + 8;                        // BF16 per staged P row
+    constexpr int WR = BM >= 128 ? 2 : 1, WC = 4 / WR;  // waves along rows and columns
+    constexpr int MT = BM / WR / 16, NT = BN / WC / 16;  // 16 x 16 tiles per wave
+    static_assert(BM * BK == 16 * kGemmThreads, "a thread stages 16 values of one row");
     static_assert((kTW / 2 / 8) % 2 == 1, "tap rows an odd multiple of 8 dwords");
     constexpr bool kExactA = sizeof(TI) == 2 && !kW;
     constexpr int kPA = kExactA ? 1 : 3;  // A planes in use
-    __shared__ __bf16 As[kPA][kBM][kKS];
+    __shared__ __bf16 As[kPA][BM][kKS];
     __shared__ __bf16 Ts[3][kRampSkew][kTW];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wr = wave >> 1, wc = wave & 1;
+    const int wr = wave / WC, wc = wave % WC;
     // each XCD takes whole row tiles, their column tiles consecutive (P rows stay in its L2)
     const unsigned lblk = xcd_block(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
-    const long long r0 = (long long)(lblk / gridDim.y) * kBM;
+    const long long r0 = (long long)(lblk / gridDim.y) * BM;
     const int c0 = (int)(lblk % gridDim.y) * BN;
-    // staging assignment: thread -> (row or column tid / 2, 16 k-values at kh)
-    const int srow = tid >> 1, kh = (tid & 1) * 16;
-    const long long arow = r0 + srow;
-    const bool arow_ok = arow < A.rows;
-    const TI *prow = static_cast<const TI *>(A.in) + (arow_ok ? arow : 0) * (long long)A.nC;
-    const float *wrow = kW && A.w ? A.w + (arow_ok ? arow % A.wrows : 0) * (long long)A.nC : nullptr;
+    // staging assignment: thread -> (row, 16 k-values at kh)
+    const int srow = tid / (BK / 16), kh = tid % (BK / 16) * 16;
+    const bool arow_ok = r0 + srow < A.rows;
+    const long long arow = arow_ok ? r0 + srow : 0;
+    const TI *prow = static_cast<const TI *>(A.in) + arow * (long long)A.nC;
+    const float *wrow = kW && A.w ? A.w + arow % A.wrows * (long long)A.nC : nullptr;
     const float *w2row =
-        kW && A.w2 ? A.w2 + (arow_ok ? (arow / A.w2div) % A.w2rows : 0) * (long long)A.nC : nullptr;
-    const bool vec = ((size_t)A.nC * sizeof(TI)) % 16 == 0 && reinterpret_cast<uintptr_t>(A.in) % 16 == 0;
-    // weight rows 16-byte aligned (FP32 rows of nC, bases from the allocator)
-    const bool wvec = A.nC % 4 == 0 && reinterpret_cast<uintptr_t>(A.w) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(A.w2) % 16 == 0;
+        kW && A.w2 ? A.w2 + (arow / A.w2div) % A.w2rows * (long long)A.nC : nullptr;
     // B from the tap table: per K step the window of kTW taps (each plane, each skewed
     // copy) from which column c of H reads h[k0 + k - c], k < 32; the window starts at
     // u0 + k0, and each lane's B fragment of tile t sits at a fixed offset in it
@@ -104,41 +113,26 @@ __global__ __launch_bounds__(256) void ramp_gemm_kernel(MfmaArgs A)
     int boff[NT];  // Ts element offset of the fragment h[s .. s + 7], s = k0 + fk - c
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-        const int s0 = fk - (c0 + wc * (BN / 2) + 16 * t + fr);  // s at k0 = 0
+        const int s0 = fk - (c0 + wc * (BN / WC) + 16 * t + fr);  // s at k0 = 0
         const int r = (-s0) & (kRampSkew - 1);               // copy whose row holds it aligned
         boff[t] = r * kTW + (s0 - dlo + r - u0);             // in [0, kTW - 8], a multiple of 8
     }
 
-    f32x4 acc[4][NT];
+    f32x4 acc[MT][NT];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int t = 0; t < NT; ++t) acc[i][t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 
-    for (int k0 = 0; k0 < A.Kp; k0 += kBK) {
+    for (int k0 = 0; k0 < A.Kp; k0 += BK) {
         // ---- stage A: 16 consecutive k of one row, weighted and split
         {
             float x[16];
             const int kb = k0 + kh;
-            if (vec && arow_ok && kb + 16 <= A.nC) {
-                if constexpr (sizeof(TI) == 4) {
+            if (arow_ok && kb + 16 <= A.nC) {
+                const Run<TI> u = *reinterpret_cast<const Run<TI> *>(prow + kb);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float4 u = *reinterpret_cast<const float4 *>(prow + kb + 4 * q);
-                        x[4 * q] = u.x, x[4 * q + 1] = u.y, x[4 * q + 2] = u.z, x[4 * q + 3] = u.w;
-                    }
-                } else {
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        const uint4 u = *reinterpret_cast<const uint4 *>(prow + kb + 8 * q);
-                        const uint32_t d[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            x[8 * q + 2 * j] = __uint_as_float(d[j] << 16);
-                            x[8 * q + 2 * j + 1] = __uint_as_float(d[j] & 0xffff0000u);
-                        }
-                    }
-                }
+                for (int j = 0; j < 16; ++j) x[j] = widen(u.v[j]);
             } else {
 #pragma unroll
                 for (int j = 0; j < 16; ++j) x[j] = (arow_ok && kb + j < A.nC) ? widen(prow[kb + j]) : 0.0f;
@@ -149,23 +143,19 @@ __global__ __launch_bounds__(256) void ramp_gemm_kernel(MfmaArgs A)
 #pragma unroll
             for (int j = 0; j < 16; ++j) wt[j] = 1.0f;
             if constexpr (kW) {
-                if (wvec && arow_ok && kb + 16 <= A.nC) {
+                if (arow_ok && kb + 16 <= A.nC) {
                     // 16-byte loads: a wave's scalar weight loads each touch 32 rows' cache
                     // lines, and 16 of them per step bound the kernel by its memory
                     // instruction rate
                     if (wrow) {
+                        const Run<float> u = *reinterpret_cast<const Run<float> *>(wrow + kb);
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const float4 u = *reinterpret_cast<const float4 *>(wrow + kb + 4 * q);
-                            wt[4 * q] *= u.x, wt[4 * q + 1] *= u.y, wt[4 * q + 2] *= u.z, wt[4 * q + 3] *= u.w;
-                        }
+                        for (int j = 0; j < 16; ++j) wt[j] *= u.v[j];
                     }
                     if (w2row) {
+                        const Run<float> u = *reinterpret_cast<const Run<float> *>(w2row + kb);
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const float4 u = *reinterpret_cast<const float4 *>(w2row + kb + 4 * q);
-                            wt[4 * q] *= u.x, wt[4 * q + 1] *= u.y, wt[4 * q + 2] *= u.z, wt[4 * q + 3] *= u.w;
-                        }
+                        for (int j = 0; j < 16; ++j) wt[j] *= u.v[j];
                     }
                 } else {
 #pragma unroll
@@ -206,32 +196,35 @@ __global__ __launch_bounds__(256) void ramp_gemm_kernel(MfmaArgs A)
         }
         __syncthreads();
 
-        // ---- multiply this wave's 64 x 64 quadrant
-        bf16x8 ah[4], al[4], all[4];
+        // ---- multiply this wave's part, 32 k at a time
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = wr * 64 + 16 * i + fr;
-            ah[i] = *reinterpret_cast<const bf16x8 *>(&As[0][r][fk]);
-            if constexpr (!kExactA) {
-                al[i] = *reinterpret_cast<const bf16x8 *>(&As[1][r][fk]);
-                all[i] = *reinterpret_cast<const bf16x8 *>(&As[2][r][fk]);
-            }
-        }
+        for (int kk = 0; kk < BK; kk += 32) {
+            bf16x8 ah[MT], al[MT], all[MT];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const bf16x8 bh = *reinterpret_cast<const bf16x8 *>(&Ts[0][0][0] + boff[t]);
-            const bf16x8 bl = *reinterpret_cast<const bf16x8 *>(&Ts[1][0][0] + boff[t]);
-            const bf16x8 bll = *reinterpret_cast<const bf16x8 *>(&Ts[2][0][0] + boff[t]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < MT; ++i) {
+                const int r = wr * (BM / WR) + 16 * i + fr;
+                ah[i] = *reinterpret_cast<const bf16x8 *>(&As[0][r][kk + fk]);
                 if constexpr (!kExactA) {
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(all[i], bh, acc[i][t], 0, 0, 0);
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bl, acc[i][t], 0, 0, 0);
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh, acc[i][t], 0, 0, 0);
+                    al[i] = *reinterpret_cast<const bf16x8 *>(&As[1][r][kk + fk]);
+                    all[i] = *reinterpret_cast<const bf16x8 *>(&As[2][r][kk + fk]);
                 }
-                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bll, acc[i][t], 0, 0, 0);
-                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl, acc[i][t], 0, 0, 0);
-                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh, acc[i][t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const bf16x8 bh = *reinterpret_cast<const bf16x8 *>(&Ts[0][0][0] + boff[t] + kk);
+                const bf16x8 bl = *reinterpret_cast<const bf16x8 *>(&Ts[1][0][0] + boff[t] + kk);
+                const bf16x8 bll = *reinterpret_cast<const bf16x8 *>(&Ts[2][0][0] + boff[t] + kk);
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    if constexpr (!kExactA) {
+                        acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(all[i], bh, acc[i][t], 0, 0, 0);
+                        acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bl, acc[i][t], 0, 0, 0);
+                        acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[i], bh, acc[i][t], 0, 0, 0);
+                    }
+                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bll, acc[i][t], 0, 0, 0);
+                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bl, acc[i][t], 0, 0, 0);
+                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[i], bh, acc[i][t], 0, 0, 0);
+                }
             }
         }
         __syncthreads();  // the next K step overwrites the planes
@@ -239,25 +232,26 @@ __global__ __launch_bounds__(256) void ramp_gemm_kernel(MfmaArgs A)
 
     // ---- store: D lane l holds rows 4 (l / 16) + j, column l % 16 of each 16 x 16 tile
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const int col = c0 + wc * (BN / 2) + 16 * t + (lane & 15);
-        if (col >= A.nC) continue;
+    for (int i = 0; i < MT; ++i) {
+        const long long row0 = r0 + wr * (BM / WR) + 16 * i + 4 * (lane >> 4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int t = 0; t < NT; ++t) {
+            const int col = c0 + wc * (BN / WC) + 16 * t + (lane & 15);
+            if (col >= A.nC) continue;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const long long row = r0 + wr * 64 + 16 * i + 4 * (lane >> 4) + j;
-                if (row >= A.rows) continue;
-                A.out[row * A.nC + col] = acc[i][t][j];
-            }
+            for (int j = 0; j < 4; ++j)
+                if (row0 + j < A.rows) A.out[(row0 + j) * A.nC + col] = acc[i][t][j];
+        }
     }
 }
 
 template <typename TI, bool kW>
-void launch_gemm_p(int bn, dim3 grid, hipStream_t stream, const MfmaArgs &A)
+void launch_gemm_p(int bm, dim3 grid, hipStream_t stream, const MfmaArgs &A)
 {
-    if (bn == 256) hipLaunchKernelGGL((ramp_gemm_kernel<TI, kW, 256>), grid, dim3(256), 0, stream, A);
-    else hipLaunchKernelGGL((ramp_gemm_kernel<TI, kW, 128>), grid, dim3(256), 0, stream, A);
+    const dim3 wg(kGemmThreads);
+    if (bm == 32) hipLaunchKernelGGL((ramp_gemm_kernel<TI, kW, 32, 64, 128>), grid, wg, 0, stream, A);
+    else if (bm == 64) hipLaunchKernelGGL((ramp_gemm_kernel<TI, kW, 64, 128, 64>), grid, wg, 0, stream, A);
+    else hipLaunchKernelGGL((ramp_gemm_kernel<TI, kW, 128, 256, 32>), grid, wg, 0, stream, A);
 }
 
 }  // namespace
@@ -283,21 +277,38 @@ fbct_status launch_ramp_gemm(const RampOperand &H, const void *in, fbct_dtype ti
     A.wrows = rw.w ? rw.wrows : 1;
     A.w2div = rw.w2 ? rw.w2div : 1;
     A.w2rows = rw.w2 ? rw.w2rows : 1;
-    if (H.Np % kRampTileN != 0 || H.Np < H.nC || H.Kp % kBK != 0 || H.Kp < H.nC || H.Lg != ramp_table_len(H.Np, H.Kp))
+    if (H.Np % kRampTileN != 0 || H.Np < H.nC || H.Kp % 32 != 0 || H.Kp < H.nC || H.Lg != ramp_table_len(H.Np, H.Kp))
         return fail(FBCT_ERR_UNSUPPORTED, "ramp filter: operand planes not padded to the tile");
-    // 256-column tiles (the input rows are read by half as many workgroups) unless they
-    // pad the columns further than 128-column tiles do
-    const int bn = (H.nC + 255) / 256 * 256 == (H.nC + 127) / 128 * 128 ? 256 : 128;
-    const long long gx = (rows + kBM - 1) / kBM;
+    // Tile shape (rows x columns x K step).  The widest, 128 x 256 x 32, splits each input
+    // element for the fewest workgroups and is the fastest where it pads the columns no further
+    // than 128-wide tiles and leaves enough workgroups (1024 columns: 184320 BF16 rows 1.64 ms
+    // against 1.73 with 64 x 128; 15744 rows 133 against 147 us; but 512 columns, 23040 rows 75
+    // against 63 us).  Else 64 x 128 x 64, half the K steps and twice the workgroups of the
+    // 128 x 128 x 32 tile used before (888 columns, 62976 rows: 447 against 464 us).  With fewer
+    // than about 320 such tiles the chip is not full and the length of a workgroup's chain is
+    // what counts: 32 x 64 x 128 has four times the workgroups and half the K steps (512
+    // columns, 360 rows: 10.7 against 21 us, 55 us before; 888 columns, 1968 rows: 32.7
+    // against 34.8; 3936 rows, 434 tiles: 52.9 against 45.1).
+    const auto cdiv = [](long long a, long long b) { return (a + b - 1) / b; };
+    int bm, bn;
+    const bool wide = H.nC >= 768 && cdiv(H.nC, 256) * 256 == cdiv(H.nC, 128) * 128 &&
+                      cdiv(rows, 128) * cdiv(H.nC, 256) >= 384;
+    if (wide || rows > (1LL << 29))  // (the grid holds fewer than 2^32 threads per axis)
+        bm = 128, bn = 256;
+    else if (cdiv(rows, 64) * cdiv(H.nC, 128) >= 320)
+        bm = 64, bn = 128;
+    else
+        bm = 32, bn = 64;
+    const long long gx = (rows + bm - 1) / bm;
     if (gx > 0x7fffffffLL || gx * ((H.nC + bn - 1) / bn) > 0xffffffffLL)
         return fail(FBCT_ERR_UNSUPPORTED, "ramp filter: too many rows");
-    dim3 grid((unsigned)gx, (H.nC + bn - 1) / bn);
+    const dim3 grid((unsigned)gx, (H.nC + bn - 1) / bn);
     if (ti == FBCT_BF16) {
-        if (w) launch_gemm_p<uint16_t, true>(bn, grid, stream, A);
-        else launch_gemm_p<uint16_t, false>(bn, grid, stream, A);
+        if (w) launch_gemm_p<uint16_t, true>(bm, grid, stream, A);
+        else launch_gemm_p<uint16_t, false>(bm, grid, stream, A);
     } else {
-        if (w) launch_gemm_p<float, true>(bn, grid, stream, A);
-        else launch_gemm_p<float, false>(bn, grid, stream, A);
+        if (w) launch_gemm_p<float, true>(bm, grid, stream, A);
+        else launch_gemm_p<float, false>(bm, grid, stream, A);
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "ramp_gemm_kernel launch: %s", hipGetErrorString(e));
