@@ -5,8 +5,8 @@
 // FBP/transform.cu:61-89 (times 1/(U^2+t^2)), launched once per view with a memcpy
 // and a device sync per view (BP/transform.cu:110-118).
 //
-// Here one launch covers every view and slice: a thread owns a pixel of S slices, loops
-// over all views with the per-view (cos, sin) read as uniform scalars, computes the
+// Here one launch covers every view and a group of slices: a thread owns a pixel of S
+// slices, loops over its views with the per-view (cos, sin) read as uniform scalars, computes the
 // column coordinate, in-range decision, taps and weight once per (pixel, view) and
 // applies them to the S slices, accumulates in registers and stores once.  The detector
 // row is read with two gathers per update; the 1-D texture's clamp-to-edge linear
@@ -42,7 +42,12 @@ struct BpArgs {
     long long img_stride, sino_stride;
     int nX, nY, nViews, nCols;
     float R, xmin, ymin, dx, dy;
-    float xi_scale, xi_offset;
+    float xi_scale;
+    // dShift - dLeft/dCol - 1/2 = ct_col + ct_offset, |ct_offset| <= 1/2: the column coordinate between the
+    // column centres is formed relative to column ct_col (mid-detector as a rule), where its
+    // FP32 rounding is that of the distance from it
+    float ct_offset;
+    int ct_col;
     int edge_exact;
     double tan_min, tan_max;
     float atan_c[kBpAtanMax];  // correction polynomial R(s), s = z^2, lowest order first
@@ -82,17 +87,23 @@ __device__ __forceinline__ float fan_atan(const BpArgs &A, float z)
     }
 }
 
-// Column coordinate xi of the pixel in view v (xi_raw of BP/transform.cu:85), its
-// in-range flag and the FP32 U, t.
+// Column coordinate of the pixel in view v relative to the centre of column ct_col (xi_raw of
+// BP/transform.cu:85 less 1/2 and ct_col), and the FP32 U, t.
 template <int kNc>
-__device__ __forceinline__ bool column_of(const BpArgs &A, const PixelGeo &p, int v, float &xi, float &U, float &t)
+__device__ __forceinline__ float column_of(const BpArgs &A, const PixelGeo &p, int v, float &U, float &t)
 {
     const float2 cs = A.cs[v];
     U = fmaf(-p.y, cs.y, fmaf(-p.x, cs.x, A.R));  // projection onto the iso-ray
     t = fmaf(p.x, cs.y, -p.y * cs.x);             // distance to the centre ray
-    xi = fmaf(fan_atan<kNc>(A, t * __builtin_amdgcn_rcpf(U)), A.xi_scale, A.xi_offset);
-    bool in = xi > 0.0f && xi < (float)A.nCols;
-    if (A.edge_exact && (fabsf(xi) < kEdgeBand || fabsf(xi - (float)A.nCols) < kEdgeBand)) {
+    return fmaf(fan_atan<kNc>(A, t * __builtin_amdgcn_rcpf(U)), A.xi_scale, A.ct_offset);
+}
+
+// The in-range decision 0 < xi < nCols.
+__device__ __forceinline__ bool in_range(const BpArgs &A, const PixelGeo &p, int v, float ct)
+{
+    const float lo = -0.5f - (float)A.ct_col, hi = lo + (float)A.nCols;
+    bool in = ct > lo && ct < hi;
+    if (A.edge_exact && (fabsf(ct - lo) < kEdgeBand || fabsf(ct - hi) < kEdgeBand)) {
         const double2 c = A.csd[v];
         const double Ud = (double)A.R - p.xd * c.x - p.yd * c.y;
         const double td = p.xd * c.y - p.yd * c.x;
@@ -101,14 +112,15 @@ __device__ __forceinline__ bool column_of(const BpArgs &A, const PixelGeo &p, in
     return in;
 }
 
-// Texel-centre linear interpolation position: interpolate at xi - 1/2, clamped to the
-// row; returns the left tap c0 in [0, nCols-2] and the weight of c0+1.
-__device__ __forceinline__ int interp_pos(float xi, int nCols, float &al)
+// Linear interpolation position: ct clamped to the column centres; returns the left tap c0
+// in [0, nCols-2] and the weight of c0+1.
+__device__ __forceinline__ int interp_pos(const BpArgs &A, float ct, float &al)
 {
-    const float ct = fminf(fmaxf(xi - 0.5f, 0.0f), (float)(nCols - 1));
-    const float fc = fminf(floorf(ct), (float)max(nCols - 2, 0));
-    al = ct - fc;
-    return (int)fc;
+    const float first = (float)-A.ct_col;
+    const float cc = fminf(fmaxf(ct, first), first + (float)(A.nCols - 1));
+    const float fc = fminf(floorf(cc), first + (float)max(A.nCols - 2, 0));
+    al = cc - fc;
+    return (int)fc + A.ct_col;
 }
 
 // Weights of the taps c0 and c0 + 1 of one view: (1 - al, al), times the fan-beam
@@ -127,52 +139,140 @@ __device__ __forceinline__ void bp_tap_weights(float al, float U, float t, float
     }
 }
 
-// Slices [slice0 + S*blockIdx.z, +S) of the batch.
-template <bool kWeighted, int S, int kNc>
-__global__ __launch_bounds__(kBpTx *kBpTy) void bp_kernel(BpArgs A, int slice0)
+// Few slices (S = 1..4): a wave owns an 8 x 8 pixel block and reads its taps from global
+// memory, both columns of an update (of all S slices, where they lie interleaved) in one
+// load.  The W waves of a workgroup share the block and split the views (chunks of kBpChunk
+// views dealt round-robin), so a small image still fills the chip; their FP32 partial sums
+// meet in LDS and are added in FP64 in wave order.  A chunk's coordinates are computed together
+// (independent chains, the loads of kBpChunk views in flight); when every active pixel of the
+// wave lies between the centres of the first and the last column in all of them, which one
+// comparison per view decides, the taps need no clamp and the update no in-range test.  Any
+// other chunk takes the general path, view by view.
+//
+// Bound: VALU issue for one slice (about 36 instruction slots per update, a quarter of them two
+// reciprocals; 512 x 512 pixels, 984 views: 177 us, and 284 us for the one-thread-per-pixel loop
+// over all views that this replaces; 256 x 256, 360 views: 147 -> 24 us), for more slices the
+// vector L1, which takes about 20 cycles per gathered load whatever its width: 224 / 327 / 431 us
+// for 2 / 3 / 4 planes, 201 / 256 / 236 us interleaved (one, two and two loads per update).
+constexpr int kBpBlk = 8;    // pixel block side: one pixel per lane
+constexpr int kBpChunk = 4;  // views evaluated together
+
+// taps c0 and c0 + 1 of S interleaved slices, as they lie in memory
+template <int S>
+struct __attribute__((packed, aligned(4))) TapPair {
+    float v[2 * S];
+};
+
+template <bool kWeighted, bool kIl, int S, int kNc, int W>
+__global__ __launch_bounds__(64 * W) void bp_direct_kernel(BpArgs A, int slice0)
 {
-    unsigned t, g;  // XCD-aware (tile, slice group)
-    xcd_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x * gridDim.y, gridDim.z, t, g);
-    const int i = (t % gridDim.x) * kBpTx + threadIdx.x % kBpTx;
-    const int j = (t / gridDim.x) * kBpTy + threadIdx.x / kBpTx;
+    unsigned tbx, tby, g;
+    xcd_blocked_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, gridDim.z,
+                     tbx, tby, g);
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int i = (int)tbx * kBpBlk + (lane & 7), j = (int)tby * kBpBlk + (lane >> 3);
     const size_t sl = (size_t)slice0 + (size_t)S * g;
-    if (i >= A.nX || j >= A.nY) return;
-    const PixelGeo pg = pixel_geo(A, i, j);
+    const PixelGeo pg = pixel_geo(A, min(i, A.nX - 1), min(j, A.nY - 1));
+    const int2 fr = A.fov_row[min(j, A.nY - 1)];
+    const bool valid = i < A.nX && j < A.nY;
+    constexpr int kSl = kIl ? S : 1;       // slices a tap holds
+    constexpr int kPl = kIl ? 1 : S;       // planes read per update
+    const float *sino[kPl];
+#pragma unroll
+    for (int s = 0; s < kPl; ++s) sino[s] = A.sino + (sl + s) * A.sino_stride;
     float acc[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) acc[s] = 0.0f;
-    const int2 fr = A.fov_row[j];
-    if (i >= fr.x && i <= fr.y) {
-        const float *sino = A.sino + sl * A.sino_stride;
-        const int c1max = A.nCols - 1;
-        for (int v = 0; v < A.nViews; ++v) {
-            float xi, U, t;
-            if (!column_of<kNc>(A, pg, v, xi, U, t)) continue;
-            float al;
-            const int c0 = interp_pos(xi, A.nCols, al);
-            const int c1 = min(c0 + 1, c1max);
-            const float *P = sino + (size_t)v * A.nCols;
+    const float mid = 0.5f * (float)(A.nCols - 1), midr = mid - (float)A.ct_col;
+
+    if (valid && i >= fr.x && i <= fr.y) {
+        // one update by the general path
+        auto update = [&](int v) {
+            float U, t, al;
+            const float ct = column_of<kNc>(A, pg, v, U, t);
+            if (!in_range(A, pg, v, ct)) return;
+            const int c0 = interp_pos(A, ct, al);
+            const int c1 = min(c0 + 1, A.nCols - 1);
             float w0, w1;
             bp_tap_weights<kWeighted>(al, U, t, w0, w1);
 #pragma unroll
             for (int s = 0; s < S; ++s) {
-                const float p0 = P[(size_t)s * A.sino_stride + c0];
-                const float p1 = P[(size_t)s * A.sino_stride + c1];
-                acc[s] = fmaf(w1, p1, fmaf(w0, p0, acc[s]));
+                const float *P = sino[s / kSl] + (size_t)v * A.nCols * kSl + s % kSl;
+                acc[s] = fmaf(w1, P[c1 * kSl], fmaf(w0, P[c0 * kSl], acc[s]));
+            }
+        };
+        int v0 = wave * kBpChunk;
+        for (; v0 + kBpChunk <= A.nViews; v0 += W * kBpChunk) {
+            float ct[kBpChunk], U[kBpChunk], t[kBpChunk];
+            bool ok = true;
+#pragma unroll
+            for (int m = 0; m < kBpChunk; ++m) {
+                ct[m] = column_of<kNc>(A, pg, v0 + m, U[m], t[m]);
+                ok = ok && fabsf(ct[m] - midr) < mid - kEdgeBand;
+            }
+            if (__all(ok)) {
+                const size_t row = (size_t)v0 * A.nCols * kSl;
+                TapPair<kSl> p[kBpChunk][kPl];
+                float w0[kBpChunk], w1[kBpChunk];
+#pragma unroll
+                for (int m = 0; m < kBpChunk; ++m) {
+                    const float fc = floorf(ct[m]);
+                    const unsigned off = (unsigned)((int)fc + A.ct_col) * (4u * kSl);
+#pragma unroll
+                    for (int s = 0; s < kPl; ++s)
+                        p[m][s] = load_at(
+                            reinterpret_cast<const TapPair<kSl> *>(sino[s] + row + (size_t)m * A.nCols * kSl), off);
+                    bp_tap_weights<kWeighted>(ct[m] - fc, U[m], t[m], w0[m], w1[m]);
+                }
+#pragma unroll
+                for (int m = 0; m < kBpChunk; ++m)
+#pragma unroll
+                    for (int s = 0; s < S; ++s)
+                        acc[s] = fmaf(w1[m], p[m][s / kSl].v[kSl + s % kSl], fmaf(w0[m], p[m][s / kSl].v[s % kSl], acc[s]));
+            } else {
+                for (int m = 0; m < kBpChunk; ++m) update(v0 + m);
             }
         }
+        for (int v = v0; v < min(v0 + kBpChunk, A.nViews); ++v) update(v);
     }
+
+    if constexpr (W == 1) {
+        if (valid) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) A.img[(sl + s) * A.img_stride + (size_t)j * A.nX + i] = acc[s];
+            for (int s = 0; s < S; ++s) A.img[(sl + s) * A.img_stride + (size_t)j * A.nX + i] = acc[s];
+        }
+    } else {
+        __shared__ float part[W][S][64];
+#pragma unroll
+        for (int s = 0; s < S; ++s) part[wave][s][lane] = acc[s];
+        __syncthreads();
+        // slice s of the block is summed by wave s mod W
+        for (int s = wave; s < S; s += W) {
+            double sum = 0.0;
+#pragma unroll
+            for (int w = 0; w < W; ++w) sum += (double)part[w][s][lane];
+            if (valid) A.img[(sl + s) * A.img_stride + (size_t)j * A.nX + i] = (float)sum;
+        }
+    }
 }
 
-// Staged variant for S = 4, 8, 16 slices: per batch of kBpStageVB views the workgroup
+// Staged variant for S = 8, 16 slices: per batch of kBpStageVB views the workgroup
 // copies the 64 detector columns around its tile into LDS once (coalesced, the S slices
 // of a column contiguous, so a tap of all S slices is S/4 16-byte LDS reads instead of
 // S gathers).  The window of a view starts at the smallest column coordinate of the
 // tile's four corner pixels (t/U, and so xi, is extremal at a corner; lane 4m + c
 // evaluates corner c of view m); a pixel whose taps leave the window reads them from
-// global memory.  Results are those of bp_kernel (same arithmetic per update).
+// global memory.  A batch whose taps all lie in the window and between the detector's end
+// columns runs without clamps and in-range tests, its views' coordinates computed together,
+// as in bp_direct_kernel.  VG view groups of 256 threads each stage and sum every VG-th
+// batch of the same tile (partial sums added in FP64 at the end), so that few tiles still
+// fill the chip.
+//
+// Bound: VALU issue and the LDS reads, about even.  64 slices of 512 x 512 pixels, 984 views:
+// 3.29 -> 2.12 ms by giving each wave an 8 x 8 block (its 16-byte reads stop conflicting: a
+// 16 x 4 strip spans more columns than the 16 that fall in distinct bank groups) and by the
+// batch path (4 independent chains instead of one).
 constexpr int kBpStageCols = 64;
 constexpr int kBpStageVB = 4;
 
@@ -182,52 +282,68 @@ struct BpStage {
     float val[kBpStageVB][kBpStageCols][kPitch];
 };
 
-template <bool kWeighted, int S, int kNc>
-__global__ __launch_bounds__(kBpTx *kBpTy) void bp_staged_kernel(BpArgs A, int slice0)
+template <bool kWeighted, bool kIl, int S, int kNc, int VG>
+__global__ __launch_bounds__(kBpTx *kBpTy *VG) void bp_staged_kernel(BpArgs A, int slice0)
 {
     static_assert(S % 4 == 0, "a staged column is read four slices at a time");
     constexpr int VB = kBpStageVB, SQ = S / 4;
-    __shared__ BpStage<S> st;
+    __shared__ BpStage<S> stages[VG];
     unsigned tbx, tby, g;  // blocked, XCD-aware order (neighbouring tiles share staged columns in L2)
     xcd_blocked_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, gridDim.z,
                      tbx, tby, g);
     const int tx0 = (int)tbx * kBpTx, ty0 = (int)tby * kBpTy;
     const int lane = (int)threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    // wave w takes tile rows 4w..4w+3; each 16 lanes of it a 4x4 pixel block, whose
-    // detector columns lie close together (fewer LDS bank conflicts than a 16-pixel row)
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) & 3);
+    const int vg = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));
+    BpStage<S> &st = stages[vg];
+    // each wave an 8x8 quarter of the tile, each 16 lanes of it a 4x4 block: the wave's taps
+    // lie within 14 adjacent staged columns or so (8 pixels along the diagonal at 1.2 columns
+    // a pixel), and 16 adjacent columns (pitch S + 4) start in different bank groups
     static_assert(kBpTx == 16 && kBpTy == 16, "lane layout assumes 16x16 tiles");
-    const int i = tx0 + 4 * (lane >> 4) + (lane & 3);
-    const int j = ty0 + 4 * wave + ((lane >> 2) & 3);
+    const int i = tx0 + 8 * (wave & 1) + 4 * ((lane >> 4) & 1) + (lane & 3);
+    const int j = ty0 + 8 * (wave >> 1) + 4 * (lane >> 5) + ((lane >> 2) & 3);
     const size_t sl = (size_t)slice0 + (size_t)S * g;
-    // no early exit: every thread stages and waits
+    // every thread of a tile with FOV pixels stages and waits
     const bool valid = i < A.nX && j < A.nY;
     const PixelGeo pg = pixel_geo(A, min(i, A.nX - 1), min(j, A.nY - 1));
     const int2 fr = A.fov_row[min(j, A.nY - 1)];
     const bool inside = valid && i >= fr.x && i <= fr.y;
+    float *out = A.img + (size_t)j * A.nX + i;
+    if (!__syncthreads_or(inside)) {
+        if (valid && vg == 0)
+            for (int s = 0; s < S; ++s) out[(sl + s) * A.img_stride] = 0.0f;
+        return;
+    }
     const PixelGeo pc = pixel_geo(A, min(tx0 + ((lane & 1) ? kBpTx - 1 : 0), A.nX - 1),
                                   min(ty0 + ((lane & 2) ? kBpTy - 1 : 0), A.nY - 1));
     const float *sino = A.sino + sl * A.sino_stride;  // slice group base
-    const float *sino_w = sino + (size_t)(wave * SQ) * A.sino_stride;  // this wave stages slices wave*SQ..
+    // this wave stages slices wave*SQ..: planes of them, or (interleaved by four) a quarter
+    // of a quad of slices (SQ < 4) or a quad (SQ = 4)
+    constexpr int kSl = kIl ? 4 : 1;
+    const float *sino_w = sino + (size_t)(wave * SQ / kSl * kSl) * A.sino_stride + wave * SQ % kSl;
     const unsigned sbytes = (unsigned)A.sino_stride * 4u;
     float acc[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) acc[s] = 0.0f;
+    const float mid = 0.5f * (float)(A.nCols - 1), midr = mid - (float)A.ct_col;
 
     // Staging is software-pipelined: while a batch is read from LDS, the next batch's
     // columns are loaded into registers, and written to LDS between the two barriers that
     // follow.
     auto window = [&](int v0, int (&c_lo)[VB]) {
-        float xi, U, tt;
-        (void)column_of<kNc>(A, pc, min(v0 + (lane >> 2) % VB, A.nViews - 1), xi, U, tt);
-        int wlo = (int)floorf(fminf(fmaxf(xi - 0.5f, -1.0e6f), 1.0e6f));
+        float U, tt;
+        const float ct = column_of<kNc>(A, pc, min(v0 + (lane >> 2) % VB, A.nViews - 1), U, tt);
+        int wlo = (int)floorf(fminf(fmaxf(ct, -1.0e6f), 1.0e6f)) + A.ct_col;
 #pragma unroll
         for (int sh = 1; sh <= 2; sh <<= 1) wlo = min(wlo, __shfl_xor(wlo, sh));
 #pragma unroll
         for (int m = 0; m < VB; ++m)
             c_lo[m] = min(max(__builtin_amdgcn_readlane(wlo, 4 * m) - 1, 0), max(A.nCols - kBpStageCols, 0));
     };
-    float q[VB][SQ];  // next batch: this wave's slices of lane's column, per view
+    struct __attribute__((packed, aligned(4))) Cols {
+        float v[SQ];
+    };
+    Cols q[VB];  // next batch: this wave's slices of lane's column, per view
     auto load_batch = [&](int v0, const int (&c_lo)[VB]) {
 #pragma unroll
         for (int m = 0; m < VB; ++m) {
@@ -235,9 +351,13 @@ __global__ __launch_bounds__(kBpTx *kBpTy) void bp_staged_kernel(BpArgs A, int s
             // groups only when four sinograms span less than 4 GiB)
             const unsigned off =
                 ((unsigned)min(v0 + m, A.nViews - 1) * (unsigned)A.nCols + (unsigned)min(c_lo[m] + lane, A.nCols - 1)) *
-                4u;
+                (4u * kSl);
+            if constexpr (kIl) {
+                q[m] = load_at(reinterpret_cast<const Cols *>(sino_w), off);
+            } else {
 #pragma unroll
-            for (int k = 0; k < SQ; ++k) q[m][k] = load_at(sino_w, off + (unsigned)k * sbytes);
+                for (int k = 0; k < SQ; ++k) q[m].v[k] = load_at(sino_w, off + (unsigned)k * sbytes);
+            }
         }
     };
     auto store_batch = [&](int v0, const int (&c_lo)[VB]) {
@@ -246,66 +366,109 @@ __global__ __launch_bounds__(kBpTx *kBpTy) void bp_staged_kernel(BpArgs A, int s
             if (v0 + m >= A.nViews || c_lo[m] + lane >= A.nCols) continue;
             float *dst = &st.val[m][lane][wave * SQ];
             if constexpr (SQ % 4 == 0) {
-#pragma unroll
-                for (int k = 0; k < SQ; k += 4)
-                    *reinterpret_cast<float4 *>(dst + k) = make_float4(q[m][k], q[m][k + 1], q[m][k + 2], q[m][k + 3]);
+                *reinterpret_cast<float4 *>(dst) = make_float4(q[m].v[0], q[m].v[1], q[m].v[2], q[m].v[3]);
             } else if constexpr (SQ == 2) {
-                *reinterpret_cast<float2 *>(dst) = make_float2(q[m][0], q[m][1]);
+                *reinterpret_cast<float2 *>(dst) = make_float2(q[m].v[0], q[m].v[1]);
             } else {
-                dst[0] = q[m][0];
+                dst[0] = q[m].v[0];
+            }
+        }
+    };
+    // one update of view v0 + m by the general path
+    auto update = [&](int v, int wlo, int m) {
+        float U, tt, al;
+        const float ct = column_of<kNc>(A, pg, v, U, tt);
+        if (!in_range(A, pg, v, ct)) return;
+        const int c0 = interp_pos(A, ct, al);
+        float w0, w1;
+        bp_tap_weights<kWeighted>(al, U, tt, w0, w1);
+        const int lc = c0 - wlo;
+        if ((unsigned)lc < (unsigned)(kBpStageCols - 1) && c0 + 1 < A.nCols) {
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+                acc[s] = fmaf(w1, st.val[m][lc + 1][s], fmaf(w0, st.val[m][lc][s], acc[s]));
+        } else {
+            const int c1 = min(c0 + 1, A.nCols - 1);
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const float *P = sino + (size_t)(s / kSl * kSl) * A.sino_stride + (size_t)v * A.nCols * kSl + s % kSl;
+                acc[s] = fmaf(w1, P[c1 * kSl], fmaf(w0, P[c0 * kSl], acc[s]));
             }
         }
     };
     int c_lo[VB], c_nx[VB];
-    window(0, c_nx);
-    load_batch(0, c_nx);
-    for (int v0 = 0; v0 < A.nViews; v0 += VB) {
+    window(vg * VB, c_nx);
+    load_batch(vg * VB, c_nx);
+    for (int vb = 0; vb < A.nViews; vb += VG * VB) {
+        const int v0 = vb + vg * VB;
 #pragma unroll
         for (int m = 0; m < VB; ++m) c_lo[m] = c_nx[m];
         __syncthreads();  // the previous batch's reads are done
         store_batch(v0, c_lo);
         __syncthreads();
-        if (v0 + VB < A.nViews) {
-            window(v0 + VB, c_nx);
-            load_batch(v0 + VB, c_nx);
+        if (vb + VG * VB < A.nViews) {
+            window(v0 + VG * VB, c_nx);
+            load_batch(v0 + VG * VB, c_nx);
         }
         if (!inside) continue;
-#pragma unroll 1
-        for (int m = 0; m < VB; ++m) {
-            const int v = v0 + m;
-            if (v >= A.nViews) break;
-            float xi, U, tt;
-            if (!column_of<kNc>(A, pg, v, xi, U, tt)) continue;
-            float al;
-            const int c0 = interp_pos(xi, A.nCols, al);
-            float w0, w1;
-            bp_tap_weights<kWeighted>(al, U, tt, w0, w1);
-            const int lc = c0 - c_lo[m];
-            float p0[S], p1[S];
-            if ((unsigned)lc < (unsigned)(kBpStageCols - 1) && c0 + 1 < A.nCols) {
+        if (v0 + VB <= A.nViews) {
+            float ct[VB], U[VB], tt[VB];
+            bool ok = true;
 #pragma unroll
-                for (int s = 0; s < S; s += 4) {
-                    const float4 a = *reinterpret_cast<const float4 *>(&st.val[m][lc][s]);
-                    const float4 b = *reinterpret_cast<const float4 *>(&st.val[m][lc + 1][s]);
-                    p0[s] = a.x, p0[s + 1] = a.y, p0[s + 2] = a.z, p0[s + 3] = a.w;
-                    p1[s] = b.x, p1[s + 1] = b.y, p1[s + 2] = b.z, p1[s + 3] = b.w;
-                }
-            } else {
-                const float *P = sino + (size_t)v * A.nCols;
-                const int c1 = min(c0 + 1, A.nCols - 1);
-#pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    p0[s] = P[(size_t)s * A.sino_stride + c0];
-                    p1[s] = P[(size_t)s * A.sino_stride + c1];
-                }
+            for (int m = 0; m < VB; ++m) {
+                ct[m] = column_of<kNc>(A, pg, v0 + m, U[m], tt[m]);
+                ok = ok && fabsf(ct[m] - midr) < mid - kEdgeBand;
+                ok = ok && (unsigned)((int)floorf(ct[m]) + (A.ct_col - c_lo[m])) < (unsigned)(kBpStageCols - 1);
             }
+            if (__all(ok)) {
 #pragma unroll
-            for (int s = 0; s < S; ++s) acc[s] = fmaf(w1, p1[s], fmaf(w0, p0[s], acc[s]));
+                for (int m = 0; m < VB; ++m) {
+                    const float fc = floorf(ct[m]);
+                    const int lc = (int)fc + (A.ct_col - c_lo[m]);
+                    float w0, w1;
+                    bp_tap_weights<kWeighted>(ct[m] - fc, U[m], tt[m], w0, w1);
+                    const float *p = &st.val[m][lc][0];
+#pragma unroll
+                    for (int s = 0; s < S; s += 4) {
+                        const float4 a = *reinterpret_cast<const float4 *>(p + s);
+                        const float4 b = *reinterpret_cast<const float4 *>(p + BpStage<S>::kPitch + s);
+                        acc[s] = fmaf(w1, b.x, fmaf(w0, a.x, acc[s]));
+                        acc[s + 1] = fmaf(w1, b.y, fmaf(w0, a.y, acc[s + 1]));
+                        acc[s + 2] = fmaf(w1, b.z, fmaf(w0, a.z, acc[s + 2]));
+                        acc[s + 3] = fmaf(w1, b.w, fmaf(w0, a.w, acc[s + 3]));
+                    }
+                }
+                continue;
+            }
+        }
+#pragma unroll 1
+        for (int m = 0; m < VB && v0 + m < A.nViews; ++m) {
+            int wlo = c_lo[0];
+#pragma unroll
+            for (int k = 1; k < VB; ++k) wlo = m == k ? c_lo[k] : wlo;
+            update(v0 + m, wlo, m);
         }
     }
-    if (!valid) return;
+    if constexpr (VG == 1) {
+        if (!valid) return;
 #pragma unroll
-    for (int s = 0; s < S; ++s) A.img[(sl + s) * A.img_stride + (size_t)j * A.nX + i] = acc[s];
+        for (int s = 0; s < S; ++s) out[(sl + s) * A.img_stride] = acc[s];
+    } else {
+        // the groups' partial sums meet in LDS; group g adds and stores slices g, g + VG, ...
+        static_assert(sizeof(BpStage<S>) >= sizeof(float) * S * kBpTx * kBpTy, "partial sums fit the staging space");
+        const int t = (int)threadIdx.x & 255;
+        __syncthreads();
+        float *part = &st.val[0][0][0];
+#pragma unroll
+        for (int s = 0; s < S; ++s) part[s * 256 + t] = acc[s];
+        __syncthreads();
+        for (int s = vg; s < S; s += VG) {
+            double sum = 0.0;
+#pragma unroll
+            for (int w = 0; w < VG; ++w) sum += (double)(&stages[w].val[0][0][0])[s * 256 + t];
+            if (valid) out[(sl + s) * A.img_stride] = (float)sum;
+        }
+    }
 }
 
 // ------------------------------------------------------------------ transpose
@@ -712,7 +875,8 @@ BpArgs make_args(const fbct_plan &p, const DeviceTables &t, const float *sino, f
     A.dy = p.g.dy;
     A.fov_row = t.fov_row;
     A.xi_scale = p.d.bp_xi_scale;
-    A.xi_offset = p.d.bp_xi_offset;
+    A.ct_offset = p.d.bp_ct_offset;
+    A.ct_col = p.d.bp_ct_col;
     A.edge_exact = p.d.bp_edge_exact;
     A.tan_min = p.d.bp_tan_min;
     A.tan_max = p.d.bp_tan_max;
@@ -720,48 +884,99 @@ BpArgs make_args(const fbct_plan &p, const DeviceTables &t, const float *sino, f
     return A;
 }
 
-template <bool kWeighted, int kNc>
+// Waves per block: the views are split until the launch has 8192 waves (8 per SIMD), at
+// least 4 ways (256 x 256 pixels, one slice: 51, 31, 27, 24, 29 us with 1, 2, 4, 8, 16; 512 x
+// 512: 216, 210, 180, 177, 231 us).
+template <bool kWeighted, bool kIl, int S, int kNc>
+void launch_bp_direct(const BpArgs &A, int groups, int slice0, hipStream_t stream)
+{
+    const dim3 grid((A.nX + kBpBlk - 1) / kBpBlk, (A.nY + kBpBlk - 1) / kBpBlk, groups);
+    const long long blocks = (long long)grid.x * grid.y * groups;
+    if (blocks * 4 >= 8192)
+        hipLaunchKernelGGL((bp_direct_kernel<kWeighted, kIl, S, kNc, 4>), grid, dim3(64 * 4), 0, stream, A, slice0);
+    else if (blocks * 8 >= 8192)
+        hipLaunchKernelGGL((bp_direct_kernel<kWeighted, kIl, S, kNc, 8>), grid, dim3(64 * 8), 0, stream, A, slice0);
+    else
+        hipLaunchKernelGGL((bp_direct_kernel<kWeighted, kIl, S, kNc, 16>), grid, dim3(64 * 16), 0, stream, A, slice0);
+}
+
+// View groups per workgroup: 1 from four workgroups per CU on, 2 from two, else 4 (256 x 256
+// pixels, 256 workgroups of 16 slices: 158, 100, 79 us with 1, 2, 4; 512 workgroups: 177, 131,
+// 153; 512 x 512, 1024 workgroups: 591, 637, 759).
+template <bool kWeighted, bool kIl, int S, int kNc>
+void launch_bp_staged(const BpArgs &A, dim3 tiles, int groups, int slice0, hipStream_t stream)
+{
+    const dim3 grid(tiles.x, tiles.y, groups);
+    const long long wgs = (long long)tiles.x * tiles.y * groups;
+    constexpr int nt = kBpTx * kBpTy;
+    if (wgs >= 1024)
+        hipLaunchKernelGGL((bp_staged_kernel<kWeighted, kIl, S, kNc, 1>), grid, dim3(nt), 0, stream, A, slice0);
+    else if (wgs >= 512)
+        hipLaunchKernelGGL((bp_staged_kernel<kWeighted, kIl, S, kNc, 2>), grid, dim3(2 * nt), 0, stream, A, slice0);
+    else
+        hipLaunchKernelGGL((bp_staged_kernel<kWeighted, kIl, S, kNc, 4>), grid, dim3(4 * nt), 0, stream, A, slice0);
+}
+
+// Slice groups.  Interleaved (the filtered sinograms of FBP): 16 slices staged where the
+// tiles fill the chip evenly -- four workgroups per CU or more, or a count close below a
+// multiple of the CUs, since a CU left with one workgroup more than the others sets the time --
+// else groups of four and the rest read directly (16 slices of 512 x 512: 558 us staged, 737
+// direct; of 256 x 256, 256 tiles: 74 and 87; of 373 x 373, 576 tiles on 256 CUs: 242 and 211;
+// of 96 x 96, 36 tiles: 26 and 13).  As planes [slice][view][column]: 16, then 8 slices staged
+// from half a workgroup per CU on (8 slices of 512 x 512: 433 us staged, 859 direct; of 256 x
+// 256: 57 and 91; of 96 x 96: 23 and 14), since the direct kernel gathers each slice.
+template <bool kWeighted, bool kIl, int kNc>
 void launch_bp_groups(const BpArgs &A, dim3 tiles, int n, hipStream_t stream)
 {
-    // slice groups of 16/8/4/2 while they leave enough workgroups to fill the chip, the
-    // remainder one slice per group; groups of 4 or more stage their detector columns
     const long long nt = (long long)tiles.x * tiles.y;
     // the staged kernels address a wave's (up to 4) sinograms by 32-bit byte offsets
     const bool stage_ok = (unsigned long long)A.sino_stride * 16ull < (1ull << 32);
+    const long long cus = 256;
     int done = 0;
-    for (int S : {16, 8, 4, 2, 1}) {
-        const int groups = (n - done) / S;
-        if (groups == 0 || (S > 1 && nt * groups < 2048) || (S >= 4 && !stage_ok)) continue;
-        const dim3 grid(tiles.x, tiles.y, groups);
-        switch (S) {
-        case 16: hipLaunchKernelGGL((bp_staged_kernel<kWeighted, 16, kNc>), grid, dim3(kBpTx * kBpTy), 0, stream, A, done); break;
-        case 8: hipLaunchKernelGGL((bp_staged_kernel<kWeighted, 8, kNc>), grid, dim3(kBpTx * kBpTy), 0, stream, A, done); break;
-        case 4: hipLaunchKernelGGL((bp_staged_kernel<kWeighted, 4, kNc>), grid, dim3(kBpTx * kBpTy), 0, stream, A, done); break;
-        case 2: hipLaunchKernelGGL((bp_kernel<kWeighted, 2, kNc>), grid, dim3(kBpTx * kBpTy), 0, stream, A, done); break;
-        default: hipLaunchKernelGGL((bp_kernel<kWeighted, 1, kNc>), grid, dim3(kBpTx * kBpTy), 0, stream, A, done); break;
-        }
-        done += groups * S;
-        if (done == n) break;
+    const int g16 = n / 16;
+    const long long w16 = nt * g16;
+    const bool fills = w16 >= 4 * cus || 100 * w16 >= 85 * cus * ((w16 + cus - 1) / cus);
+    if (stage_ok && g16 > 0 && (kIl ? fills : w16 >= cus / 2)) {
+        launch_bp_staged<kWeighted, kIl, 16, kNc>(A, tiles, g16, done, stream);
+        done += 16 * g16;
     }
+    if constexpr (!kIl) {
+        const int g8 = (n - done) / 8;
+        if (stage_ok && g8 > 0 && nt * g8 >= cus / 2) {
+            launch_bp_staged<kWeighted, kIl, 8, kNc>(A, tiles, g8, done, stream);
+            done += 8 * g8;
+        }
+    }
+    for (int S : {4, 3, 2, 1}) {
+        const int groups = (n - done) / S;
+        if (groups == 0) continue;
+        if (S == 4) launch_bp_direct<kWeighted, kIl, 4, kNc>(A, groups, done, stream);
+        else if (S == 3) launch_bp_direct<kWeighted, kIl, 3, kNc>(A, groups, done, stream);
+        else if (S == 2) launch_bp_direct<kWeighted, kIl, 2, kNc>(A, groups, done, stream);
+        else launch_bp_direct<kWeighted, kIl, 1, kNc>(A, groups, done, stream);
+        done += groups * S;
+    }
+}
+
+template <bool kWeighted, bool kIl>
+void launch_bp_nc(const BpArgs &A, int nc, int n, hipStream_t stream)
+{
+    const dim3 tiles((A.nX + kBpTx - 1) / kBpTx, (A.nY + kBpTy - 1) / kBpTy);
+    if (nc == 9) launch_bp_groups<kWeighted, kIl, 9>(A, tiles, n, stream);
+    else if (nc == 5) launch_bp_groups<kWeighted, kIl, 5>(A, tiles, n, stream);
+    else launch_bp_groups<kWeighted, kIl, 0>(A, tiles, n, stream);
 }
 
 }  // namespace
 
 fbct_status launch_bp(const fbct_plan &p, const DeviceTables &t, const float *sino, float *img, int n,
-                      bool weighted, hipStream_t stream)
+                      bool weighted, bool interleaved, hipStream_t stream)
 {
-    BpArgs A = make_args(p, t, sino, img);
-    const dim3 tiles((p.g.nX + kBpTx - 1) / kBpTx, (p.g.nY + kBpTy - 1) / kBpTy);
+    const BpArgs A = make_args(p, t, sino, img);
     const int nc = p.d.bp_atan_nc;
-    if (weighted) {
-        if (nc == 9) launch_bp_groups<true, 9>(A, tiles, n, stream);
-        else if (nc == 5) launch_bp_groups<true, 5>(A, tiles, n, stream);
-        else launch_bp_groups<true, 0>(A, tiles, n, stream);
-    } else {
-        if (nc == 9) launch_bp_groups<false, 9>(A, tiles, n, stream);
-        else if (nc == 5) launch_bp_groups<false, 5>(A, tiles, n, stream);
-        else launch_bp_groups<false, 0>(A, tiles, n, stream);
-    }
+    if (interleaved) launch_bp_nc<true, true>(A, nc, n, stream);
+    else if (weighted) launch_bp_nc<true, false>(A, nc, n, stream);
+    else launch_bp_nc<false, false>(A, nc, n, stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "bp_kernel launch: %s", hipGetErrorString(e));
     return FBCT_OK;

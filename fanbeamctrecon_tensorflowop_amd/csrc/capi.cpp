@@ -32,7 +32,7 @@ fbct_status filter_rows(const fbct_plan &p, const fbct::DeviceTables &t, const f
                         fbct_filter_mode mode, hipStream_t st)
 {
     return mode == FBCT_FILTER_FP64 ? fbct::launch_ramp_filter(p, t, in, out, rows, st)
-                                    : fbct::launch_ramp_filter_mfma(p, t, in, out, rows, st);
+                                    : fbct::launch_ramp_filter_mfma(p, t, in, out, rows, fbct::RowWeights{}, false, st);
 }
 
 size_t sino_bytes(const fbct_plan *p, int64_t n, int dtype = FBCT_F32)
@@ -142,7 +142,7 @@ fbct_status fbct_bp(fbct_plan *plan, const float *sino, float *image, int n_slic
     if ((s = check_io(plan, image, FBCT_F32, sino, FBCT_F32, n_slices, "fbct_bp")) != FBCT_OK) return s;
     const fbct::DeviceTables *t = nullptr;
     if ((s = fbct::device_tables(plan, &t)) != FBCT_OK) return s;
-    return fbct::launch_bp(*plan, *t, sino, image, n_slices, false, static_cast<hipStream_t>(stream));
+    return fbct::launch_bp(*plan, *t, sino, image, n_slices, false, false, static_cast<hipStream_t>(stream));
 }
 
 fbct_status fbct_bp_adjoint(fbct_plan *plan, const float *image, float *sino, int n_slices, void *stream)
@@ -162,7 +162,7 @@ fbct_status fbct_fbp_backproject(fbct_plan *plan, const float *sino, float *imag
     if ((s = check_io(plan, image, FBCT_F32, sino, FBCT_F32, n_slices, "fbct_fbp_backproject")) != FBCT_OK) return s;
     const fbct::DeviceTables *t = nullptr;
     if ((s = fbct::device_tables(plan, &t)) != FBCT_OK) return s;
-    return fbct::launch_bp(*plan, *t, sino, image, n_slices, true, static_cast<hipStream_t>(stream));
+    return fbct::launch_bp(*plan, *t, sino, image, n_slices, true, false, static_cast<hipStream_t>(stream));
 }
 
 fbct_status fbct_fbp_backproject_adjoint(fbct_plan *plan, const float *image, float *sino, int n_slices,
@@ -225,24 +225,19 @@ fbct_status fbct_fbp_ex(fbct_plan *plan, const float *sino, float *image, int n_
     hipStream_t st = static_cast<hipStream_t>(stream);
     float *q = static_cast<float *>(workspace);
     const int64_t rows = (int64_t)n_slices * plan->g.nViews;
-    if (flags == 0) {
-        if ((s = filter_rows(*plan, *t, sino, q, rows, FBCT_FILTER_MFMA, st)) != FBCT_OK) return s;
-    } else {
-        // pre-weights multiply the rows as the MFMA filter stages them (row r = slice * nViews + view)
-        fbct::RowWeights rw;
-        if (flags & FBCT_FBP_COSINE) {
-            if ((s = fbct::device_cosine(plan, t, &rw.w)) != FBCT_OK) return s;
-            rw.wrows = 1;
-        }
-        if (flags & FBCT_FBP_SHORT_SCAN) {
-            if ((s = fbct::device_parker(plan, t, &rw.w2)) != FBCT_OK) return s;
-            rw.w2div = 1;
-            rw.w2rows = plan->g.nViews;
-        }
-        fbct::RampOperand H{t->ramp_planes, plan->g.nCols, plan->d.ramp_np, plan->d.ramp_kp, plan->d.ramp_lg};
-        if ((s = fbct::launch_ramp_gemm(H, sino, FBCT_F32, q, rows, rw, st)) != FBCT_OK) return s;
+    // pre-weights multiply the rows as the MFMA filter stages them (row r = slice * nViews + view)
+    fbct::RowWeights rw;
+    if (flags & FBCT_FBP_COSINE) {
+        if ((s = fbct::device_cosine(plan, t, &rw.w)) != FBCT_OK) return s;
+        rw.wrows = 1;
     }
-    return fbct::launch_bp(*plan, *t, q, image, n_slices, true, st);
+    if (flags & FBCT_FBP_SHORT_SCAN) {
+        if ((s = fbct::device_parker(plan, t, &rw.w2)) != FBCT_OK) return s;
+        rw.w2div = 1;
+        rw.w2rows = plan->g.nViews;
+    }
+    if ((s = fbct::launch_ramp_filter_mfma(*plan, *t, sino, q, rows, rw, true, st)) != FBCT_OK) return s;
+    return fbct::launch_bp(*plan, *t, q, image, n_slices, true, true, st);
 }
 
 fbct_status fbct_fbp(fbct_plan *plan, const float *sino, float *image, int n_slices, void *workspace,

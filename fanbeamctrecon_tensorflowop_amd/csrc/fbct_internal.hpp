@@ -168,7 +168,8 @@ struct Derived {
     float two_r;          // 2 * rFOV/dx (FP sample coordinate extent)
     FpBundleCfg fpb[kFpNumCfg];
     float bp_xi_scale;    // 1/dCol
-    float bp_xi_offset;   // dShift - dLeft/dCol
+    int bp_ct_col;        // dShift - dLeft/dCol - 1/2 = bp_ct_col + bp_ct_offset, the latter in
+    float bp_ct_offset;   // [-1/2, 1/2]: column coordinates relative to column bp_ct_col
     float r2;             // rFOV*rFOV (float, as the reference)
     float bpa_tan;        // tan |dCol|: BP^T candidate half-width per unit distance from the source
     // In-range decision 0 < xi < nCols taken in FP64 near the two edges: with
@@ -365,8 +366,10 @@ fbct_status launch_fp(const fbct_plan &p, const DeviceTables &t, const void *img
                       void *sino, fbct_dtype to, int n, hipStream_t stream, const float *target = nullptr);
 fbct_status launch_fp_adjoint(const fbct_plan &p, const DeviceTables &t, const void *sino,
                               fbct_dtype ti, void *img, fbct_dtype to, int n, hipStream_t stream);
+// interleaved: the sinograms lie as launch_ramp_filter_mfma leaves them when asked to
+// interleave (weighted form only); otherwise as [slice][view][column].
 fbct_status launch_bp(const fbct_plan &p, const DeviceTables &t, const float *sino, float *img,
-                      int n, bool weighted, hipStream_t stream);
+                      int n, bool weighted, bool interleaved, hipStream_t stream);
 fbct_status launch_bp_adjoint(const fbct_plan &p, const DeviceTables &t, const float *img,
                               float *sino, int n, bool weighted, hipStream_t stream);
 fbct_status launch_ramp_filter(const fbct_plan &p, const DeviceTables &t, const float *in,
@@ -390,11 +393,13 @@ struct RowWeights {
     int w2div = 1, w2rows = 1;
 };
 fbct_status launch_ramp_gemm(const RampOperand &H, const void *in, fbct_dtype ti, float *out, int64_t rows,
-                             const RowWeights &rw, hipStream_t stream);
+                             const RowWeights &rw, hipStream_t stream, int il_views = 0);
 // q: filtered projections, FP32 [n][nViews][nRows][nCols].
 fbct_status launch_cone_bp(const fbct_cone_plan &p, const ConeDeviceTables &t, const float *q,
                            void *vol, fbct_dtype to, int n, hipStream_t stream);
-fbct_status launch_ramp_filter_mfma(const fbct_plan &p, const DeviceTables &t, const float *in,
-                                    float *out, int64_t rows, hipStream_t stream);
+// interleaved: the outputs (whole slices, rows = slices * nViews) in groups of four slices,
+// each [view][column][slice of the group]; the last group holds the remaining slices.
+fbct_status launch_ramp_filter_mfma(const fbct_plan &p, const DeviceTables &t, const float *in, float *out,
+                                    int64_t rows, const RowWeights &rw, bool interleaved, hipStream_t stream);
 
 }  // namespace fbct

@@ -39,7 +39,34 @@ struct MfmaArgs {
     const float *w2;   // optional second factor [w2rows][nC], row r uses w2[(r / w2div) % w2rows]
     long long rows;
     int nC, Np, Kp, Lg, wrows, w2div, w2rows;
+    int il_views;      // > 0: outputs interleaved (RampLayout), views per slice; 0: as the inputs
+    long long il_full; // rows in groups of four slices
+    int il_rest;       // slices of the last group (0: none)
 };
+
+// Interleaved output: slices in groups of four (the last group holds the rest), a group's
+// sinograms as [view][column][slice of the group].  The GEMM's rows then run over the views
+// with the group's slices innermost: row r of the product is the input row in_row(r), and
+// its column c is stored at out_base(r) + c * group size.
+struct __attribute__((packed, aligned(4))) Quad {
+    float v[4];
+};
+
+struct IlRow {
+    long long in_row, out_base;
+    int step;
+};
+
+__device__ __forceinline__ IlRow il_row(const MfmaArgs &A, long long r)
+{
+    if (A.il_views == 0) return {r, r * A.nC, 1};
+    const bool rest = r >= A.il_full;
+    const int sl = rest ? max(A.il_rest, 1) : 4;  // (rows past the last one may be asked for)
+    const long long block = 4LL * A.il_views;
+    const long long b0 = rest ? A.il_full : r / block * block;
+    const int local = (int)(r - b0), v = local / sl, s = local - v * sl;
+    return {b0 + (long long)s * A.il_views + v, (b0 + (long long)v * sl) * A.nC + s, sl};
+}
 
 __device__ __forceinline__ void split3(float x, __bf16 &hi, __bf16 &lo, __bf16 &ll)
 {
@@ -99,7 +126,7 @@ __global__ __launch_bounds__(kGemmThreads) void ramp_gemm_kernel(MfmaArgs A)
     // staging assignment: thread -> (row, 16 k-values at kh)
     const int srow = tid / (BK / 16), kh = tid % (BK / 16) * 16;
     const bool arow_ok = r0 + srow < A.rows;
-    const long long arow = arow_ok ? r0 + srow : 0;
+    const long long arow = arow_ok ? il_row(A, r0 + srow).in_row : 0;
     const TI *prow = static_cast<const TI *>(A.in) + arow * (long long)A.nC;
     const float *wrow = kW && A.w ? A.w + arow % A.wrows * (long long)A.nC : nullptr;
     const float *w2row =
@@ -234,13 +261,22 @@ __global__ __launch_bounds__(kGemmThreads) void ramp_gemm_kernel(MfmaArgs A)
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const long long row0 = r0 + wr * (BM / WR) + 16 * i + 4 * (lane >> 4);
+        // a lane's four rows are the four slices of one (view, column): one 16-byte store
+        const bool quad = A.il_views > 0 && row0 < A.il_full;
+        IlRow o[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = il_row(A, row0 + j);
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             const int col = c0 + wc * (BN / WC) + 16 * t + (lane & 15);
             if (col >= A.nC) continue;
+            if (quad) {
+                *reinterpret_cast<Quad *>(A.out + o[0].out_base + 4LL * col) = Quad{{acc[i][t][0], acc[i][t][1], acc[i][t][2], acc[i][t][3]}};
+                continue;
+            }
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                if (row0 + j < A.rows) A.out[(row0 + j) * A.nC + col] = acc[i][t][j];
+                if (row0 + j < A.rows) A.out[o[j].out_base + (long long)col * o[j].step] = acc[i][t][j];
         }
     }
 }
@@ -257,7 +293,7 @@ void launch_gemm_p(int bm, dim3 grid, hipStream_t stream, const MfmaArgs &A)
 }  // namespace
 
 fbct_status launch_ramp_gemm(const RampOperand &H, const void *in, fbct_dtype ti, float *out, int64_t rows,
-                             const RowWeights &rw, hipStream_t stream)
+                             const RowWeights &rw, hipStream_t stream, int il_views)
 {
     if (rows <= 0) return FBCT_OK;
     if ((rw.w && rw.wrows <= 0) || (rw.w2 && (rw.w2div <= 0 || rw.w2rows <= 0)))
@@ -277,6 +313,15 @@ fbct_status launch_ramp_gemm(const RampOperand &H, const void *in, fbct_dtype ti
     A.wrows = rw.w ? rw.wrows : 1;
     A.w2div = rw.w2 ? rw.w2div : 1;
     A.w2rows = rw.w2 ? rw.w2rows : 1;
+    A.il_views = il_views;
+    A.il_full = 0;
+    A.il_rest = 0;
+    if (il_views > 0) {
+        const int64_t n = rows / il_views;
+        if (n * il_views != rows) return fail(FBCT_ERR_INVALID_ARGUMENT, "ramp filter: rows are not whole slices");
+        A.il_full = n / 4 * 4 * il_views;
+        A.il_rest = (int)(n % 4);
+    }
     if (H.Np % kRampTileN != 0 || H.Np < H.nC || H.Kp % 32 != 0 || H.Kp < H.nC || H.Lg != ramp_table_len(H.Np, H.Kp))
         return fail(FBCT_ERR_UNSUPPORTED, "ramp filter: operand planes not padded to the tile");
     // Tile shape (rows x columns x K step).  The widest, 128 x 256 x 32, splits each input
@@ -316,10 +361,10 @@ fbct_status launch_ramp_gemm(const RampOperand &H, const void *in, fbct_dtype ti
 }
 
 fbct_status launch_ramp_filter_mfma(const fbct_plan &p, const DeviceTables &t, const float *in, float *out,
-                                    int64_t rows, hipStream_t stream)
+                                    int64_t rows, const RowWeights &rw, bool interleaved, hipStream_t stream)
 {
     RampOperand H{t.ramp_planes, p.g.nCols, p.d.ramp_np, p.d.ramp_kp, p.d.ramp_lg};
-    return launch_ramp_gemm(H, in, FBCT_F32, out, rows, RowWeights{}, stream);
+    return launch_ramp_gemm(H, in, FBCT_F32, out, rows, rw, stream, interleaved ? p.g.nViews : 0);
 }
 
 }  // namespace fbct

@@ -86,9 +86,10 @@ fbct_status fbct_fbp_noalloc(fbct_plan *plan, const float *sino, float *image, i
         const int c = n_slices - s0 < chunk ? n_slices - s0 : chunk;
         float *qf = static_cast<float *>(q);
         if ((s = fbct::launch_ramp_filter_mfma(*plan, *t, sino + (size_t)s0 * sino_elems, qf,
-                                               (int64_t)c * plan->g.nViews, st)) != FBCT_OK)
+                                               (int64_t)c * plan->g.nViews, fbct::RowWeights{}, true, st)) != FBCT_OK)
             return s;
-        if ((s = fbct::launch_bp(*plan, *t, qf, image + (size_t)s0 * img_elems, c, true, st)) != FBCT_OK) return s;
+        if ((s = fbct::launch_bp(*plan, *t, qf, image + (size_t)s0 * img_elems, c, true, true, st)) != FBCT_OK)
+            return s;
     }
     return FBCT_OK;
 }

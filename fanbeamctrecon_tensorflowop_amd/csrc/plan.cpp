@@ -424,8 +424,12 @@ static void build_tables(fbct_plan &p)
 
     // BP: xi_raw = (atan(t/U) - dLeft)/dCol + dShift  (BP/transform.cu:85).
     d.bp_xi_scale = static_cast<float>(1.0 / static_cast<double>(g.dCol));
-    d.bp_xi_offset = static_cast<float>(static_cast<double>(g.dShift) -
-                                        static_cast<double>(g.dLeft) / static_cast<double>(g.dCol));
+    {
+        const double c = static_cast<double>(g.dShift) - static_cast<double>(g.dLeft) / static_cast<double>(g.dCol) - 0.5;
+        const double mid = std::min(std::max(std::nearbyint(c), -1.0e6), 1.0e6);
+        d.bp_ct_col = static_cast<int>(mid);
+        d.bp_ct_offset = static_cast<float>(c - mid);
+    }
     d.r2 = g.rFOV * g.rFOV;
 
     // BP^T gathers per (view, column): gamma_c of every column in FP64 and the FOV disk
