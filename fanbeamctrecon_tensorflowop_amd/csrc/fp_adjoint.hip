@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "dtype.hpp"
 #include "fbct_internal.hpp"
@@ -122,9 +123,11 @@ __device__ __forceinline__ void candidate_rays(const FpaArgs &A, float2 cs, floa
 // evaluates a view's model; the 16 lanes of the block read it with shuffles.
 struct BlockCand {
     float cf, gx, gy, hw;  // centre column, d cf / dx, d cf / dy (per mm), half-width
+    float dx, dy, spread;  // ray direction at the centre; a bound on how far any candidate's differs
 };
 
-__device__ __forceinline__ BlockCand block_candidates(const FpaArgs &A, float2 cs, float xc, float yc, float rho)
+__device__ __forceinline__ BlockCand block_candidates(const FpaArgs &A, float2 cs, float xc, float yc, float rho,
+                                                      float h)
 {
     const float U = fmaf(-yc, cs.y, fmaf(-xc, cs.x, A.R));
     const float t = fmaf(xc, cs.y, -yc * cs.x);
@@ -136,7 +139,6 @@ __device__ __forceinline__ BlockCand block_candidates(const FpaArgs &A, float2 c
     const float k = A.c_scale * __builtin_amdgcn_rcpf(fmaf(U, U, t * t));
     b.gx = k * fmaf(U, cs.y, t * cs.x);
     b.gy = k * fmaf(t, cs.y, -U * cs.x);
-    const float h = 1.5f * A.dx;
     const float Umin = U - (fabsf(cs.x) + fabsf(cs.y)) * h;
     // every point of the block is at least Rmin from the source: its U is at least Umin,
     // and it lies within 1.415 h of the block centre, at sqrt(U^2 + t^2) from the source
@@ -159,29 +161,12 @@ __device__ __forceinline__ BlockCand block_candidates(const FpaArgs &A, float2 c
     // covers the FP32 sample positions (within 3e-4 texel of the line).  Only rays without
     // samples in the cell are dropped.
     const float hw_disk = half_width(rho);
-    const float ax = fabsf(fmaf(t, cs.y, -U * cs.x)), ay = fabsf(fmaf(U, cs.y, t * cs.x));
+    const float ax = fmaf(t, cs.y, -U * cs.x), ay = -fmaf(U, cs.y, t * cs.x);
     const float spread = fmaf(1.415f * h, rRm, hw_disk * __builtin_amdgcn_rcpf(A.c_abs));
-    const float rs = fminf(rho, fmaf(0.5f * (ax + ay), rL, fmaf(0.7072f, spread, 0.004f)));
+    const float rs = fminf(rho, fmaf(0.5f * (fabsf(ax) + fabsf(ay)), rL, fmaf(0.7072f, spread, 0.004f)));
     b.hw = half_width(rs);
+    b.dx = ax * rL, b.dy = ay * rL, b.spread = spread;
     return b;
-}
-
-// The cell's candidate range from its block's model (dxl, dyl: cell centre minus block
-// centre, mm).
-__device__ __forceinline__ void cell_candidates(const FpaArgs &A, const BlockCand &b, float dxl, float dyl, int &clo,
-                                                int &chi)
-{
-    const float cf = fmaf(b.gx, dxl, fmaf(b.gy, dyl, b.cf));
-    clo = (int)fmaxf(ceilf(cf - b.hw), 0.0f);
-    chi = (int)fminf(floorf(cf + b.hw), (float)(A.nCols - 1));
-}
-
-// The model of view j of a group of 16 (lane (lane & ~15) | j holds it): every lane of
-// the wave takes part.
-__device__ __forceinline__ BlockCand block_model_of(const BlockCand &mine, int j)
-{
-    const int src = ((int)threadIdx.x & 48) | j;
-    return BlockCand{__shfl(mine.cf, src), __shfl(mine.gx, src), __shfl(mine.gy, src), __shfl(mine.hw, src)};
 }
 
 // W_c(i, j): total bilinear weight pixel (fi, fj) receives from the N samples of ray
@@ -464,41 +449,59 @@ __global__ __launch_bounds__(kAdjThreads) void fp_adjoint_kernel(FpaArgs A)
 // (2 rFOV/dx - n + 1/2 < 1, square images); otherwise the gather kernels run.  Every
 // variant below evaluates a slice with the same arithmetic in the same order, so results
 // do not depend on how many slices share a launch.
-constexpr int kCellTile = kAdjCellTile;  // cells per tile side; a tile yields 15 x 15 pixels
+constexpr int kCellTile = kAdjCellTile;  // cells per tile side; a tile yields 7 x 7 pixels
 constexpr int kCellOut = kCellTile - 1;
-constexpr int kCells = kCellTile * kCellTile;  // one per thread
+constexpr int kCells = kCellTile * kCellTile;  // one per lane
 constexpr int kCombineS = 4;                   // slices combined per LDS pass
 constexpr float kCellRho = 0.70710678f;        // half a cell diagonal (texels)
 
-// Closed-form sums over the samples of ray g = (u0, w0, du, dw) (inv = (1/du, 1/dw), N
-// samples) that lie in cell (fci, fcj): r = (n, sum of u-fractions, sum of
-// w-fractions, sum of their products).  The bilinear weights the cell's corners (0,0)
-// (1,0) (0,1) (1,1) receive are r0 - r1 - r2 + r3, r1 - r3, r2 - r3 and r3 (formed once
-// per cell from the accumulated sums in cell_combine).
-__device__ __forceinline__ void cell_sums(float4 g, float2 inv, float N, float fci, float fcj, float r[4])
+// A ray as the cell kernels read it: u0, w0, du, dw; 1/du, 1/dw, -u0/du, -w0/dw; samples N,
+// du dw / 12.
+struct RayRec {
+    float4 p, q;
+    float2 n;
+};
+
+// Closed-form sums over the samples of a ray that lie in cell (fci, fcj): their number n, and
+// the sums n ta of the u-fractions, n tm of the w-fractions and n g of their products.  The
+// bilinear weights the cell's corners (0,0) (1,0) (0,1) (1,1) receive are n (1 - ta - tm + g),
+// n (ta - g), n (tm - g) and n g (formed once per cell from the accumulated sums in
+// cell_combine).
+//
+// (ulo, uhi) and (wlo, whi) are the cell's boundaries in the order the ray meets them: (fci, fci +
+// 1) for du > 0, the other way round for du < 0; kMixed: in either order, sorted here.
+struct CellSums {
+    float n, ta, tm, g;  // samples, their mean fractions, the mean of the fractions' products
+};
+template <bool kMixed>
+__device__ __forceinline__ CellSums cell_sums(const RayRec &ray, float fci, float fcj, float ulo, float uhi, float wlo,
+                                              float whi)
 {
     // sample range inside the cell, per axis, then intersected with [0, N): the samples
     // that precede boundary b along the ray number ceil((b - u0) / du) in either
     // direction (a sample exactly on b goes to the cell it leaves, where its bilinear
-    // weights are the same), so the range is [ceil(min q), ceil(max q)); the upper
-    // boundary uses the expression its other cell uses for its lower one
-    const float eu = fci - g.x, ew = fcj - g.y;
-    const float qu0 = eu * inv.x, qu1 = (fci + 1.0f - g.x) * inv.x;
-    const float qw0 = ew * inv.y, qw1 = (fcj + 1.0f - g.y) * inv.y;
-    const float lou = ceilf(fminf(qu0, qu1)), hiu = ceilf(fmaxf(qu0, qu1));
-    const float low = ceilf(fminf(qw0, qw1)), hiw = ceilf(fmaxf(qw0, qw1));
-    const float klo = fminf(fmaxf(fmaxf(lou, low), 0.0f), N);
-    const float khi = fminf(fminf(hiu, hiw), N);
-    const float n = fmaxf(khi - klo, 0.0f);
-    // fractions of the first sample: the cell index is subtracted before the step is
-    // added, so the FP32 rounding is that of the distance, not of the texel coordinate
-    const float ta = fmaf(klo, g.z, -eu), tm = fmaf(klo, g.w, -ew);
-    const float t1 = 0.5f * fmaf(n, n, -n);                    // sum of j < n
-    const float t2 = t1 * fmaf(n, 2.0f / 3.0f, -1.0f / 3.0f);  // sum of j^2
-    r[0] = n;
-    r[1] = fmaf(g.z, t1, n * ta);  // sum of u-fractions
-    r[2] = fmaf(g.w, t1, n * tm);  // sum of w-fractions
-    r[3] = fmaf(ta, r[2], g.z * fmaf(tm, t1, g.w * t2));  // sum of products: ta r2 + du (tm t1 + dw t2)
+    // weights are the same), so the range is [ceil(min q), ceil(max q)); both cells that share
+    // a boundary evaluate the same expression for it
+    float qul = fmaf(ulo, ray.q.x, ray.q.z), quh = fmaf(uhi, ray.q.x, ray.q.z);
+    float qwl = fmaf(wlo, ray.q.y, ray.q.w), qwh = fmaf(whi, ray.q.y, ray.q.w);
+    if constexpr (kMixed) {
+        const float a = fminf(qul, quh), b = fminf(qwl, qwh);
+        quh = fmaxf(qul, quh), qwh = fmaxf(qwl, qwh);
+        qul = a, qwl = b;
+    }
+    const float klo = ceilf(fmaxf(fmaxf(qul, qwl), 0.0f));
+    const float khi = ceilf(fminf(fminf(quh, qwh), ray.n.x));
+    CellSums c;
+    c.n = fmaxf(khi - klo, 0.0f);
+    // the fractions are linear in the sample index, so their means are those of the middle
+    // (half-integer) index, and the mean of their products is the product of the means plus
+    // du dw times the variance (n^2 - 1) / 12 of the indices.  The cell index is subtracted
+    // before the step is added, so the FP32 rounding is that of the distance, not of the texel
+    // coordinate.
+    const float kc = fmaf(c.n, 0.5f, klo - 0.5f);
+    c.ta = fmaf(kc, ray.p.z, ray.p.x - fci), c.tm = fmaf(kc, ray.p.w, ray.p.y - fcj);
+    c.g = fmaf(ray.n.y, fmaf(c.n, c.n, -1.0f), c.ta * c.tm);
+    return c;
 }
 
 // True when cell (ci, cj) can hold samples: every sample lies in the FOV disk of radius
@@ -514,46 +517,74 @@ __device__ __forceinline__ bool cell_in_fov(const FpaArgs &A, float fci, float f
     return fmaf(ex, ex, ey * ey) <= rr * rr;
 }
 
-// Adds the S-slice contribution of one ray to the cell's sums.
-template <int S>
-__device__ __forceinline__ void cell_accumulate(float4 g, float2 inv, float N, const float (&sv)[S],
-                                                float fci, float fcj, float (&acc)[4][S])
-{
-    float r[4];
-    cell_sums(g, inv, N, fci, fcj, r);
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int s = 0; s < S; ++s) acc[q][s] = fmaf(r[q], sv[s], acc[q][s]);
-}
+// A workgroup owns a tile of 8 x 8 cells, one per lane, and its four waves a quarter of the views
+// each (their sums meet in LDS at the end), so that small images fill the chip too.  A wave runs
+// without workgroup barriers: the columns around its candidate rays are staged by the wave, for
+// itself, in 64 LDS slots (the windows of 4, 3, 2 or 1 views, 16, 21, 32 or 64 columns wide, as
+// the tile's geometry in the current group of views needs), each slot holding a ray's record and
+// its S values.  LDS operations of a wave complete in order, so rewriting the slots needs no
+// wait.
+//
+// The candidate columns of a cell come from one linear model per (tile, view) -- evaluated for
+// 16 views at a time, one per lane, and read back as wave-uniform scalars: a cell's first
+// candidate is two FMAs and a ceil, and the number of candidates is uniform (the widest range
+// that fits the half-width), so the candidate loop has no divergence.  Columns beyond the
+// detector are staged as rays without samples, so it has no clamps either.
+//
+// Bound: VALU issue (0.7 of it, a third of the instructions issued in pairs): per wave and view
+// about 2.15 candidates (1.55 rays meet a cell at 512 x 512 / 888 columns) of 25 instructions and
+// 4 S multiply-adds, and 30 for the model, the staging and the loop.  Measured on 512 x 512 pixels, 984
+// views, 888 columns: 1 slice 940 -> 603 us, 4 slices 1.30 ms -> 835 us (with the rays read by every
+// cell from global memory, and staged per workgroup between barriers); 16 slices 2.0 -> 1.78 ms;
+// 256 x 256, 360 views, 512 columns: 1 slice 162 -> 115 us, 4 slices 614 -> 145 us; 104 x 104, 147
+// views: 81 -> 19 us.  Tiles of 16 x 16 cells (four waves side by side) have less overlap (1.14
+// against 1.31 cells per pixel) and measured the same within 5% at 512 x 512 (596 us for 1 slice) and
+// slower on smaller images (156 us at 256 x 256).
+constexpr int kWvGroup = 16;      // views whose models are evaluated together
+constexpr int kWvSlots = 64;      // staged columns per wave
+constexpr int kWvSplit = 4;       // waves per workgroup, each a quarter of the views
+constexpr float kWvHalf = 3.5f;   // cell centres lie within this many texels of the tile's centre
 
-// Cell (lx, ly) of this thread in the 16 x 16 tile: wave w takes cell rows 4w..4w+3 and
-// each 16 lanes of it a 4 x 4 block, whose candidate columns lie close together (fewer
-// LDS bank conflicts on the staged columns than a 16-cell row).
+// Slot stride in dwords: record (10), S values (from dword 10, or 12 for S >= 4), and padding
+// so that 16 adjacent slots start in different bank groups (an odd multiple of 4 dwords).
+template <int S>
+struct alignas(16) WvStage {
+    static constexpr int kDw = S == 16 ? 28 : S >= 4 ? 20 : 12;
+    float slot[kWvSlots * kDw];
+};
+
+template <int S>
+union CellShared {
+    static constexpr int kC = S < kCombineS ? S : kCombineS;
+    WvStage<S> stage[kWvSplit];
+    float part[(kWvSplit - 1) * 4 * kC * kCells];
+};
+
+// Cell (lx, ly) of this lane in the tile: each 16 lanes a 4 x 4 block, whose candidate columns
+// lie close together (few LDS bank conflicts).
 __device__ __forceinline__ void tile_cell(int &lx, int &ly)
 {
-    static_assert(kCellTile == 16 && kCells == 256, "lane layout assumes 16 x 16 cells, 256 threads");
-    const int t = (int)threadIdx.x, lane = t & 63;
-    lx = 4 * (lane >> 4) + (lane & 3);
-    ly = 4 * (t >> 6) + ((lane >> 2) & 3);
+    const int lane = (int)threadIdx.x & 63;
+    lx = 4 * ((lane >> 4) & 1) + (lane & 3);
+    ly = 4 * (lane >> 5) + ((lane >> 2) & 3);
 }
 
 // Combines the cell sums acc[4][S] (n, Su, Sw, Suw, each times the ray values) of the
-// tile's cells, as corner partials, into its 15 x 15 pixels of
-// slices [s0, s0 + S), kCombineS slices per pass through part (4 x kCombineS x kCells
-// floats of LDS, free when called; every thread calls it).  Pixel (px, py) collects
-// corner dx of cell px - dx (dx = 0, 1), and, on the borders, the clamped outer corner
-// of cell -1 (pixel 0) or of cell n-1 (pixel n-1).
+// tile's cells, as corner partials, into its 7 x 7 pixels of slices [s0, s0 + S),
+// kCombineS slices per pass through part (4 x kCombineS x kCells floats of LDS, free when
+// called).  Pixel (px, py) collects corner dx of cell px - dx (dx = 0, 1), and, on the borders,
+// the clamped outer corner of cell -1 (pixel 0) or of cell n-1 (pixel n-1).  Every thread of
+// the workgroup calls it; those with own = false only keep the barriers.
 template <int S, typename TO>
 __device__ __forceinline__ void cell_combine(const FpaArgs &A, float *part, const float (&acc)[4][S], int tx, int ty,
-                                             int s0)
+                                             int s0, bool own)
 {
     int lx, ly;
     tile_cell(lx, ly);
     const int cid = ly * kCellTile + lx;
     const int px = tx * kCellOut + lx, py = ty * kCellOut + ly;
-    const bool out = lx < kCellOut && ly < kCellOut && px < A.nX && py < A.nY;
-    int xc[3], xd[3], yc[3], yd[3];  // local cell column and corner of each x (y) term
+    const bool out = own && lx < kCellOut && ly < kCellOut && px < A.nX && py < A.nY;
+    int xc[4], xd[4], yc[4], yd[4];  // local cell column and corner of each x (y) term (4: a side of one pixel)
     int nxt = 0, nyt = 0;
     xc[nxt] = lx + 1, xd[nxt++] = 0;
     xc[nxt] = lx, xd[nxt++] = 1;
@@ -566,14 +597,16 @@ __device__ __forceinline__ void cell_combine(const FpaArgs &A, float *part, cons
 #pragma unroll
     for (int sb = 0; sb < S; sb += kCombineS) {
         constexpr int kC = S < kCombineS ? S : kCombineS;
+        if (own) {
 #pragma unroll
-        for (int k = 0; k < kC; ++k) {  // corner weights from the sums (n, Su, Sw, Suw)
-            const float sn = acc[0][sb + k], su = acc[1][sb + k], sw = acc[2][sb + k], suw = acc[3][sb + k];
-            const float c01 = sw - suw;
-            part[(0 * kC + k) * kCells + cid] = (sn - su) - c01;
-            part[(1 * kC + k) * kCells + cid] = su - suw;
-            part[(2 * kC + k) * kCells + cid] = c01;
-            part[(3 * kC + k) * kCells + cid] = suw;
+            for (int k = 0; k < kC; ++k) {  // corner weights from the sums (n, Su, Sw, Suw)
+                const float sn = acc[0][sb + k], su = acc[1][sb + k], sw = acc[2][sb + k], suw = acc[3][sb + k];
+                const float c01 = sw - suw;
+                part[(0 * kC + k) * kCells + cid] = (sn - su) - c01;
+                part[(1 * kC + k) * kCells + cid] = su - suw;
+                part[(2 * kC + k) * kCells + cid] = c01;
+                part[(3 * kC + k) * kCells + cid] = suw;
+            }
         }
         __syncthreads();
         if (out) {
@@ -592,285 +625,307 @@ __device__ __forceinline__ void cell_combine(const FpaArgs &A, float *part, cons
     }
 }
 
-// Cell tile (tx, ty): cells tx*15-1 .. tx*15+14 (and likewise in y), output pixels
-// tx*15 .. tx*15+14, slices [s0, s0 + S), every ray read from global memory.  Every
-// thread of the workgroup calls it; part: 4 x min(S, kCombineS) x kCells floats of LDS.
-template <int S, typename TI, typename TO>
-__device__ __forceinline__ void cell_tile(const FpaArgs &A, int tx, int ty, int s0, float *part)
+// First view of quarter r of the views: a multiple of 4 (whole staging batches).
+__device__ __forceinline__ int view_quarter(int nViews, int r)
 {
+    return r == 4 ? nViews : min(4 * (int)(((long long)nViews * r + 8) / 16), nViews);
+}
+
+// Cell tile (tx, ty): cells tx*7-1 .. tx*7+6 (and likewise in y), output pixels tx*7 .. tx*7+6,
+// slices [s0, s0 + S) (a ragged last group repeats its last slice).  Every thread of the
+// workgroup calls it.
+template <int S, typename TI, typename TO>
+__device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, int tx, int ty, int s0)
+{
+    static_assert(kCells == 64 && kWvSplit * kCells == kAdjThreads, "a tile's cells on the lanes of a wave");
+    constexpr int kDw = WvStage<S>::kDw;
+    // 16 slices: the next batch's rays are loaded into registers while the current ones are
+    // evaluated (three waves per SIMD: 1.78 against 2.16 ms for 16 slices); with fewer slices the
+    // other waves hide the loads, and the registers are worth more (1 slice 656 against 702 us)
+    constexpr bool kAhead = S == 16;
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     int lx, ly;
     tile_cell(lx, ly);
     const int ci = tx * kCellOut - 1 + lx, cj = ty * kCellOut - 1 + ly;  // >= -1
     const float fci = (float)ci, fcj = (float)cj;
+    float *slots = sh.stage[wave].slot;
     const TI *sino[S];
 #pragma unroll
     for (int s = 0; s < S; ++s)
         sino[s] = static_cast<const TI *>(A.sino) + (size_t)min(s0 + s, A.nSlices - 1) * A.sino_stride;
-    float acc[4][S];
+    // the tile's centre and this cell's offset from it (mm); cell c's centre is texel
+    // coordinate c + 1/2, at (c + 1 - r) dx
+    const float bx = ((float)(ci - lx) + 4.5f - A.r) * A.dx, by = ((float)(cj - ly) + 4.5f - A.r) * A.dx;
+    const float dxl = ((float)lx - kWvHalf) * A.dx, dyl = ((float)ly - kWvHalf) * A.dx;
+
+    // Of view vb + (lane & 15): a cell's first candidate is slot ceil(gx dxl + gy dyl + e) of the
+    // view's window, which starts at column wlo; nit candidates follow one another.
+    struct Model {
+        float gx, gy, e;
+        int nit, wlo;
+    };
+    // Models of the views [vb, min(vb + 16, vend)); returns the widest window among them.
+    auto models = [&](int vb, int vend, Model &M, int &dirs) {
+        const int v = min(vb + (lane & (kWvGroup - 1)), vend - 1);
+        const BlockCand b = block_candidates(A, A.cs[v], bx, by, kCellRho, kWvHalf * A.dx);
+        // candidates of a cell: ceil(cf - hw) and the following nit - 1 columns (no interval of
+        // length 2 hw holds more integers; 0.001 and 0.01 cover the FP32 column coordinates)
+        const float ext = kWvHalf * A.dx * (fabsf(b.gx) + fabsf(b.gy));
+        const float nit = floorf(fmaf(2.0f, b.hw, 0.001f)) + 1.0f;
+        const float lo = ceilf(b.cf - ext - b.hw - 0.01f);
+        M.gx = b.gx, M.gy = b.gy, M.e = (b.cf - lo) - b.hw;
+        M.wlo = (int)fminf(fmaxf(lo, -1.0e9f), 1.0e9f);
+        // the signs of du (1: positive, 2: negative) and dw (4, 8) that every ray in reach of the
+        // tile shares, in all the group's views (0: mixed): any slot read lies within hw + 2
+        // columns of the cell's own, and samples run towards the source, against (dx, dy)
+        const float sp = b.spread + (b.hw + 2.0f) * __builtin_amdgcn_rcpf(A.c_abs);
+        dirs = (__all(b.dx < -sp) ? 1 : 0) | (__all(b.dx > sp) ? 2 : 0) | (__all(b.dy < -sp) ? 4 : 0) |
+               (__all(b.dy > sp) ? 8 : 0);
+        M.nit = (int)fminf(nit, 1.0e9f);
+        float need = ceilf(M.e + ext + 0.01f) + nit;
+        need = need < 1.0e9f ? need : 1.0e9f;  // also for a block at the source (not a number)
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int s = 0; s < S; ++s) acc[q][s] = 0.0f;
-
-    const bool active = ci <= A.nX - 1 && cj <= A.nY - 1 && cell_in_fov(A, fci, fcj);
-    // block of 4 x 4 cells of this lane's group of 16: centre and this cell's offset (mm);
-    // cell ci's centre is texel coordinate ci + 1/2, at (ci + 1 - r) dx
-    const float bx = (float)(tx * kCellOut - 1 + (lx & ~3)) + 2.5f - A.r;  // centre, texel units
-    const float by = (float)(ty * kCellOut - 1 + (ly & ~3)) + 2.5f - A.r;
-    const float dxl = ((float)(lx & 3) - 1.5f) * A.dx, dyl = ((float)(ly & 3) - 1.5f) * A.dx;
-    // all lanes run the view loop (the models are shared by shuffles); inactive cells skip
-    // the rays, and a wave without an active cell skips it all
-    if (__any(active)) {
-        for (int vb = 0; vb < A.nViews; vb += 16) {
-            // lane j of each group of 16 evaluates the model of view vb + j
-            const int vj = min(vb + ((int)threadIdx.x & 15), A.nViews - 1);
-            const BlockCand mine = block_candidates(A, A.cs[vj], bx * A.dx, by * A.dx, kCellRho);
-            const int nv = min(16, A.nViews - vb);
-            for (int j = 0; j < nv; ++j) {
-                const BlockCand bm = block_model_of(mine, j);
-                if (!active) continue;
-                const int v = vb + j;
-                int clo, chi;
-                cell_candidates(A, bm, dxl, dyl, clo, chi);
-                // 32-bit element offsets from the tables' bases (a plan's tables hold fewer than
-                // 2^26 rays)
-                const unsigned rbase = (unsigned)v * (unsigned)A.nCols;
-                for (int c = clo; c <= chi; ++c) {
-                    const unsigned rb = rbase + (unsigned)c;
-                    const float N = (float)load_at(A.ray_n, rb * 4u);
-                    const float4 g = load_at(A.ray_geo, rb * 16u);
-                    const float2 inv = load_at(A.ray_inv, rb * 8u);
-                    const unsigned boff = rb * (unsigned)sizeof(TI);
-                    float sv[S];
-#pragma unroll
-                    for (int s = 0; s < S; ++s) sv[s] = load_f_at(sino[s], boff);
-                    cell_accumulate<S>(g, inv, N, sv, fci, fcj, acc);
-                }
-            }
-        }
-    }
-    cell_combine<S, TO>(A, part, acc, tx, ty, s0);
-}
-
-template <int S, typename TI, typename TO>
-__global__ __launch_bounds__(kAdjThreads) void fp_adjoint_cell_kernel(FpaArgs A)
-{
-    __shared__ float part[4 * (S < kCombineS ? S : kCombineS) * kCells];
-    cell_tile<S, TI, TO>(A, blockIdx.x, blockIdx.y, blockIdx.z * S, part);
-}
-
-// Staged cell tile for S >= 4 slices: the sinogram columns around the tile's candidate
-// rays are staged in LDS per batch of kStageVB views, as in the staged gather (window
-// from the tile's four corner cells), each column's ray tables packed in one 32-byte
-// record.  Per view the candidate columns run in three ascending stretches: left of the
-// window (global memory), inside it (LDS only) and right of it (global memory), so the
-// hot middle loop carries no global addressing and no branch.
-template <int S, int VB>
-struct CellStage {
-    // floats per staged column: S + 4 (a 16-byte multiple, off the bank period) for the
-    // slice groups, one value for a single slice
-    static constexpr int kPitch = S >= 4 ? S + 4 : 1;
-    float val[VB][kStageCols][kPitch];
-    // ray tables of the staged columns: (u0, w0, du, dw) and (1/du, 1/dw, N, 0), each
-    // a 16-byte record so that 16 lanes reading distinct columns hit distinct banks
-    float4 geo[VB][kStageCols];
-    float4 aux[VB][kStageCols];
-};
-
-template <int S, int VB>
-union CellShared {
-    CellStage<S, VB> stage;
-    float part[4 * (S < kCombineS ? S : kCombineS) * kCells];
-};
-
-// VB views per staging batch (VB <= 16: lanes 4m + c evaluate the window corners).
-// S = 1 (the uneven batch's slices): wave 2 stages the values.
-template <int S, int VB, typename TI, typename TO>
-__device__ __forceinline__ void cell_staged_tile(const FpaArgs &A, CellShared<S, VB> &sh, int tx, int ty, int s0)
-{
-    static_assert(S == 1 || S % 4 == 0, "a staged column is read four slices at a time");
-    static_assert(VB >= 1 && VB <= 16, "window corners of at most 16 views per batch");
-    constexpr int SQ = S >= 4 ? S / 4 : 1;  // slices staged per wave
-    CellStage<S, VB> &st = sh.stage;
-    int lx, ly;
-    tile_cell(lx, ly);
-    const int ci = tx * kCellOut - 1 + lx, cj = ty * kCellOut - 1 + ly;  // >= -1
-    // no early exit: every thread stages and waits
-    const bool active = ci <= A.nX - 1 && cj <= A.nY - 1 && cell_in_fov(A, (float)ci, (float)cj);
-    const int lane = (int)threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const float fci = (float)ci, fcj = (float)cj;
-    const float x = (fci + 1.0f - A.r) * A.dx;
-    const float y = (fcj + 1.0f - A.r) * A.dx;
-    // corner cell of this lane for the window: lane 4m + c evaluates corner c
-    const int wci = (lane & 1) ? min(tx * kCellOut + kCellOut - 1, A.nX - 1) : tx * kCellOut - 1;
-    const int wcj = (lane & 2) ? min(ty * kCellOut + kCellOut - 1, A.nY - 1) : ty * kCellOut - 1;
-    const float cx = ((float)wci + 1.0f - A.r) * A.dx;
-    const float cy = ((float)wcj + 1.0f - A.r) * A.dx;
-    // the group's slices are addressed from its first one by 32-bit byte offsets (the
-    // launch checks that S sinograms span less than 4 GiB); a ragged last group repeats
-    // its last slice
-    const TI *gbase = static_cast<const TI *>(A.sino) + (size_t)s0 * A.sino_stride;
-    const int last = A.nSlices - 1 - s0;
-    const unsigned sbytes = (unsigned)A.sino_stride * (unsigned)sizeof(TI);
+        for (int sh2 = 1; sh2 < kWvGroup; sh2 <<= 1) need = fmaxf(need, __shfl_xor(need, sh2));
+        return __builtin_amdgcn_readfirstlane((int)need);
+    };
+    auto lane_f = [](float x, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), k)); };
 
     float acc[4][S];
+    float4 pg;  // the slot's next ray: u0, w0, du, dw,
+    float2 pi;  // 1/du, 1/dw,
+    int pn;     // samples,
+    TI pv[S];   // and its values (storage bits: widened when they are written to LDS)
+    auto load_ray = [&](bool ok, int v, int c) {
+        pg = make_float4(0.0f, 0.0f, 0.0f, 0.0f), pi = make_float2(0.0f, 0.0f), pn = 0;
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+        for (int s = 0; s < S; ++s) pv[s] = 0;
+        if (ok) {
+            const unsigned rb = (unsigned)v * (unsigned)A.nCols + (unsigned)c;
+            pg = A.ray_geo[rb];
+            pi = A.ray_inv[rb];
+            pn = A.ray_n[rb];
 #pragma unroll
-        for (int s = 0; s < S; ++s) acc[q][s] = 0.0f;
-
-    // a candidate column outside the staged window (rare): tables and values from global
-    // memory, one slice at a time so that the path holds few registers (the scheduling
-    // barrier keeps the loads from being hoisted together); the same FMAs as
-    // cell_accumulate
-    auto global_ray = [&](int v, int c) {
-        const size_t rb = (size_t)v * A.nCols + c;
-        float r[4];
-        const float4 g = A.ray_geo[rb];
-        cell_sums(g, A.ray_inv[rb], (float)A.ray_n[rb], fci, fcj, r);
-        unsigned off = (unsigned)rb * (unsigned)sizeof(TI);
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const float val = load_f_at(gbase, off);
-            if (s < last) off += sbytes;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[q][s] = fmaf(r[q], val, acc[q][s]);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int s = 0; s < S; ++s) pv[s] = sino[s][rb];
         }
     };
-
-    // Staging is software-pipelined: while a batch is evaluated from LDS, the next batch's
-    // values and ray records are loaded into registers (each wave SQ slices of every
-    // view's columns, and the records of the views m = wave mod 4), and written to LDS
-    // between the two barriers that follow.
-    constexpr int kRecViews = (VB + 3) / 4;  // views whose records one wave loads
-    auto window = [&](int v0, int (&c_lo)[VB]) {
-        int wlo, whi;
-        candidate_rays(A, A.cs[min(v0 + (lane >> 2) % VB, A.nViews - 1)], cx, cy, kCellRho, wlo, whi);
+    auto store_ray = [&]() {
+        float *d = slots + lane * kDw;
+        const float n = (float)pn, dd = pg.z * pg.w * (1.0f / 12.0f);
+        *reinterpret_cast<float4 *>(d) = pg;
+        *reinterpret_cast<float4 *>(d + 4) = make_float4(pi.x, pi.y, -pg.x * pi.x, -pg.y * pi.y);
+        if constexpr (S >= 4) {
+            *reinterpret_cast<float2 *>(d + 8) = make_float2(n, dd);
 #pragma unroll
-        for (int sh2 = 1; sh2 <= 2; sh2 <<= 1) wlo = min(wlo, __shfl_xor(wlo, sh2));
-#pragma unroll
-        for (int m = 0; m < VB; ++m)
-            c_lo[m] = min(max(__builtin_amdgcn_readlane(wlo, 4 * m) - 1, 0), max(A.nCols - kStageCols, 0));
+            for (int s = 0; s < S; s += 4)
+                *reinterpret_cast<float4 *>(d + 12 + s) =
+                    make_float4(widen(pv[s]), widen(pv[s + 1]), widen(pv[s + 2]), widen(pv[s + 3]));
+        } else {
+            *reinterpret_cast<float4 *>(d + 8) = make_float4(n, dd, widen(pv[0]), widen(pv[S - 1]));
+        }
+        // the wave's lanes read each other's slots: keep the order, LDS keeps it too
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     };
-    TI pv[VB][SQ];                // next batch: this wave's values of lane's column (storage bits)
-    float4 pg[kRecViews];         // its ray records: geo
-    float2 pi[kRecViews];         //   1 / steps
-    int pn[kRecViews];            //   samples
-    auto load_batch = [&](int v0, const int (&c_lo)[VB]) {
+    struct Ray {
+        RayRec rec;
+        float v[S];
+    };
+    auto read_ray = [&](const float *d, Ray &r) {
+        r.rec.p = *reinterpret_cast<const float4 *>(d);
+        r.rec.q = *reinterpret_cast<const float4 *>(d + 4);
+        if constexpr (S >= 4) {
+            r.rec.n = *reinterpret_cast<const float2 *>(d + 8);
 #pragma unroll
-        for (int m = 0; m < VB; ++m) {
-            const int c = min(c_lo[m] + lane, A.nCols - 1);
-            const unsigned boff = (unsigned)((size_t)min(v0 + m, A.nViews - 1) * A.nCols + c) * (unsigned)sizeof(TI);
-            if constexpr (S == 1) {
-                if (wave == 0) pv[m][0] = load_at(gbase, boff);
-            } else {
-#pragma unroll
-                for (int q = 0; q < SQ; ++q)
-                    pv[m][q] = load_at(gbase, (unsigned)min(wave * SQ + q, last) * sbytes + boff);
+            for (int s = 0; s < S; s += 4) {
+                const float4 t4 = *reinterpret_cast<const float4 *>(d + 12 + s);
+                r.v[s] = t4.x, r.v[s + 1] = t4.y, r.v[s + 2] = t4.z, r.v[s + 3] = t4.w;
             }
-        }
-#pragma unroll
-        for (int r = 0; r < kRecViews; ++r) {
-            const int m = wave + 4 * r;
-            if (m >= VB) break;
-            const int c = min(c_lo[m] + lane, A.nCols - 1);
-            const size_t rb = (size_t)min(v0 + m, A.nViews - 1) * A.nCols + c;
-            pg[r] = A.ray_geo[rb];
-            pi[r] = A.ray_inv[rb];
-            pn[r] = A.ray_n[rb];
+        } else {
+            const float4 t4 = *reinterpret_cast<const float4 *>(d + 8);
+            r.rec.n = make_float2(t4.x, t4.y);
+            r.v[0] = t4.z;
+            if constexpr (S == 2) r.v[1] = t4.w;
         }
     };
-    auto store_batch = [&](int v0, const int (&c_lo)[VB]) {
+    float ulo = fci, uhi = fci + 1.0f, wlo = fcj, whi = fcj + 1.0f;  // boundaries in the order of the group's rays
+    auto add_ray = [&](auto mixed, const Ray &ray) {
+        constexpr bool kMixed = decltype(mixed)::value;
+        const CellSums c = cell_sums<kMixed>(ray.rec, fci, fcj, kMixed ? fci : ulo, kMixed ? fci + 1.0f : uhi,
+                                             kMixed ? fcj : wlo, kMixed ? fcj + 1.0f : whi);
+        if constexpr (S <= 2) {
 #pragma unroll
-        for (int m = 0; m < VB; ++m) {
-            if (v0 + m >= A.nViews || c_lo[m] + lane >= A.nCols) continue;
-            if constexpr (S == 1) {
-                if (wave == 0) st.val[m][lane][0] = widen(pv[m][0]);
-            } else {
-                float *dst = &st.val[m][lane][wave * SQ];  // this wave's SQ slots of the column
-                if constexpr (SQ % 4 == 0) {
-#pragma unroll
-                    for (int q = 0; q < SQ; q += 4)
-                        *reinterpret_cast<float4 *>(dst + q) = make_float4(
-                            widen(pv[m][q]), widen(pv[m][q + 1]), widen(pv[m][q + 2]), widen(pv[m][q + 3]));
-                } else if constexpr (SQ == 2) {
-                    *reinterpret_cast<float2 *>(dst) = make_float2(widen(pv[m][0]), widen(pv[m][1]));
-                } else {
-#pragma unroll
-                    for (int q = 0; q < SQ; ++q) dst[q] = widen(pv[m][q]);
-                }
+            for (int s = 0; s < S; ++s) {
+                const float nv = c.n * ray.v[s];
+                acc[0][s] += nv;
+                acc[1][s] = fmaf(c.ta, nv, acc[1][s]);
+                acc[2][s] = fmaf(c.tm, nv, acc[2][s]);
+                acc[3][s] = fmaf(c.g, nv, acc[3][s]);
             }
-        }
+        } else {
+            const float r[4] = {c.n, c.n * c.ta, c.n * c.tm, c.n * c.g};
 #pragma unroll
-        for (int r = 0; r < kRecViews; ++r) {
-            const int m = wave + 4 * r;
-            if (m >= VB || v0 + m >= A.nViews || c_lo[m] + lane >= A.nCols) continue;
-            st.geo[m][lane] = pg[r];
-            st.aux[m][lane] = make_float4(pi[r].x, pi[r].y, (float)pn[r], 0.0f);
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int s = 0; s < S; ++s) acc[q][s] = fmaf(r[q], ray.v[s], acc[q][s]);
+        }
+    };
+    // nit >= 1 adjacent slots from d
+    auto add_rays = [&](auto mixed, const float *d, int nit) {
+        if constexpr (S <= 2) {  // two rays in flight
+            for (; nit > 1; nit -= 2, d += 2 * kDw) {
+                Ray r0, r1;
+                read_ray(d, r0);
+                read_ray(d + kDw, r1);
+                add_ray(mixed, r0);
+                add_ray(mixed, r1);
+            }
+            if (nit > 0) {
+                Ray r;
+                read_ray(d, r);
+                add_ray(mixed, r);
+            }
+        } else {
+            do {
+                Ray r;
+                read_ray(d, r);
+                add_ray(mixed, r);
+                d += kDw;
+            } while (--nit > 0);
         }
     };
 
-    int c_lo[VB], c_nx[VB];
-    window(0, c_nx);
-    load_batch(0, c_nx);
-    for (int v0 = 0; v0 < A.nViews; v0 += VB) {
-#pragma unroll
-        for (int m = 0; m < VB; ++m) c_lo[m] = c_nx[m];
-        __syncthreads();  // the previous batch's reads are done
-        store_batch(v0, c_lo);
-        __syncthreads();
-        if (v0 + VB < A.nViews) {
-            window(v0 + VB, c_nx);
-            load_batch(v0 + VB, c_nx);
-        }
-        if (!active) continue;
-        // (each cell evaluates its own candidates here: the shared block model of the
-        // unstaged tile ran 3.5% slower in this kernel, which holds more registers)
-#pragma unroll 1
-        for (int m = 0; m < VB; ++m) {
-            const int v = v0 + m;
-            if (v >= A.nViews) break;
-            int clo, chi;
-            candidate_rays(A, A.cs[v], x, y, kCellRho, clo, chi);
-            const int wlo = c_lo[m], whi = c_lo[m] + kStageCols - 1;  // staged window
-            int c = clo;
-            for (; c <= min(chi, wlo - 1); ++c) global_ray(v, c);
-            for (; c <= min(chi, whi); ++c) {
-                const int lc = c - wlo;
-                // the ray record is read before the values: LDS reads complete in order,
-                // so the sums can run while the values are still in flight
-                const float4 ax = st.aux[m][lc];
-                const float4 gg = st.geo[m][lc];
-                float sv[S];
-                if constexpr (S == 1) {
-                    sv[0] = st.val[m][lc][0];
-                } else {
-#pragma unroll
-                    for (int s = 0; s < S; s += 4) {
-                        const float4 t4 = *reinterpret_cast<const float4 *>(&st.val[m][lc][s]);
-                        sv[s] = t4.x, sv[s + 1] = t4.y, sv[s + 2] = t4.z, sv[s + 3] = t4.w;
+    // Sums of the views [v_begin, v_end) into acc.
+    auto run = [&](int v_begin, int v_end) {
+        Model M;
+        int dirs;
+        int need = models(v_begin, v_end, M, dirs);
+        int wd, nv, lm, lc;  // window width, views per batch, this lane's view and column in them
+        auto set_window = [&]() {
+            nv = __builtin_amdgcn_readfirstlane(need <= 16 ? 4 : need <= 21 ? 3 : need <= 32 ? 2 : 1);
+            wd = __builtin_amdgcn_readfirstlane(need <= 16 ? 16 : need <= 21 ? 21 : need <= 32 ? 32 : 64);
+            lm = (int)(lane >= wd) + (int)(lane >= 2 * wd) + (int)(lane >= 3 * wd);
+            lc = lane - lm * wd;
+        };
+        auto load_batch = [&](int vb, int v0, int gend) {
+            const int v = v0 + lm;
+            const int c = __shfl(M.wlo, min(v - vb, kWvGroup - 1)) + lc;
+            load_ray(lm < nv && v < gend && (unsigned)c < (unsigned)A.nCols, v, c);
+        };
+        set_window();
+        if (kAhead && need <= kWvSlots) load_batch(v_begin, v_begin, min(v_begin + kWvGroup, v_end));
+        for (int vb = v_begin; vb < v_end; vb += kWvGroup) {
+            const int gend = min(vb + kWvGroup, v_end), vn = gend;
+            const Model C = M;
+            if (need <= kWvSlots) {
+                const int cwd = wd, cnv = nv, cdirs = dirs;
+                ulo = cdirs & 2 ? fci + 1.0f : fci, uhi = cdirs & 2 ? fci : fci + 1.0f;
+                wlo = cdirs & 8 ? fcj + 1.0f : fcj, whi = cdirs & 8 ? fcj : fcj + 1.0f;
+                auto group = [&](auto mixed) {
+                    for (int v0 = vb; v0 < gend; v0 += cnv) {
+                        if (!kAhead) load_batch(vb, v0, gend);
+                        store_ray();
+                        if constexpr (kAhead) {
+                            if (v0 + cnv < gend) {
+                                load_batch(vb, v0 + cnv, gend);
+                            } else if (vn < v_end) {  // the next group's models and first batch
+                                need = models(vn, v_end, M, dirs);
+                                set_window();
+                                if (need <= kWvSlots) load_batch(vn, vn, min(vn + kWvGroup, v_end));
+                            }
+                        }
+                        const int nb = min(cnv, gend - v0);
+                        for (int m = 0; m < nb; ++m) {
+                            const int k = v0 + m - vb;
+                            const float f = fmaf(lane_f(C.gx, k), dxl, fmaf(lane_f(C.gy, k), dyl, lane_f(C.e, k)));
+                            add_rays(mixed, slots + ((int)ceilf(f) + m * cwd) * kDw, __builtin_amdgcn_readlane(C.nit, k));
+                        }
+                    }
+                };
+                // (one copy of the loop for 16 slices: the other costs a wave per SIMD)
+                if (S < 16 && (cdirs & 3) && (cdirs & 12)) group(std::false_type{});
+                else group(std::true_type{});
+            } else {
+                // windows wider than the slots: 64 columns at a time, each cell's range per lane
+                for (int v = vb; v < gend; ++v) {
+                    const BlockCand b = block_candidates(A, A.cs[v], bx, by, kCellRho, kWvHalf * A.dx);
+                    const float cf = fmaf(b.gx, dxl, fmaf(b.gy, dyl, b.cf));
+                    const int clo = (int)fmaxf(ceilf(cf - b.hw), 0.0f);
+                    const int chi = (int)fminf(floorf(cf + b.hw), (float)(A.nCols - 1));
+                    const float ext = kWvHalf * A.dx * (fabsf(b.gx) + fabsf(b.gy)) + b.hw + 0.01f;
+                    const int wlo = __builtin_amdgcn_readfirstlane((int)fmaxf(ceilf(b.cf - ext), 0.0f));
+                    const int whi = __builtin_amdgcn_readfirstlane((int)fminf(floorf(b.cf + ext), (float)(A.nCols - 1)));
+                    for (int w = wlo; w <= whi; w += kWvSlots) {
+                        load_ray(w + lane < A.nCols, v, w + lane);
+                        store_ray();
+                        for (int c = max(clo, w); c <= min(chi, w + kWvSlots - 1); ++c) {
+                            Ray r;
+                            read_ray(slots + (c - w) * kDw, r);
+                            add_ray(std::true_type{}, r);
+                        }
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
                     }
                 }
-                __builtin_amdgcn_sched_barrier(0);  // keep all the reads ahead of the sums
-                cell_accumulate<S>(gg, make_float2(ax.x, ax.y), ax.z, sv, fci, fcj, acc);
+                if (kAhead && vn < v_end) {
+                    need = models(vn, v_end, M, dirs);
+                    set_window();
+                    if (need <= kWvSlots) load_batch(vn, vn, min(vn + kWvGroup, v_end));
+                }
             }
-            for (; c <= chi; ++c) global_ray(v, c);
+            if (!kAhead && vn < v_end) {
+                need = models(vn, v_end, M, dirs);
+                set_window();
+            }
         }
+    };
+
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int s = 0; s < S; ++s) acc[q][s] = 0.0f;
+    // cells outside the FOV disk hold no samples; a tile without any other cell skips the views
+    if (__any(ci <= A.nX - 1 && cj <= A.nY - 1 && cell_in_fov(A, fci, fcj))) {
+        const int v0 = view_quarter(A.nViews, wave), v1 = view_quarter(A.nViews, wave + 1);
+        if (v0 < v1) run(v0, v1);
     }
-    __syncthreads();  // staging reads are done: the union turns into corner weights
-    cell_combine<S, TO>(A, sh.part, acc, tx, ty, s0);
+    __syncthreads();  // the staging space turns into partial sums
+    constexpr int kC = CellShared<S>::kC;
+#pragma unroll
+    for (int sb = 0; sb < S; sb += kCombineS) {
+        if (wave > 0) {
+            float *mine = sh.part + (wave - 1) * 4 * kC * kCells + lane;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int k = 0; k < kC; ++k) mine[(q * kC + k) * kCells] = acc[q][sb + k];
+        }
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int k = 0; k < kC; ++k) {
+                    const float *p = sh.part + (q * kC + k) * kCells + lane;
+                    constexpr int kG = 4 * kC * kCells;
+                    acc[q][sb + k] = (acc[q][sb + k] + p[0]) + (p[kG] + p[2 * kG]);
+                }
+        }
+        __syncthreads();
+    }
+    cell_combine<S, TO>(A, sh.part, acc, tx, ty, s0, wave == 0);
 }
 
+// Waves per SIMD that the registers are held to: one slice 667, 662, 668 us at 5, 6, 8; four 878,
+// 835, 1234 (spills) at 5, 6, 8.
 template <int S, typename TI, typename TO>
-__global__ __launch_bounds__(kAdjThreads) void fp_adjoint_cell_staged_kernel(FpaArgs A)
+__global__ __launch_bounds__(kAdjThreads, S == 16 ? 2 : S == 8 ? 4 : 6) void fp_adjoint_cell_kernel(FpaArgs A, int slice0)
 {
-    __shared__ CellShared<S, kStageVB> sh;
+    __shared__ CellShared<S> sh;
     unsigned tx, ty, g;  // blocked, XCD-aware order (neighbouring tiles share staged columns in L2)
     xcd_blocked_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, gridDim.z,
                      tx, ty, g);
-    cell_staged_tile<S, kStageVB, TI, TO>(A, sh, (int)tx, (int)ty, (int)g * S);
+    cell_tile<S, TI, TO>(A, sh, (int)tx, (int)ty, slice0 + (int)g * S);
 }
 
 // Uneven batch: slice s has its own geometry (desc[s]); work item = (slice, tile), items
@@ -878,16 +933,13 @@ __global__ __launch_bounds__(kAdjThreads) void fp_adjoint_cell_staged_kernel(Fpa
 // [-1, n-1] takes 15 x 15-pixel cell tiles, as a single-slice call does; any other slice
 // TX x (256/TX) gather tiles.  A fixed grid strides over all items, the XCDs taking
 // them in chunks of 64, and a slice's tiles run in blocked order, so the tiles resident
-// on one XCD cover a compact part of one image and share their rays through its L2.  VB > 0: the cell tiles stage their sinogram columns and ray records
-// in LDS, VB views per batch (the same arithmetic in the same order as the unstaged
-// tile, VB = 0).
-template <int TX, int VB, typename TI, typename TO>
-__global__ __launch_bounds__(kAdjThreads) void fp_adjoint_batch_kernel(const FpaSliceDesc *__restrict__ desc,
+// on one XCD cover a compact part of one image and share their rays through its L2.
+template <int TX, typename TI, typename TO>
+__global__ __launch_bounds__(kAdjThreads, 6) void fp_adjoint_batch_kernel(const FpaSliceDesc *__restrict__ desc,
                                                                        const int *__restrict__ prefix, int n,
                                                                        int total, const TI *sino, TO *img)
 {
-    __shared__ CellShared<1, (VB > 0 ? VB : 1)> sh;
-    float *part = sh.part;
+    __shared__ CellShared<1> sh;
     const int first = (int)xcd_chunk(blockIdx.x, gridDim.x);
     for (int item = first; item < total; item += gridDim.x) {
         int lo = 0, hi = n - 1;  // last slice with prefix[s] <= item
@@ -926,8 +978,7 @@ __global__ __launch_bounds__(kAdjThreads) void fp_adjoint_batch_kernel(const Fpa
         unsigned tx, ty;
         if (adj_cells_fit(A.far_x, A.far_y)) {  // same test as the single-slice launch
             blocked_tile(local, adj_cell_tiles(A.nX), adj_cell_tiles(A.nY), tx, ty);
-            if constexpr (VB > 0) cell_staged_tile<1, VB, TI, TO>(A, sh, (int)tx, (int)ty, 0);
-            else cell_tile<1, TI, TO>(A, (int)tx, (int)ty, 0, part);
+            cell_tile<1, TI, TO>(A, sh, (int)tx, (int)ty, 0);
         } else {
             blocked_tile(local, (A.nX + TX - 1) / TX, (A.nY + 256 / TX - 1) / (256 / TX), tx, ty);
             adjoint_tile<1, TX, TI, TO>(A, (int)tx, (int)ty, 0);
@@ -938,28 +989,28 @@ __global__ __launch_bounds__(kAdjThreads) void fp_adjoint_batch_kernel(const Fpa
 }  // namespace
 
 template <int S, typename TI, typename TO>
-static void launch_fpa_k(dim3 grid, hipStream_t stream, const FpaArgs &A)
+static void launch_fpa_k(int groups, hipStream_t stream, const FpaArgs &A, int slice0)
 {
-    if (adj_cells_fit(A.far_x, A.far_y) && (S < 4 || (long long)S * A.sino_stride * (long long)sizeof(TI) < (1LL << 32))) {
-        const dim3 cg(adj_cell_tiles(A.nX), adj_cell_tiles(A.nY), grid.z);
-        if constexpr (S >= 4)
-            hipLaunchKernelGGL((fp_adjoint_cell_staged_kernel<S, TI, TO>), cg, dim3(kAdjThreads), 0, stream, A);
-        else
-            hipLaunchKernelGGL((fp_adjoint_cell_kernel<S, TI, TO>), cg, dim3(kAdjThreads), 0, stream, A);
-    } else if constexpr (S >= 4) {
-        hipLaunchKernelGGL((fp_adjoint_staged_kernel<S, TI, TO>), grid, dim3(kAdjThreads), 0, stream, A);
-    } else {
-        hipLaunchKernelGGL((fp_adjoint_kernel<S, TI, TO>), grid, dim3(kAdjThreads), 0, stream, A);
+    if (adj_cells_fit(A.far_x, A.far_y)) {
+        const dim3 grid(adj_cell_tiles(A.nX), adj_cell_tiles(A.nY), groups);
+        hipLaunchKernelGGL((fp_adjoint_cell_kernel<S, TI, TO>), grid, dim3(kAdjThreads), 0, stream, A, slice0);
+        return;
     }
+    const dim3 grid((A.nX + kAdjTx - 1) / kAdjTx, (A.nY + kAdjTy - 1) / kAdjTy, groups);
+    if constexpr (S >= 4)
+        hipLaunchKernelGGL((fp_adjoint_staged_kernel<S, TI, TO>), grid, dim3(kAdjThreads), 0, stream, A);
+    else
+        hipLaunchKernelGGL((fp_adjoint_kernel<S, TI, TO>), grid, dim3(kAdjThreads), 0, stream, A);
 }
 
 template <int S>
-static fbct_status launch_fpa_t(fbct_dtype ti, fbct_dtype to, dim3 grid, hipStream_t stream, const FpaArgs &A)
+static fbct_status launch_fpa_t(fbct_dtype ti, fbct_dtype to, int groups, hipStream_t stream, const FpaArgs &A,
+                                int slice0)
 {
-    if (ti == FBCT_F32 && to == FBCT_F32) launch_fpa_k<S, float, float>(grid, stream, A);
-    else if (ti == FBCT_BF16 && to == FBCT_F32) launch_fpa_k<S, bf16_t, float>(grid, stream, A);
-    else if (ti == FBCT_F32 && to == FBCT_BF16) launch_fpa_k<S, float, bf16_t>(grid, stream, A);
-    else if (ti == FBCT_BF16 && to == FBCT_BF16) launch_fpa_k<S, bf16_t, bf16_t>(grid, stream, A);
+    if (ti == FBCT_F32 && to == FBCT_F32) launch_fpa_k<S, float, float>(groups, stream, A, slice0);
+    else if (ti == FBCT_BF16 && to == FBCT_F32) launch_fpa_k<S, bf16_t, float>(groups, stream, A, slice0);
+    else if (ti == FBCT_F32 && to == FBCT_BF16) launch_fpa_k<S, float, bf16_t>(groups, stream, A, slice0);
+    else if (ti == FBCT_BF16 && to == FBCT_BF16) launch_fpa_k<S, bf16_t, bf16_t>(groups, stream, A, slice0);
     else return fail(FBCT_ERR_INVALID_ARGUMENT, "fbct_fp_adjoint: unknown storage type");
     return FBCT_OK;
 }
@@ -990,21 +1041,33 @@ fbct_status launch_fp_adjoint(const fbct_plan &p, const DeviceTables &t, const v
     A.c_abs = fabsf(p.d.fpa_c_scale);
     A.far_x = p.d.fpa_far_x;
     A.far_y = p.d.fpa_far_y;
-    const unsigned gx = (p.g.nX + kAdjTx - 1) / kAdjTx, gy = (p.g.nY + kAdjTy - 1) / kAdjTy;
-    // Slices that share the geometry are processed together when there are enough
-    // workgroups left to fill the device.
-    const long long tiles = (long long)gx * gy;
-    fbct_status st;
-    if (n >= 16 && tiles * ((n + 15) / 16) >= 1024)
-        st = launch_fpa_t<16>(ti, to, dim3(gx, gy, (n + 15) / 16), stream, A);
-    else if (n >= 8 && tiles * ((n + 7) / 8) >= 1024)
-        st = launch_fpa_t<8>(ti, to, dim3(gx, gy, (n + 7) / 8), stream, A);
-    else if (n >= 4 && tiles * ((n + 3) / 4) >= 1024)
-        st = launch_fpa_t<4>(ti, to, dim3(gx, gy, (n + 3) / 4), stream, A);
-    else if (n >= 2 && tiles * ((n + 1) / 2) >= 1024)
-        st = launch_fpa_t<2>(ti, to, dim3(gx, gy, (n + 1) / 2), stream, A);
-    else
-        st = launch_fpa_t<1>(ti, to, dim3(gx, gy, n), stream, A);
+    const long long gx = (p.g.nX + kAdjTx - 1) / kAdjTx, gy = (p.g.nY + kAdjTy - 1) / kAdjTy;
+    fbct_status st = FBCT_OK;
+    if (adj_cells_fit(A.far_x, A.far_y)) {
+        // groups of 16 slices, the rest in groups of the next size up, padded with the last slice
+        // (512 x 512: 1, 2, 4, 8, 16 slices take 603, 656, 835, 1117, 1780 us, so that 11 to 15 go
+        // as 16, but 9 and 10 as 8 and the rest)
+        for (int done = 0; done < n && st == FBCT_OK;) {
+            const int left = n - done;
+            const int S = left >= 11 ? 16 : left >= 5 ? 8 : left >= 3 ? 4 : left;
+            const int groups = std::max(left / S, 1);
+            if (S == 16) st = launch_fpa_t<16>(ti, to, groups, stream, A, done);
+            else if (S == 8) st = launch_fpa_t<8>(ti, to, groups, stream, A, done);
+            else if (S == 4) st = launch_fpa_t<4>(ti, to, groups, stream, A, done);
+            else if (S == 2) st = launch_fpa_t<2>(ti, to, groups, stream, A, done);
+            else st = launch_fpa_t<1>(ti, to, groups, stream, A, done);
+            done += groups * S;
+        }
+    } else {
+        // Slices that share the geometry are processed together when there are enough
+        // workgroups left to fill the device.
+        const long long tiles = gx * gy;
+        if (n >= 16 && tiles * ((n + 15) / 16) >= 1024) st = launch_fpa_t<16>(ti, to, (n + 15) / 16, stream, A, 0);
+        else if (n >= 8 && tiles * ((n + 7) / 8) >= 1024) st = launch_fpa_t<8>(ti, to, (n + 7) / 8, stream, A, 0);
+        else if (n >= 4 && tiles * ((n + 3) / 4) >= 1024) st = launch_fpa_t<4>(ti, to, (n + 3) / 4, stream, A, 0);
+        else if (n >= 2 && tiles * ((n + 1) / 2) >= 1024) st = launch_fpa_t<2>(ti, to, (n + 1) / 2, stream, A, 0);
+        else st = launch_fpa_t<1>(ti, to, n, stream, A, 0);
+    }
     if (st != FBCT_OK) return st;
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "fp_adjoint_kernel launch: %s", hipGetErrorString(e));
@@ -1012,26 +1075,21 @@ fbct_status launch_fp_adjoint(const fbct_plan &p, const DeviceTables &t, const v
 }
 
 template <int TX, typename TI, typename TO>
-static void launch_fpa_batch_t(int vb, dim3 grid, hipStream_t stream, const BatchDevice &bd, const int *prefix, int n,
+static void launch_fpa_batch_t(dim3 grid, hipStream_t stream, const BatchDevice &bd, const int *prefix, int n,
                                int total, const void *sino, void *img)
 {
-    const TI *si = static_cast<const TI *>(sino);
-    TO *io = static_cast<TO *>(img);
-    switch (vb) {
-    case 4: hipLaunchKernelGGL((fp_adjoint_batch_kernel<TX, 4, TI, TO>), grid, dim3(kAdjThreads), 0, stream, bd.fpa_desc, prefix, n, total, si, io); break;
-    case 8: hipLaunchKernelGGL((fp_adjoint_batch_kernel<TX, 8, TI, TO>), grid, dim3(kAdjThreads), 0, stream, bd.fpa_desc, prefix, n, total, si, io); break;
-    default: hipLaunchKernelGGL((fp_adjoint_batch_kernel<TX, 0, TI, TO>), grid, dim3(kAdjThreads), 0, stream, bd.fpa_desc, prefix, n, total, si, io); break;
-    }
+    hipLaunchKernelGGL((fp_adjoint_batch_kernel<TX, TI, TO>), grid, dim3(kAdjThreads), 0, stream, bd.fpa_desc, prefix, n,
+                       total, static_cast<const TI *>(sino), static_cast<TO *>(img));
 }
 
 template <int TX>
-static void launch_fpa_batch_x(fbct_dtype ti, fbct_dtype to, int vb, dim3 grid, hipStream_t stream,
-                               const BatchDevice &bd, const int *prefix, int n, int total, const void *sino, void *img)
+static void launch_fpa_batch_x(fbct_dtype ti, fbct_dtype to, dim3 grid, hipStream_t stream, const BatchDevice &bd,
+                               const int *prefix, int n, int total, const void *sino, void *img)
 {
-    if (ti == FBCT_F32 && to == FBCT_F32) launch_fpa_batch_t<TX, float, float>(vb, grid, stream, bd, prefix, n, total, sino, img);
-    else if (ti == FBCT_BF16 && to == FBCT_F32) launch_fpa_batch_t<TX, bf16_t, float>(vb, grid, stream, bd, prefix, n, total, sino, img);
-    else if (ti == FBCT_F32 && to == FBCT_BF16) launch_fpa_batch_t<TX, float, bf16_t>(vb, grid, stream, bd, prefix, n, total, sino, img);
-    else launch_fpa_batch_t<TX, bf16_t, bf16_t>(vb, grid, stream, bd, prefix, n, total, sino, img);
+    if (ti == FBCT_F32 && to == FBCT_F32) launch_fpa_batch_t<TX, float, float>(grid, stream, bd, prefix, n, total, sino, img);
+    else if (ti == FBCT_BF16 && to == FBCT_F32) launch_fpa_batch_t<TX, bf16_t, float>(grid, stream, bd, prefix, n, total, sino, img);
+    else if (ti == FBCT_F32 && to == FBCT_BF16) launch_fpa_batch_t<TX, float, bf16_t>(grid, stream, bd, prefix, n, total, sino, img);
+    else launch_fpa_batch_t<TX, bf16_t, bf16_t>(grid, stream, bd, prefix, n, total, sino, img);
 }
 
 fbct_status launch_fp_adjoint_batch(const fbct_batch &b, const BatchDevice &bd, const void *sino, fbct_dtype ti,
@@ -1048,12 +1106,11 @@ fbct_status launch_fp_adjoint_batch(const fbct_batch &b, const BatchDevice &bd, 
                               : std::min<long long>(total, (long long)b.shape.adj_wgs_per_cu * bd.num_cu);
     const dim3 grid((unsigned)wgs);
     const int *prefix = bd.fpa_prefix[k];
-    const int vb = b.shape.adj_stage_views;
     switch (b.shape.adj_tile_x) {
-    case 8: launch_fpa_batch_x<8>(ti, to, vb, grid, stream, bd, prefix, n, total, sino, img); break;
-    case 32: launch_fpa_batch_x<32>(ti, to, vb, grid, stream, bd, prefix, n, total, sino, img); break;
-    case 64: launch_fpa_batch_x<64>(ti, to, vb, grid, stream, bd, prefix, n, total, sino, img); break;
-    default: launch_fpa_batch_x<16>(ti, to, vb, grid, stream, bd, prefix, n, total, sino, img); break;
+    case 8: launch_fpa_batch_x<8>(ti, to, grid, stream, bd, prefix, n, total, sino, img); break;
+    case 32: launch_fpa_batch_x<32>(ti, to, grid, stream, bd, prefix, n, total, sino, img); break;
+    case 64: launch_fpa_batch_x<64>(ti, to, grid, stream, bd, prefix, n, total, sino, img); break;
+    default: launch_fpa_batch_x<16>(ti, to, grid, stream, bd, prefix, n, total, sino, img); break;
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "fp_adjoint_batch_kernel launch: %s", hipGetErrorString(e));

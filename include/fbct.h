@@ -280,12 +280,11 @@ typedef struct fbct_batch_shape {
                                0: one workgroup per work item                       */
     int32_t adj_tile_x;     /* FP^T pixel tile width: 8, 16, 32 or 64 (height 256/w), for
                                slices whose FP samples reach beyond the cells [-1, n-1];
-                               other slices take fixed 15 x 15-pixel cell tiles      */
+                               other slices take fixed 7 x 7-pixel cell tiles        */
     int32_t adj_wgs_per_cu; /* FP^T workgroups per compute unit in the grid, 1..32;
                                0: one workgroup per work item                       */
-    int32_t adj_stage_views; /* FP^T cell tiles: views per LDS staging batch of the
-                               sinogram columns and ray records, 4 or 8; 0: no
-                               staging (rays read from global memory)               */
+    int32_t adj_stage_views; /* 0, 4 or 8: accepted for callers that set it, without
+                               effect (cell tiles stage their rays for themselves)  */
 } fbct_batch_shape;
 
 fbct_status fbct_batch_create(fbct_plan *const *plans, int n_slices, fbct_batch **out);
