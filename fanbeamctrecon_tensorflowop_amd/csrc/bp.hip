@@ -24,6 +24,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <type_traits>
 
@@ -493,16 +494,24 @@ __global__ __launch_bounds__(kBpTx *kBpTy *VG) void bp_staged_kernel(BpArgs A, i
 // scatter with the forward kernels' coordinate would leave.  Sums are FP32 over the lines
 // of a chunk and FP64 across chunks, for the same reason.
 //
-// Work: a workgroup takes 64 adjacent columns (one per lane) of 8 adjacent views (2 per
-// thread; wave w holds views w, w + 4) and S slices (8 for most groups).  Its rays march a
+// Work: a workgroup takes 64 adjacent columns (one per lane) of 4 adjacent views (a wave each;
+// kSplit: of one view, whose lines the four waves share) and S slices.  Its rays march a
 // common axis (the one its middle ray runs closest to) in chunks of 8 lines; per chunk the
 // workgroup stages the pixels its candidates span -- the union of every ray's candidate
 // range over the chunk's lines, each bound linear in k and so extreme at a chunk end --
-// for its S slices in LDS, and each candidate is one LDS read of S slices.  Each pixel
-// staged serves about two columns of each of the 8 views.  A ray more than 60 degrees off
-// that axis (wide fans with few columns) is gathered on its own axis from global memory.
-// (Measured on 64 clinical slices: 8 slices x 2 views per thread 6.97 ms, 4 x 4 11.3 ms,
-// 8 x 4 8.39 ms, 4 x 2 10.3 ms.)
+// for its S slices in LDS, pixels outside the FOV disk as zeros, and each candidate is one LDS
+// read of S slices.  The crossing m*(k) is followed in FP32 from the chunk's first line (exact
+// products, so the fraction keeps an ulp of 1), and the number of candidates is the same for
+// the wave: lanes with fewer, and lines outside a ray's range, read a zero pixel.  A ray more
+// than 60 degrees off the axis (wide fans with few columns) is gathered on its own axis
+// from global memory.
+//
+// Bound: VALU issue (0.6) and the latency of a chunk (two barriers, the staging loads, the
+// candidates' chains).  512 x 512 pixels, 984 views, 888 columns, against two views per thread with a
+// candidate loop per lane: 1 slice 831 -> 573 us, 4 slices 831 -> 645 us, 16 slices 1.74 -> 1.56 ms;
+// 256 x 256, 360 views, 512 columns, 1 slice 164 -> 107 us.  8 slices with their float4 planes apart (a
+// 32-byte pixel made 16-byte reads conflict two-fold) 1029 -> 996 us, with the window sized by
+// the plan instead of 160 pixels (four workgroups per CU instead of three) 846 us.
 struct BpaArgs {
     const float *img;
     float *sino;
@@ -510,36 +519,39 @@ struct BpaArgs {
     const double2 *col_csd; // [nCols] cos, sin gamma_c
     const int2 *fov_row, *fov_col;
     long long img_stride, sino_stride;
-    int nX, nY, nViews, nCols;
+    int nX, nY, nViews, nCols, nSlices, win;
     double R, xmin, ymin, dx, dy;
     float rFOV, tanc, icol;  // rFOV, tan|dCol|, 1/dCol
 };
 
 constexpr int kBpaChunk = 8;                 // lines per staged chunk
-constexpr int kBpaS = 8, kBpaV = 2;          // slices per workgroup (largest groups), views per thread
-constexpr int kBpaWin = 160;                 // staged pixels per line (wider windows read global memory)
+constexpr float kBpaTan = 0.015f;            // tan^4 below an FP32 rounding
+constexpr int kBpaFar = 1 << 24;             // beyond any window
+constexpr int kBpaWin = 160;                 // most staged pixels per line
 
-struct float8_t {
-    float4 a, b;
-};
-template <int S> struct BpaTap;
-template <> struct BpaTap<1> { using T = float; };
-template <> struct BpaTap<2> { using T = float2; };
-template <> struct BpaTap<4> { using T = float4; };
-template <> struct BpaTap<8> { using T = float8_t; };
+// A staged pixel of S slices lies in S / 4 planes of float4 (16 lanes that read adjacent pixels
+// then cover all banks once), or in one plane of S floats.
+template <int S> struct BpaPlane { using T = float4; };
+template <> struct BpaPlane<1> { using T = float; };
+template <> struct BpaPlane<2> { using T = float2; };
 
 template <int S>
-__device__ __forceinline__ float tap_at(const typename BpaTap<S>::T &t, int s)
-{
-    if constexpr (S == 1) return t;
-    else return reinterpret_cast<const float *>(&t)[s];
-}
+struct BpaTap {
+    static constexpr int kP = S > 4 ? S / 4 : 1;
+    typename BpaPlane<S>::T p[kP];
+    __device__ __forceinline__ float operator[](int s) const { return reinterpret_cast<const float *>(p)[s]; }
+};
 
 // Node ray of one (view, column) on a marching axis.
 struct BpaRay {
     double a, b;               // m*(k) = a k + b
     float L0, Ls, pd, pl, hwc;
     int klo, khi;              // lines holding candidates (klo > khi: none)
+};
+
+// The same for the staged chunks: a = a32 + da, and pd, pl times the pixel pitch along the line.
+struct BpaStep {
+    float a32, da, hpd, hpl;
 };
 
 __device__ __forceinline__ void bpa_ray(const BpaArgs &A, double cth, double sth, double Rs, double Rc, bool along_y,
@@ -622,27 +634,54 @@ __device__ __forceinline__ void bpa_line(const BpaRay &r, const BpaHat &hh, floa
     }
 }
 
+// Reductions over the wave's 64 lanes by DPP (rows of 16 lanes by shifts, then across rows): the
+// result is in lane 63, read back as a wave-uniform value.
+template <typename Op>
+__device__ __forceinline__ int wave_reduce(int x, Op &&op)
+{
+    x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x111, 0xf, 0xf, false));  // row_shr:1
+    x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x112, 0xf, 0xf, false));  // row_shr:2
+    x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x114, 0xf, 0xf, false));  // row_shr:4
+    x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x118, 0xf, 0xf, false));  // row_shr:8
+    x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    x = op(x, __builtin_amdgcn_update_dpp(x, x, 0x143, 0xc, 0xf, false));  // row_bcast:31
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
 __device__ __forceinline__ int wave_min(int x)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x = min(x, __shfl_xor(x, o));
-    return x;
+    return wave_reduce(x, [](int a, int b) { return min(a, b); });
 }
 
 __device__ __forceinline__ int wave_max(int x)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x = max(x, __shfl_xor(x, o));
-    return x;
+    return wave_reduce(x, [](int a, int b) { return max(a, b); });
 }
 
 // Slices [slice0 + S*g, +S) of the batch, g = the workgroup's slice group.
-template <bool kWeighted, int S, int kBpaVpt>
+template <bool kWeighted, int S, bool kSplit>
 __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int slice0)
 {
-    constexpr int kBpaViewsWg = 4 * kBpaVpt;  // views per workgroup
-    using TapT = typename BpaTap<S>::T;
-    __shared__ TapT tile[kBpaChunk * kBpaWin];
+    constexpr int kLines = kBpaChunk / 4;  // kSplit: lines of a chunk per wave
+    constexpr int kBpaViewsWg = kSplit ? 1 : 4;  // views per workgroup
+    using TapT = BpaTap<S>;
+    constexpr int kP = TapT::kP;
+    // A.win staged pixels per line, and one more for the chunk, always zero: what a lane reads past
+    // its own candidates
+    extern __shared__ float4 bpa_lds[];
+    auto *tile = reinterpret_cast<typename BpaPlane<S>::T *>(bpa_lds);
+    const int zero_at = kBpaChunk * A.win, plane = zero_at + 1;
+    auto put = [&](int at, const TapT &t) {
+#pragma unroll
+        for (int q = 0; q < kP; ++q) tile[q * plane + at] = t.p[q];
+    };
+    auto get = [&](int at) {
+        TapT t;
+#pragma unroll
+        for (int q = 0; q < kP; ++q) t.p[q] = tile[q * plane + at];
+        return t;
+    };
+    if (threadIdx.x == 0) put(zero_at, TapT{});
     __shared__ int2 fovc[kBpaChunk];  // FOV ranges of the chunk's lines
     __shared__ int red[2][4];
     unsigned cb, vg, g;  // blocked, XCD-aware order over (column block, view group, slice group)
@@ -675,19 +714,15 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
     hh.icol = A.icol;
     hh.c3 = -A.icol * (1.0f / 3.0f);
 
-    BpaRay r[kBpaVpt];
-    bool own[kBpaVpt];  // marched on its own axis (far from the workgroup's)
+    BpaRay r;
     int kmin = INT_MAX, kmax = INT_MIN;
-#pragma unroll
-    for (int j = 0; j < kBpaVpt; ++j) {
-        const int v = (int)vg * kBpaViewsWg + wave + 4 * j;
-        const double2 vb = A.csd[min(v, A.nViews - 1)];
-        const double cth = vb.x * cg.x - vb.y * cg.y, sth = vb.y * cg.x + vb.x * cg.y;
-        own[j] = (along_y ? fabs(sth) : fabs(cth)) < 0.5;
-        bpa_ray(A, cth, sth, Rs, Rc, own[j] ? fabs(sth) >= fabs(cth) : along_y, r[j]);
-        if (!cvalid || v >= A.nViews) r[j].klo = 1, r[j].khi = 0;
-        if (!own[j] && r[j].klo <= r[j].khi) kmin = min(kmin, r[j].klo), kmax = max(kmax, r[j].khi);
-    }
+    const int v = kSplit ? (int)vg : (int)vg * kBpaViewsWg + wave;
+    const double2 vb = A.csd[min(v, A.nViews - 1)];
+    const double cth = vb.x * cg.x - vb.y * cg.y, sth = vb.y * cg.x + vb.x * cg.y;
+    const bool own = (along_y ? fabs(sth) : fabs(cth)) < 0.5;  // marched on its own axis (far from the workgroup's)
+    bpa_ray(A, cth, sth, Rs, Rc, own ? fabs(sth) >= fabs(cth) : along_y, r);
+    if (!cvalid || v >= A.nViews) r.klo = 1, r.khi = 0;
+    if (!own && r.klo <= r.khi) kmin = min(kmin, r.klo), kmax = max(kmax, r.khi);
     kmin = wave_min(kmin);
     kmax = wave_max(kmax);
     if (lane == 0) red[0][wave] = kmin, red[1][wave] = kmax;
@@ -697,18 +732,20 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
     __syncthreads();  // red is rewritten per chunk
 
     const int s_major = along_y ? A.nX : 1, s_minor = along_y ? 1 : A.nX;
-    const int n_minor = along_y ? A.nX : A.nY;
+    const int n_minor = along_y ? A.nX : A.nY, n_major = along_y ? A.nY : A.nX;
     const int2 *fov = along_y ? A.fov_row : A.fov_col;
     const float h = along_y ? (float)A.dx : (float)A.dy;
     // pixel off of the group's S slices: 32-bit byte offsets from the group's first image
     // (the launch keeps S images under 4 GiB)
+    // (a padded group repeats its last slice)
     const unsigned sbytes = (unsigned)A.img_stride * (unsigned)sizeof(float);
+    const int last = A.nSlices - 1 - (int)sl;
     auto load_taps = [&](unsigned off) {
         TapT t;
-        float *tp = reinterpret_cast<float *>(&t);
+        float *tp = reinterpret_cast<float *>(t.p);
         const unsigned b = off * (unsigned)sizeof(float);
 #pragma unroll
-        for (int s = 0; s < S; ++s) tp[s] = load_f_at(img, b + (unsigned)s * sbytes);
+        for (int s = 0; s < S; ++s) tp[s] = load_f_at(img, b + (unsigned)min(s, last) * sbytes);
         return t;
     };
     // the rare global-memory paths (wide windows, rays on their own axis): one slice at a
@@ -718,141 +755,205 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
         const unsigned b = off * (unsigned)sizeof(float);
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            lacc[s] = fmaf(w, load_f_at(img, b + (unsigned)s * sbytes), lacc[s]);
+            lacc[s] = fmaf(w, load_f_at(img, b + (unsigned)min(s, last) * sbytes), lacc[s]);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    double accd[kBpaVpt][S];
+    double accd[S];
 #pragma unroll
-    for (int j = 0; j < kBpaVpt; ++j)
-#pragma unroll
-        for (int s = 0; s < S; ++s) accd[j][s] = 0.0;
+    for (int s = 0; s < S; ++s) accd[s] = 0.0;
 
-    for (int k0 = Klo; k0 <= Khi; k0 += kBpaChunk) {
-        const int k1 = min(k0 + kBpaChunk - 1, Khi);
-        // this thread's candidate range over the chunk (bounds linear in k: ends suffice)
+    BpaStep st;
+    st.a32 = (float)r.a;
+    st.da = (float)(r.a - (double)st.a32);
+    st.hpd = h * r.pd, st.hpl = h * r.pl;
+
+    // chunks at multiples of kBpaChunk lines: a ray's sums do not depend on its workgroup
+    for (int k0 = Klo & ~(kBpaChunk - 1); k0 <= Khi; k0 += kBpaChunk) {
+        const int k1 = min(k0 + kBpaChunk - 1, n_major - 1);
+        // this thread's ray at the chunk's first line, the candidates per line, the same for the
+        // wave (no interval of length 2 hw holds more), and the pixels these reach (bounds linear
+        // in k: the ends suffice)
         int wlo = INT_MAX, whi = INT_MIN;
-#pragma unroll
-        for (int j = 0; j < kBpaVpt; ++j) {
-            const int ka = max(k0, r[j].klo), kb = min(k1, r[j].khi);
-            if (own[j] || ka > kb) continue;
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int ke = e ? kb : ka;
-                const double ms = fma(r[j].a, (double)ke, r[j].b);
-                const float hw = fminf(fmaf(fmaf((float)ke, r[j].Ls, r[j].L0), r[j].hwc, 1.0e-3f), (float)(2 * n_minor + 2));
-                wlo = min(wlo, (int)floor(ms - (double)hw));
-                whi = max(whi, (int)ceil(ms + (double)hw));
-            }
+        const double m0 = fma(r.a, (double)k0, r.b);
+        const double fl = floor(m0);
+        const float fr0 = (float)(m0 - fl);
+        const int mi0 = (int)fl;
+        const int ka = max(k0, r.klo), kb = min(k1, r.khi);
+        const bool on = !own && ka <= kb;
+        const float hwa = fmaf(fmaf((float)ka, r.Ls, r.L0), r.hwc, 1.0e-3f);
+        const float hwb = fmaf(fmaf((float)kb, r.Ls, r.L0), r.hwc, 1.0e-3f);
+        const float hw2 = on ? 2.0f * fmaxf(hwa, hwb) + 1.0e-3f : 0.0f;
+        int nit = 1;
+        while (nit < A.win && __any(hw2 >= (float)nit)) ++nit;
+        if (on && !(hw2 < (float)A.win)) {
+            wlo = -kBpaFar, whi = kBpaFar;
+        } else if (on) {
+            const float xa = fmaf((float)(ka - k0), st.a32, fr0) - hwa;
+            const float xb = fmaf((float)(kb - k0), st.a32, fr0) - hwb;
+            wlo = min(wlo, mi0 + (int)floorf(fminf(xa, xb)));
+            whi = max(whi, mi0 + (int)ceilf(fmaxf(xa, xb)) + nit);
         }
         wlo = wave_min(wlo);
         whi = wave_max(whi);
         if (lane == 0) red[0][wave] = wlo, red[1][wave] = whi;
         __syncthreads();  // also: the previous chunk's reads of the tile are done
-        const int mlo = max(min(min(red[0][0], red[0][1]), min(red[0][2], red[0][3])) - 1, 0);
-        const int mhi_all = min(max(max(red[1][0], red[1][1]), max(red[1][2], red[1][3])) + 1, n_minor - 1);
+        const int mlo = min(min(red[0][0], red[0][1]), min(red[0][2], red[0][3])) - 1;
+        const int mhi = max(max(red[1][0], red[1][1]), max(red[1][2], red[1][3])) + 1;
+        if (mlo > mhi) {  // no candidates in this chunk (uniform)
+            __syncthreads();
+            continue;
+        }
         // a window wider than the tile (wide fans): this chunk reads global memory
-        const bool wide = mhi_all - mlo + 1 > kBpaWin;
-        const int nw = wide ? 0 : max(mhi_all - mlo + 1, 0);  // 0: nothing staged
+        const bool wide = (long long)mhi - mlo + 1 > A.win;
         const int nl = k1 - k0 + 1;
-        if (threadIdx.x < (unsigned)nl) fovc[threadIdx.x] = fov[k0 + threadIdx.x];
-        if (nw > 0) {
+        if (wide) {
+            if (threadIdx.x < (unsigned)nl) fovc[threadIdx.x] = fov[k0 + threadIdx.x];
+        } else {
+            const int nw = mhi - mlo + 1;
+            // pixels outside the FOV disk (and outside the image) are staged as zeros.
             // rows (lines along x): a wave per line, lanes along it; columns: 8 lanes along
             // the chunk's lines, which are consecutive pixels of an image row
             static_assert(kBpaChunk == 8, "column staging puts the chunk's lines on 8 lanes");
+            const TapT zero{};
             if (along_y) {
-                for (int li = wave; li < nl; li += 4)
-                    for (int mm = lane; mm < nw; mm += 64)
-                        tile[li * kBpaWin + mm] = load_taps((unsigned)((k0 + li) * A.nX + mlo + mm));
+                for (int li = wave; li < nl; li += 4) {
+                    const int2 f = fov[k0 + li];
+                    for (int mm = lane; mm < nw; mm += 64) {
+                        const int m = mlo + mm;
+                        put(li * A.win + mm, m >= f.x && m <= f.y ? load_taps((unsigned)((k0 + li) * A.nX + m)) : zero);
+                    }
+                }
             } else {
                 const int li = lane & 7;
-                if (li < nl)
-                    for (int mm = (int)threadIdx.x >> 3; mm < nw; mm += 32)
-                        tile[li * kBpaWin + mm] = load_taps((unsigned)((mlo + mm) * A.nX + k0 + li));
+                if (li < nl) {
+                    const int2 f = fov[k0 + li];
+                    for (int mm = (int)threadIdx.x >> 3; mm < nw; mm += 32) {
+                        const int m = mlo + mm;
+                        put(li * A.win + mm, m >= f.x && m <= f.y ? load_taps((unsigned)(m * A.nX + k0 + li)) : zero);
+                    }
+                }
             }
         }
         __syncthreads();  // tile ready
-        // lines run uniformly over the chunk (their FOV ranges from LDS); a ray skips the
-        // lines outside its own range
         if (!wide) {
-            if (nw == 0) continue;  // no candidates in this chunk (uniform)
-            auto staged = [&](auto edge) {
-                constexpr bool kEdge = decltype(edge)::value;
-#pragma unroll
-                for (int j = 0; j < kBpaVpt; ++j) {
-                    if (own[j]) continue;
-                    float lacc[S];
-#pragma unroll
-                    for (int s = 0; s < S; ++s) lacc[s] = 0.0f;
-                    for (int k = k0; k <= k1; ++k) {
-                        if (k < r[j].klo || k > r[j].khi) continue;
-                        // every candidate lies in the window (it is the union of the
-                        // candidate ranges, one pixel wider); the clamp only keeps reads
-                        // inside the tile
-                        const TapT *row = &tile[(k - k0) * kBpaWin];
-                        bpa_line<kWeighted, kEdge>(r[j], hh, h, k, fovc[k - k0], n_minor, [&](int m, float w) {
-                            const TapT t = row[min(max(m - mlo, 0), nw - 1)];
-#pragma unroll
-                            for (int s = 0; s < S; ++s) lacc[s] = fmaf(w, tap_at<S>(t, s), lacc[s]);
-                        });
-                    }
-#pragma unroll
-                    for (int s = 0; s < S; ++s) accd[j][s] += (double)lacc[s];
-                }
-            };
-            if (edge_wg) staged(std::true_type{});
-            else staged(std::false_type{});
-        } else {
-#pragma unroll
-            for (int j = 0; j < kBpaVpt; ++j) {
-                if (own[j]) continue;
+            // general: the hat of any column and the weight at any column pitch; else max(1 - |rel|, 0)
+            // and the weight's series
+            auto staged = [&](auto general) {
+                constexpr bool kGen = decltype(general)::value;
+                if (own || r.klo > r.khi) return;
                 float lacc[S];
 #pragma unroll
                 for (int s = 0; s < S; ++s) lacc[s] = 0.0f;
-                for (int k = max(k0, r[j].klo); k <= min(k1, r[j].khi); ++k)
-                    bpa_line<kWeighted>(r[j], hh, h, k, fovc[k - k0], n_minor, [&](int m, float w) {
-                        add_taps((unsigned)(k * s_major + m * s_minor), w, lacc);
-                    });
+                int row = mi0 - mlo + (kSplit ? wave * kLines * A.win : 0);
+                const unsigned span = (unsigned)(r.khi - r.klo);
+                const int kka = kSplit ? wave * kLines : 0, kkb = kSplit ? min(kka + kLines, nl) : nl;
+                for (int kk = kka; kk < kkb; ++kk, row += A.win) {
+                    const int k = k0 + kk;
+                    // m* = mi0 + mint + mf: the fraction from exact products, so that it is
+                    // accurate to an ulp of 1 although kk a32 is not a fraction
+                    const float kf = (float)kk;
+                    const float mint = floorf(fmaf(kf, st.a32, fr0));
+                    const float mf = fmaf(kf, st.da, fmaf(kf, st.a32, -mint) + fr0);
+                    const float Lk = fmaf((float)k, r.Ls, r.L0);
+                    const float hw = fmaf(Lk, r.hwc, 1.0e-3f);
+                    const float j0 = ceilf(mf - hw);
+                    const int at0 = row + (int)(mint + j0);
+                    // candidates beyond hw, and all of a line outside the ray's range, read zeros
+                    const float last_dl = (unsigned)(k - r.klo) <= span ? hw : -3.0e38f;
+                    // (a candidate that reads zeros may lie at the source: its weight stays finite)
+                    auto weight = [&](float dl, bool own_cand) {
+                        const float L = fmaf(dl, st.hpl, Lk), d = dl * st.hpd;
+                        const float iL = own_cand ? __builtin_amdgcn_rcpf(L) : 0.0f;
+                        const float z = d * iL, z2 = z * z;
+                        const float rel = z * fmaf(z2, hh.c3, hh.icol);
+                        float w;
+                        if constexpr (kGen) {
+                            w = 1.0f - fabsf(fminf(fmaxf(rel, hh.clo), hh.chi));
+                            w = rel > hh.cut_lo && rel < hh.cut_hi ? w : 0.0f;
+                        } else {
+                            w = fmaxf(1.0f - fabsf(rel), 0.0f);
+                        }
+                        // 1 / (L^2 + d^2) = (1 - z^2) / L^2 up to z^4, |z| <= tan|dCol| < kBpaTan
+                        if constexpr (kWeighted && kGen) w = own_cand ? w * __builtin_amdgcn_rcpf(fmaf(L, L, d * d)) : 0.0f;
+                        if constexpr (kWeighted && !kGen) w *= fmaf(-z2, iL * iL, iL * iL);
+                        return w;
+                    };
+                    const float dl0 = j0 - mf;
+                    int it = 0;
+                    for (; it + 2 <= nit; it += 2) {  // two independent chains
+                        const float da = dl0 + (float)it, db = da + 1.0f;
+                        const bool ia = da <= last_dl, ib = db <= last_dl;
+                        const TapT ta = get(ia ? at0 + it : zero_at), tb = get(ib ? at0 + it + 1 : zero_at);
+                        const float wa = weight(da, ia), wb = weight(db, ib);
 #pragma unroll
-                for (int s = 0; s < S; ++s) accd[j][s] += (double)lacc[s];
-            }
+                        for (int s = 0; s < S; ++s) lacc[s] = fmaf(wb, tb[s], fmaf(wa, ta[s], lacc[s]));
+                    }
+                    if (it < nit) {
+                        const float da = dl0 + (float)it;
+                        const bool ia = da <= last_dl;
+                        const TapT ta = get(ia ? at0 + it : zero_at);
+                        const float wa = weight(da, ia);
+#pragma unroll
+                        for (int s = 0; s < S; ++s) lacc[s] = fmaf(wa, ta[s], lacc[s]);
+                    }
+                }
+#pragma unroll
+                for (int s = 0; s < S; ++s) accd[s] += (double)lacc[s];
+            };
+            if (edge_wg || A.tanc >= kBpaTan) staged(std::true_type{});
+            else staged(std::false_type{});
+        } else {
+            if (own) continue;
+            float lacc[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) lacc[s] = 0.0f;
+            for (int k = max(kSplit ? k0 + wave * kLines : k0, r.klo);
+                 k <= min(kSplit ? min(k1, k0 + wave * kLines + kLines - 1) : k1, r.khi); ++k)
+                bpa_line<kWeighted>(r, hh, h, k, fovc[k - k0], n_minor, [&](int m, float w) {
+                    add_taps((unsigned)(k * s_major + m * s_minor), w, lacc);
+                });
+#pragma unroll
+            for (int s = 0; s < S; ++s) accd[s] += (double)lacc[s];
         }
     }
 
     // rays far from the workgroup's axis: their own axis, taps from global memory, FP32
-    // sums over 8 lines and FP64 across them
-#pragma unroll
-    for (int j = 0; j < kBpaVpt; ++j) {
-        if (!own[j] || r[j].klo > r[j].khi) continue;
-        const int v = (int)vg * kBpaViewsWg + wave + 4 * j;
-        const double2 vb = A.csd[v];
-        const double sth = vb.y * cg.x + vb.x * cg.y, cth = vb.x * cg.x - vb.y * cg.y;
+    // sums over 8 lines and FP64 across them (kSplit: the chunks dealt to the waves)
+    if (own && r.klo <= r.khi) {
         const bool ay = fabs(sth) >= fabs(cth);
         const int sj = ay ? A.nX : 1, si = ay ? 1 : A.nX;
         const int nm = ay ? A.nX : A.nY;
         const int2 *fv = ay ? A.fov_row : A.fov_col;
-        const float hj = ay ? (float)A.dx : (float)A.dy;
-        for (int k0 = r[j].klo; k0 <= r[j].khi; k0 += kBpaChunk) {
+        const float ho = ay ? (float)A.dx : (float)A.dy;
+        for (int k0 = r.klo + (kSplit ? wave * kBpaChunk : 0); k0 <= r.khi; k0 += (kSplit ? 4 : 1) * kBpaChunk) {
             float lacc[S];
 #pragma unroll
             for (int s = 0; s < S; ++s) lacc[s] = 0.0f;
-            for (int k = k0; k <= min(k0 + kBpaChunk - 1, r[j].khi); ++k)
-                bpa_line<kWeighted>(r[j], hh, hj, k, fv[k], nm, [&](int m, float w) {
+            for (int k = k0; k <= min(k0 + kBpaChunk - 1, r.khi); ++k)
+                bpa_line<kWeighted>(r, hh, ho, k, fv[k], nm, [&](int m, float w) {
                     add_taps((unsigned)(k * sj + m * si), w, lacc);
                 });
 #pragma unroll
-            for (int s = 0; s < S; ++s) accd[j][s] += (double)lacc[s];
+            for (int s = 0; s < S; ++s) accd[s] += (double)lacc[s];
         }
     }
 
-    if (!cvalid) return;
+    if constexpr (kSplit) {  // the waves' lines, added in wave order
+        double *part = reinterpret_cast<double *>(bpa_lds);
 #pragma unroll
-    for (int j = 0; j < kBpaVpt; ++j) {
-        const int v = (int)vg * kBpaViewsWg + wave + 4 * j;
-        if (v >= A.nViews) continue;
-#pragma unroll
-        for (int s = 0; s < S; ++s) A.sino[(sl + s) * A.sino_stride + (size_t)v * A.nCols + c] = (float)accd[j][s];
+        for (int s = 0; s < S; ++s) {
+            __syncthreads();
+            part[threadIdx.x] = accd[s];
+            __syncthreads();
+            accd[s] = (part[lane] + part[64 + lane]) + (part[128 + lane] + part[192 + lane]);
+        }
+        if (wave != 0) return;
     }
+    if (!cvalid || v >= A.nViews) return;
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        if (s <= last) A.sino[(sl + s) * A.sino_stride + (size_t)v * A.nCols + c] = (float)accd[s];
 }
 
 BpArgs make_args(const fbct_plan &p, const DeviceTables &t, const float *sino, float *img)
@@ -1006,24 +1107,40 @@ fbct_status launch_bp_adjoint(const fbct_plan &p, const DeviceTables &t, const f
     A.rFOV = p.g.rFOV;
     A.tanc = p.d.bpa_tan;
     A.icol = p.d.bp_xi_scale;
-    // groups of kBpaS slices, the remainder in groups of 4, 2 and 1; every group size has
-    // the same workgroups (kBpaV views per thread), so a slice's result does not depend
-    // on the group it falls in
-    static_assert(kBpaS == 8, "group sizes 8, 4, 2, 1");
+    A.nSlices = n;
     // a group's images are addressed by 32-bit byte offsets: its S images stay below 4 GiB
     const unsigned long long img_bytes = (unsigned long long)p.g.nX * p.g.nY * sizeof(float);
     if (img_bytes >= (1ULL << 32))
         return fail(FBCT_ERR_UNSUPPORTED, "fbct_bp_adjoint: an image of %llu bytes exceeds 4 GiB", img_bytes);
-    const dim3 g2((p.g.nCols + 63) / 64, (p.g.nViews + 4 * kBpaV - 1) / (4 * kBpaV), 1);
-    int done = 0;
-    for (int S : {8, 4, 2, 1}) {
-        if ((unsigned long long)S * img_bytes >= (1ULL << 32)) continue;
-        const int groups = (n - done) / S;
-        if (groups == 0) continue;
-        const dim3 grid(g2.x, g2.y, groups);
+    // Four views a workgroup, a wave each, or (split) one view whose lines the waves share.  Split
+    // where few workgroups leave the chip idle -- 96 x 96 pixels, 130 views, 140 columns, 99
+    // workgroups: 82 -> 26 us for one slice; 128 x 128, 200 workgroups: 63 -> 43 us; but 200 x 200,
+    // 375 workgroups: 99 -> 76 us for one slice and 122 -> 127 us for eight, 256 x 256, 720
+    // workgroups: 107 -> 132 us -- and where the rays of four views spread so far that some march
+    // their own axis from global memory (96 x 96, 16 slices: 199 -> 42 us).  The rule looks at the
+    // plan only, so that a slice's result does not depend on the slices with it.
+    const double dcol = fabs((double)p.g.dCol), pitch = std::min(p.g.dx, p.g.dy);
+    const double dview = p.g.nViews > 1 ? fabs((double)p.angles[p.g.nViews - 1] - p.angles[0]) / (p.g.nViews - 1) : 0.0;
+    const int cblocks = (p.g.nCols + 63) / 64;
+    const bool split = (long long)cblocks * ((p.g.nViews + 3) / 4) < 300 || 64.0 * dcol + 4.0 * dview > 0.52;
+    // Staged pixels per line: what 64 columns reach at the far end of the FOV disk on a ray 45
+    // degrees off the axis, the views' spread, a chunk's slant and margins; at most the image and
+    // kBpaWin (wider windows read global memory)
+    const double reach = 64.0 * dcol * ((double)p.g.R + p.g.rFOV) / (0.7 * pitch) + 16.0 +
+                         (split ? 0.0 : 4.0 * dview * p.g.rFOV / (0.7 * pitch));
+    A.win = (int)std::min(std::min(reach, 24.0 + std::max(p.g.nX, p.g.nY)), (double)kBpaWin);
+    for (int done = 0; done < n;) {
+        const int left = n - done;
+        int S = left >= 5 ? 8 : left >= 3 ? 4 : left;  // padded with the last slice
+        while ((unsigned long long)S * img_bytes >= (1ULL << 32)) S /= 2;
+        const int groups = std::max(left / S, 1);
+        const dim3 grid(cblocks, split ? p.g.nViews : (p.g.nViews + 3) / 4, groups);
+        const size_t lds = std::max(sizeof(float) * S * (kBpaChunk * (size_t)A.win + 1), sizeof(double) * 256);
 #define FBCT_BPA(SS)                                                                                            \
-    if (weighted) hipLaunchKernelGGL((bp_adjoint_staged_kernel<true, SS, kBpaV>), grid, dim3(256), 0, stream, A, done); \
-    else hipLaunchKernelGGL((bp_adjoint_staged_kernel<false, SS, kBpaV>), grid, dim3(256), 0, stream, A, done)
+    if (split && weighted) hipLaunchKernelGGL((bp_adjoint_staged_kernel<true, SS, true>), grid, dim3(256), lds, stream, A, done); \
+    else if (split) hipLaunchKernelGGL((bp_adjoint_staged_kernel<false, SS, true>), grid, dim3(256), lds, stream, A, done); \
+    else if (weighted) hipLaunchKernelGGL((bp_adjoint_staged_kernel<true, SS, false>), grid, dim3(256), lds, stream, A, done); \
+    else hipLaunchKernelGGL((bp_adjoint_staged_kernel<false, SS, false>), grid, dim3(256), lds, stream, A, done)
         switch (S) {
         case 8: FBCT_BPA(8); break;
         case 4: FBCT_BPA(4); break;
@@ -1032,7 +1149,6 @@ fbct_status launch_bp_adjoint(const fbct_plan &p, const DeviceTables &t, const f
         }
 #undef FBCT_BPA
         done += groups * S;
-        if (done == n) break;
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "bp_adjoint_staged_kernel launch: %s", hipGetErrorString(e));
