@@ -20,6 +20,12 @@
 //     launch with that smaller tile, the others in a launch with the full one;
 //   * FP32 partial sums per slab, FP64 across slabs; one cross-lane reduction per ray at
 //     the end and one coalesced store (optionally minus a target: the FP residual).
+// What bounds it: VALU issue and LDS reads, about equally (four taps and some 25 VALU
+// instructions per cell and wave with one slice, 40 with four); memory is hardly touched.  The
+// cell's weights are kept as means (13 instructions to n's ~17 for running sums): 64 slices of
+// 512 x 512 over 984 views x 888 columns 9.97 -> 9.80 ms, one slice 340 -> 310 us, 256 x 256
+// over 360 x 512 66 -> 60 us.
+//
 // A sample belongs to the slab containing its major coordinate, decided from the same
 // FP32 position the interpolation uses, so every sample is counted exactly once.
 
@@ -146,8 +152,11 @@ __device__ __forceinline__ void fp_bundle(const FpArgs &A, int b, int v, int s0)
     const float ia = da != 0.0f ? 1.0f / da : 1.0e30f;
     const float im = dm != 0.0f ? 1.0f / dm : 1.0e30f;
     const float nia = -ia, nim = -im;
-    const float ca = da >= 0.0f ? ia + 1.0f : 1.0f;
-    const float cm = dm >= 0.0f ? im + 1.0f : 1.0f;
+    // (o / step is raised by 2^-22 of itself, more than what rounding takes from the sum, so that
+    // a cell always counts its first sample, also one whose fraction rounds to 1: the walk ends)
+    const float ca = da >= 0.0f ? fmaf(ia, 1.0f + 0x1p-22f, 1.0f) : 1.0f;
+    const float cm = dm >= 0.0f ? fmaf(im, 1.0f + 0x1p-22f, 1.0f) : 1.0f;
+    const float dd = da * dm * (1.0f / 12.0f);
     const TI *img[S];
 #pragma unroll
     for (int s = 0; s < S; ++s)
@@ -264,29 +273,38 @@ __device__ __forceinline__ void fp_bundle(const FpArgs &A, int b, int v, int s0)
             const float fa = floorf(a), fm = floorf(m);
             const float ta = a - fa, tm = m - fm;
             // samples before the next boundary along each axis: floor(distance / step) + 1
-            // with distance (fa + o) - a = o - ta, one FMA each; the three counts share one
-            // min.  A count that rounding puts one past a boundary only moves a sample lying
-            // on it (within rounding) into this cell, where its bilinear weights are the same.
-            const float ja1 = floorf(fmaf(ta, nia, ca));
-            const float jm1 = floorf(fmaf(tm, nim, cm));
-            const float n = __builtin_amdgcn_fmed3f(fminf(ja1, jm1), -1.0e30f, kend - kf);
-            const float t1 = 0.5f * fmaf(n, n, -n);                        // sum of j
-            const float t2 = t1 * fmaf(n, 2.0f / 3.0f, -1.0f / 3.0f);      // sum of j^2
-            const float sa = fmaf(da, t1, n * ta);                          // sum of a-fractions
-            const float sm = fmaf(dm, t1, n * tm);                          // sum of m-fractions
-            // sum of products: sum_j (ta + j da)(tm + j dm) = ta sm + da (tm t1 + dm t2)
-            const float sam = fmaf(ta, sm, da * fmaf(tm, t1, dm * t2));
-            const float w11 = sam, w01 = sa - sam, w10 = sm - sam, w00 = (n - sa) - w10;
+            // with distance (fa + o) - a = o - ta, one FMA each; the least of the two counts and
+            // of the samples left, one floor for all three.  A count that rounding puts one past a
+            // boundary only moves a sample lying on it (within rounding) into this cell, where its
+            // bilinear weights are the same.
+            const float n = floorf(fminf(fminf(fmaf(ta, nia, ca), fmaf(tm, nim, cm)), kend - kf));
+            // the n fractions are linear in the sample index: their means are those of the middle
+            // (half-integer) index, and the mean of their products is the product of the means
+            // plus da dm times the variance (n^2 - 1) / 12 of the indices
+            const float jc = fmaf(n, 0.5f, -0.5f);
+            const float ma = fmaf(jc, da, ta), mm = fmaf(jc, dm, tm);
+            const float mam = fmaf(dd, fmaf(n, n, -1.0f), ma * mm);
             const unsigned o = (unsigned)fmaf(fm, kRowB, fmaf(fa, kColB, obase));
             const TapT t00 = *reinterpret_cast<LdsTap *>((size_t)o);
             const TapT t01 = *reinterpret_cast<LdsTap *>((size_t)(o + (unsigned)kColB));
             const TapT t10 = *reinterpret_cast<LdsTap *>((size_t)(o + (unsigned)kRowB));
             const TapT t11 = *reinterpret_cast<LdsTap *>((size_t)(o + (unsigned)(kRowB + kColB)));
+            if constexpr (S <= 2) {  // mean weights, times n per slice
+                const float w01 = ma - mam, w10 = mm - mam, w00 = (1.0f - ma) - w10;
 #pragma unroll
-            for (int s = 0; s < S; ++s)
-                acc[s] = fmaf(w00, lane_of<S>(t00, s),
-                              fmaf(w01, lane_of<S>(t01, s),
-                                   fmaf(w10, lane_of<S>(t10, s), fmaf(w11, lane_of<S>(t11, s), acc[s]))));
+                for (int s = 0; s < S; ++s)
+                    acc[s] = fmaf(n, fmaf(w00, lane_of<S>(t00, s),
+                                          fmaf(w01, lane_of<S>(t01, s),
+                                               fmaf(w10, lane_of<S>(t10, s), mam * lane_of<S>(t11, s)))), acc[s]);
+            } else {
+                const float sa = n * ma, sm = n * mm;
+                const float w11 = n * mam, w01 = sa - w11, w10 = sm - w11, w00 = (n - sa) - w10;
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+                    acc[s] = fmaf(w00, lane_of<S>(t00, s),
+                                  fmaf(w01, lane_of<S>(t01, s),
+                                       fmaf(w10, lane_of<S>(t10, s), fmaf(w11, lane_of<S>(t11, s), acc[s]))));
+            }
             kf += n;
         }
 #pragma unroll
@@ -305,14 +323,14 @@ __device__ __forceinline__ void fp_bundle(const FpArgs &A, int b, int v, int s0)
     }
 }
 
-// Items order[item0 + t] (t < gridDim.x) of slice group blockIdx.y; item = v * nb + b.
+// Items order[item0 + t] (t < gridDim.x) of slice group blockIdx.y (from slice0); item = v * nb + b.
 template <int S, int G, typename TI, typename TO>
-__global__ __launch_bounds__(kFpThreads) void fp_kernel(FpArgs A, const int32_t *__restrict__ order, int item0)
+__global__ __launch_bounds__(kFpThreads) void fp_kernel(FpArgs A, const int32_t *__restrict__ order, int item0, int slice0)
 {
     unsigned t, g;  // XCD-aware (item, slice group)
     xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x, gridDim.y, t, g);
     const int vb = order[item0 + (int)t];
-    fp_bundle<S, G, TI, TO>(A, vb % A.nb, vb / A.nb, g * S);
+    fp_bundle<S, G, TI, TO>(A, vb % A.nb, vb / A.nb, slice0 + (int)g * S);
 }
 
 // Uneven batch: slice s has its own geometry (desc[s]); work item = (slice, view,
@@ -366,20 +384,67 @@ __global__ __launch_bounds__(kFpThreads) void fp_batch_kernel(const FpSliceDesc 
 }  // namespace
 
 template <int S, int G, typename TI, typename TO>
-static void launch_fp_s(dim3 grid, size_t lds, hipStream_t stream, const FpArgs &A, const int32_t *order, int item0)
+static void launch_fp_s(dim3 grid, size_t lds, hipStream_t stream, const FpArgs &A, const int32_t *order, int item0, int slice0)
 {
-    hipLaunchKernelGGL((fp_kernel<S, G, TI, TO>), grid, dim3(kFpThreads), lds, stream, A, order, item0);
+    hipLaunchKernelGGL((fp_kernel<S, G, TI, TO>), grid, dim3(kFpThreads), lds, stream, A, order, item0, slice0);
 }
 
 template <int S, int G>
 static fbct_status launch_fp_t(fbct_dtype ti, fbct_dtype to, dim3 grid, size_t lds, hipStream_t stream,
-                               const FpArgs &A, const int32_t *order, int item0)
+                               const FpArgs &A, const int32_t *order, int item0, int slice0)
 {
-    if (ti == FBCT_F32 && to == FBCT_F32) launch_fp_s<S, G, float, float>(grid, lds, stream, A, order, item0);
-    else if (ti == FBCT_BF16 && to == FBCT_F32) launch_fp_s<S, G, bf16_t, float>(grid, lds, stream, A, order, item0);
-    else if (ti == FBCT_F32 && to == FBCT_BF16) launch_fp_s<S, G, float, bf16_t>(grid, lds, stream, A, order, item0);
-    else if (ti == FBCT_BF16 && to == FBCT_BF16) launch_fp_s<S, G, bf16_t, bf16_t>(grid, lds, stream, A, order, item0);
+    if (ti == FBCT_F32 && to == FBCT_F32) launch_fp_s<S, G, float, float>(grid, lds, stream, A, order, item0, slice0);
+    else if (ti == FBCT_BF16 && to == FBCT_F32) launch_fp_s<S, G, bf16_t, float>(grid, lds, stream, A, order, item0, slice0);
+    else if (ti == FBCT_F32 && to == FBCT_BF16) launch_fp_s<S, G, float, bf16_t>(grid, lds, stream, A, order, item0, slice0);
+    else if (ti == FBCT_BF16 && to == FBCT_BF16) launch_fp_s<S, G, bf16_t, bf16_t>(grid, lds, stream, A, order, item0, slice0);
     else return fail(FBCT_ERR_INVALID_ARGUMENT, "fbct_fp: unknown storage type");
+    return FBCT_OK;
+}
+
+// Slices [slice0, slice0 + S groups) of a call, S at a time, in bundles of configuration cfg.
+static fbct_status launch_fp_groups(const fbct_plan &p, const DeviceTables &t, FpArgs A, int S, int cfg, int slice0,
+                                    int groups, fbct_dtype ti, fbct_dtype to, hipStream_t stream)
+{
+    const FpBundleCfg &bc = p.d.fpb[cfg];
+    A.major = t.fp_major[cfg];
+    A.slabs = t.fp_slabs[cfg];
+    A.rows = t.fp_rows[cfg];
+    A.nb = bc.nb;
+    A.nslab = bc.nslab;
+    const size_t bytes = (size_t)fp_pitch(cfg) * bc.cap * sizeof(float) * S;
+    if (bytes > 160 * 1024) return fail(FBCT_ERR_UNSUPPORTED, "fbct_fp: slab tile of %zu bytes exceeds LDS", bytes);
+    // The LDS tile sets how many workgroups a CU holds (up to kFpWgsPerCu, where the
+    // registers cap it).  Items whose largest tile fits the rows of that many workgroups
+    // get a launch of their own with that smaller tile; the others (ordered first) a
+    // launch with the plan's full tile.
+    const size_t row_bytes = (size_t)fp_pitch(cfg) * sizeof(float) * S;
+    const int small_cap = (int)std::min<size_t>((size_t)bc.cap, (160 * 1024 / kFpWgsPerCu) / row_bytes);
+    const std::vector<int16_t> &orows = p.fp_order_rows[cfg];
+    const int nitems = (int)orows.size();
+    // first item with at most small_cap rows (counts are non-increasing)
+    const int split = (int)(std::upper_bound(orows.begin(), orows.end(), (int16_t)small_cap,
+                                             [](int16_t cap_v, int16_t r) { return r <= cap_v; }) -
+                            orows.begin());
+    for (int part = 0; part < 2; ++part) {
+        const int item0 = part == 0 ? 0 : split;
+        const int count = part == 0 ? split : nitems - split;
+        if (count == 0) continue;
+        A.cap = part == 0 ? bc.cap : small_cap;
+        const size_t lds = (size_t)A.cap * row_bytes;
+        const dim3 grid((unsigned)count, (unsigned)groups);
+        fbct_status st;
+        if (cfg == 0) {
+            if (S == 2) st = launch_fp_t<2, 4>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0, slice0);
+            else st = launch_fp_t<1, 4>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0, slice0);
+        } else {
+            if (S == 4) st = launch_fp_t<4, 8>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0, slice0);
+            else if (S == 2) st = launch_fp_t<2, 8>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0, slice0);
+            else st = launch_fp_t<1, 8>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0, slice0);
+        }
+        if (st != FBCT_OK) return st;
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "fp_kernel launch: %s", hipGetErrorString(e));
+    }
     return FBCT_OK;
 }
 
@@ -400,64 +465,33 @@ fbct_status launch_fp(const fbct_plan &p, const DeviceTables &t, const void *img
     A.nCols = p.g.nCols;
     A.scale = p.d.fp_scale;
     A.nSlices = n;
-    hipError_t e;
 
-    // Slices per workgroup S and bundle configuration: share each sample's position and
-    // weights across 4 slices with 32-ray bundles (smaller tile), else 2 or 1 slices with
-    // 64-ray bundles, while the grid keeps >= 2048 workgroups and the tile <= 80 KB.
+    // Slices per workgroup S and bundle configuration.  Four slices share a cell's position and
+    // weights with 32-ray bundles (smaller tile) while a launch keeps >= 2048 workgroups; three
+    // count as four (512 x 512: 629 us, 840 as two pairs).  Else pairs while >= 1024 workgroups
+    // remain (104 x 104, 7 slices: 22 us, 27 singly): in 64-ray bundles while eight workgroups'
+    // tiles fit a CU (256 x 256 at 512 columns: 65 us, 76 with 32 rays), in 32-ray bundles beyond
+    // (373 x 373 at 611 columns: 127 us, 155 with 64).  A single slice always takes 64-ray bundles
+    // unless their tile exceeds 80 KB, as the uneven batch does by default.
     const size_t kMaxTile = 80 * 1024;
     auto tile_bytes = [&](int cfg, int S) { return (size_t)fp_pitch(cfg) * p.d.fpb[cfg].cap * sizeof(float) * S; };
-    auto grid_wgs = [&](int cfg, int S) { return (long long)p.d.fpb[cfg].nb * p.g.nViews * ((n + S - 1) / S); };
-    int S = 1, cfg = 0;
-    if (n >= 4 && tile_bytes(1, 4) <= kMaxTile && grid_wgs(1, 4) >= 2048) {
-        S = 4;
-        cfg = 1;
-    } else if (n >= 2 && grid_wgs(0, 2) >= 2048) {
-        S = 2;
-        cfg = tile_bytes(0, 2) <= kMaxTile ? 0 : 1;
-    } else if (tile_bytes(0, 1) > kMaxTile) {
-        cfg = 1;
-    }
-    const FpBundleCfg &bc = p.d.fpb[cfg];
-    A.major = t.fp_major[cfg];
-    A.slabs = t.fp_slabs[cfg];
-    A.rows = t.fp_rows[cfg];
-    A.nb = bc.nb;
-    A.nslab = bc.nslab;
-    if (tile_bytes(cfg, S) > 160 * 1024)
-        return fail(FBCT_ERR_UNSUPPORTED, "fbct_fp: slab tile of %zu bytes exceeds LDS", tile_bytes(cfg, S));
-    // The LDS tile sets how many workgroups a CU holds (up to kFpWgsPerCu, where the
-    // registers cap it).  Items whose largest tile fits the rows of that many workgroups
-    // get a launch of their own with that smaller tile; the others (ordered first) a
-    // launch with the plan's full tile.
-    const size_t row_bytes = (size_t)fp_pitch(cfg) * sizeof(float) * S;
-    const int small_cap = (int)std::min<size_t>((size_t)bc.cap, (160 * 1024 / kFpWgsPerCu) / row_bytes);
-    const std::vector<int16_t> &orows = p.fp_order_rows[cfg];
-    const int nitems = (int)orows.size();
-    // first item with at most small_cap rows (counts are non-increasing)
-    const int split = (int)(std::upper_bound(orows.begin(), orows.end(), (int16_t)small_cap,
-                                             [](int16_t cap_v, int16_t r) { return r <= cap_v; }) -
-                            orows.begin());
-    const unsigned groups = (unsigned)((n + S - 1) / S);
-    for (int part = 0; part < 2; ++part) {
-        const int item0 = part == 0 ? 0 : split;
-        const int count = part == 0 ? split : nitems - split;
-        if (count == 0) continue;
-        A.cap = part == 0 ? bc.cap : small_cap;
-        const size_t lds = (size_t)A.cap * row_bytes;
-        const dim3 grid((unsigned)count, groups);
-        fbct_status st;
-        if (cfg == 0) {
-            if (S == 2) st = launch_fp_t<2, 4>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0);
-            else st = launch_fp_t<1, 4>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0);
-        } else {
-            if (S == 4) st = launch_fp_t<4, 8>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0);
-            else if (S == 2) st = launch_fp_t<2, 8>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0);
-            else st = launch_fp_t<1, 8>(ti, to, grid, lds, stream, A, t.fp_order[cfg], item0);
+    auto group_wgs = [&](int cfg) { return (long long)p.d.fpb[cfg].nb * p.g.nViews; };
+    int done = 0;
+    while (done < n) {
+        const int left = n - done;
+        int S = 1, cfg = tile_bytes(0, 1) > kMaxTile ? 1 : 0, groups = left;
+        if (left >= 3 && tile_bytes(1, 4) <= kMaxTile && group_wgs(1) * ((left + 3) / 4) >= 2048) {
+            S = 4, cfg = 1;
+            // one or two slices over: a launch of their own where a group alone fills the chip (373 x
+            // 373, 5 slices: 369 us padded to 8, 290 as 4 and 1), else padded
+            groups = left % 4 != 0 && (left % 4 == 3 || left < 4 || group_wgs(1) < 2048) ? left / 4 + 1 : left / 4;
+        } else if (left >= 2 && tile_bytes(1, 2) <= kMaxTile && group_wgs(1) * ((left + 1) / 2) >= 1024) {
+            S = 2, cfg = tile_bytes(0, 2) <= 20 * 1024 ? 0 : 1;
+            groups = (left + 1) / 2;
         }
+        const fbct_status st = launch_fp_groups(p, t, A, S, cfg, done, groups, ti, to, stream);
         if (st != FBCT_OK) return st;
-        e = hipGetLastError();
-        if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "fp_kernel launch: %s", hipGetErrorString(e));
+        done += S * groups;
     }
     return FBCT_OK;
 }
