@@ -121,9 +121,16 @@ void build(fbct_cone_plan &p)
             }
     }
     d.xi_scale = (float)(flat ? D / dc : 1.0 / dc);
-    d.xi_offset = (float)((double)g.dShift - (double)g.colLeft / dc);
+    {
+        const double c = (double)g.dShift - (double)g.colLeft / dc - 0.5, r = -(double)g.rowBottom / dr - 0.5;
+        const double cm = std::min(std::max(std::nearbyint(c), -1.0e6), 1.0e6);
+        const double rm = std::min(std::max(std::nearbyint(r), -1.0e6), 1.0e6);
+        d.ct_col = (int)cm;
+        d.ct_offset = (float)(c - cm);
+        d.rt_row = (int)rm;
+        d.rt_offset = (float)(r - rm);
+    }
     d.zr_scale = (float)(D / dr);
-    d.zr_offset = (float)(-(double)g.rowBottom / dr);
     d.r2 = g.rFOV * g.rFOV;
     // 0 < xi < nCols  <=>  t/U strictly between the detector edge values (either order)
     const double e0 = (double)g.colLeft - (double)g.dShift * dc;

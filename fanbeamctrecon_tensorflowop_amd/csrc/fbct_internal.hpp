@@ -239,8 +239,12 @@ namespace fbct {
 
 // Scalars of a cone plan's backprojection, derived once in FP64 on the host.
 struct ConeDerived {
-    float xi_scale, xi_offset;  // flat: xi = (t/U) xi_scale + xi_offset; curved: atan(t/U) xi_scale + xi_offset
-    float zr_scale, zr_offset;  // zeta = z (1/U) zr_scale + zr_offset
+    // column coordinate relative to the central column ct_col (so that FP32 keeps its fraction):
+    // flat: ct = (t/U) xi_scale + ct_offset, curved: atan(t/U) xi_scale + ct_offset; texel centres
+    // are whole numbers.  Rows likewise: rt = z (1/U) zr_scale + rt_offset, relative to rt_row.
+    float xi_scale, ct_offset;
+    float zr_scale, rt_offset;
+    int ct_col, rt_row;
     float r2;                   // rFOV^2 (float)
     int edge_exact;             // 1: the in-range decision near the edges is retaken in FP64 on t/U
     double tan_min, tan_max;    //    0 < xi < nCols  <=>  tan_min < t/U < tan_max
