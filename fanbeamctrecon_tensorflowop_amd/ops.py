@@ -26,8 +26,6 @@ the forward pass is kept for the backward pass.
 """
 from __future__ import annotations
 
-import math
-
 import torch
 
 from . import torch_ops  # noqa: F401  (registers torch.ops.fbct.*)
@@ -116,10 +114,11 @@ def fdk(proj: torch.Tensor, plan: FanBeamPlan) -> torch.Tensor:
 
 def _attr_list(a):
     """An op attribute (tensor, array or sequence of floats) as a list of Python floats."""
-    if isinstance(a, torch.Tensor):
-        a = a.detach().cpu().reshape(-1).tolist()
-    elif hasattr(a, "tolist"):
-        a = a.reshape(-1).tolist()
+    if hasattr(a, "tolist"):
+        floats = str(getattr(a, "dtype", "")).endswith(("float16", "float32", "float64"))  # Python floats already
+        a = (a.detach().cpu() if isinstance(a, torch.Tensor) else a).reshape(-1).tolist()
+        if floats:
+            return a
     return [float(v) for v in a]
 
 
@@ -127,8 +126,22 @@ def _shape_list(s):
     return [int(v) for v in s]
 
 
+def _needs_autograd(x):
+    """Whether a call has to go through the ops' autograd kernels: a gradient is asked for, or
+    something (a transform, a compiler, a tensor subclass) may look at the call there."""
+    return (torch.compiler.is_compiling() or type(x) is not torch.Tensor
+            or (x.requires_grad and torch.is_grad_enabled())
+            or torch._C._functorch.peek_interpreter_stack() is not None)
+
+
 def _call(op, x, angle, parameter, vol_shape, proj_shape):
-    return op(x, _attr_list(angle), _attr_list(parameter), _shape_list(vol_shape), _shape_list(proj_shape))
+    # The autograd kernels convert the attributes to Python lists and back once more (360 views: 36
+    # of 57 us a call); without a gradient to record the op is dispatched below them.
+    args = (_attr_list(angle), _attr_list(parameter), _shape_list(vol_shape), _shape_list(proj_shape))
+    if _needs_autograd(x):
+        return op(x, *args)
+    with torch._C._AutoDispatchBelowAutograd():
+        return op(x, *args)
 
 
 def fp_fan_curve(volume, angle, parameter, vol_shape, proj_shape):

@@ -21,9 +21,11 @@ matched adjoint op; the operators are linear, so backward keeps nothing from for
 """
 from __future__ import annotations
 
+import array
 import math
 from typing import List
 
+import numpy as np
 import torch
 
 from .plan import get_plan
@@ -31,8 +33,21 @@ from .plan import get_plan
 __all__ = ["OPS"]
 
 
+_impl = torch.library.Library("fbct", "IMPL")
+
+
+def _register(fn):
+    """The custom op ``fbct::<name of fn>``.  On device tensors the dispatcher calls fn itself: the
+    wrapper that custom_op puts around it compares inputs and outputs for aliasing on every call (10
+    us), and the outputs here are new tensors."""
+    op = torch.library.custom_op("fbct::" + fn.__name__, mutates_args=())(fn)
+    _impl.impl(fn.__name__, fn, "CUDA")
+    return op
+
+
 def _plan(angle, parameter):
-    return get_plan(list(parameter), list(angle))
+    # float64 arrays from the lists' own numbers (numpy's conversion of a list takes half as long again)
+    return get_plan(np.frombuffer(array.array("d", parameter)), np.frombuffer(array.array("d", angle)))
 
 
 def _slices(x, plan, per_slice, what):
@@ -72,14 +87,14 @@ def _fdk_in(x, plan, what):
 
 # ------------------------------------------------------------------ forward ops
 
-@torch.library.custom_op("fbct::fp_fan_curve", mutates_args=())
+@_register
 def fp_fan_curve(volume: torch.Tensor, angle: List[float], parameter: List[float], vol_shape: List[int],
                  proj_shape: List[int]) -> torch.Tensor:
     plan = _plan(angle, parameter)
     return _shaped(plan.fp(_img_in(volume, plan, "fp_fan_curve")), proj_shape, "fp_fan_curve")
 
 
-@torch.library.custom_op("fbct::fp_fan_curve_adjoint", mutates_args=())
+@_register
 def fp_fan_curve_adjoint(projection: torch.Tensor, angle: List[float], parameter: List[float],
                          vol_shape: List[int], proj_shape: List[int]) -> torch.Tensor:
     plan = _plan(angle, parameter)
@@ -87,14 +102,14 @@ def fp_fan_curve_adjoint(projection: torch.Tensor, angle: List[float], parameter
                    "fp_fan_curve_adjoint")
 
 
-@torch.library.custom_op("fbct::bp_fan_curve", mutates_args=())
+@_register
 def bp_fan_curve(projection: torch.Tensor, angle: List[float], parameter: List[float], vol_shape: List[int],
                  proj_shape: List[int]) -> torch.Tensor:
     plan = _plan(angle, parameter)
     return _shaped(plan.bp(_sino_in(projection, plan, "bp_fan_curve")), vol_shape, "bp_fan_curve")
 
 
-@torch.library.custom_op("fbct::bp_fan_curve_adjoint", mutates_args=())
+@_register
 def bp_fan_curve_adjoint(volume: torch.Tensor, angle: List[float], parameter: List[float],
                          vol_shape: List[int], proj_shape: List[int]) -> torch.Tensor:
     plan = _plan(angle, parameter)
@@ -102,14 +117,14 @@ def bp_fan_curve_adjoint(volume: torch.Tensor, angle: List[float], parameter: Li
                    "bp_fan_curve_adjoint")
 
 
-@torch.library.custom_op("fbct::fbp_fan_curve", mutates_args=())
+@_register
 def fbp_fan_curve(projection: torch.Tensor, angle: List[float], parameter: List[float], vol_shape: List[int],
                   proj_shape: List[int]) -> torch.Tensor:
     plan = _plan(angle, parameter)
     return _shaped(plan.fbp(_sino_in(projection, plan, "fbp_fan_curve")), vol_shape, "fbp_fan_curve")
 
 
-@torch.library.custom_op("fbct::fbp_fan_curve_adjoint", mutates_args=())
+@_register
 def fbp_fan_curve_adjoint(volume: torch.Tensor, angle: List[float], parameter: List[float],
                           vol_shape: List[int], proj_shape: List[int]) -> torch.Tensor:
     plan = _plan(angle, parameter)
@@ -123,7 +138,7 @@ def fbp_fan_curve_adjoint(volume: torch.Tensor, angle: List[float], parameter: L
                    "fbp_fan_curve_adjoint")
 
 
-@torch.library.custom_op("fbct::back_projection", mutates_args=())
+@_register
 def back_projection(projection: torch.Tensor, angle: List[float], parameter: List[float], vol_shape: List[int],
                     proj_shape: List[int]) -> torch.Tensor:
     """The FDK op: nZ = nRows = 1 (FDK/FBP.cc:85,98) makes it the FBP of every slice; the
