@@ -930,7 +930,7 @@ __global__ __launch_bounds__(kAdjThreads, S == 16 ? 2 : S == 8 ? 4 : 6) void fp_
 
 // Uneven batch: slice s has its own geometry (desc[s]); work item = (slice, tile), items
 // of slice s are [prefix[s], prefix[s+1]).  A slice whose samples stay in the cells
-// [-1, n-1] takes 15 x 15-pixel cell tiles, as a single-slice call does; any other slice
+// [-1, n-1] takes 7 x 7-pixel cell tiles, as a single-slice call does; any other slice
 // TX x (256/TX) gather tiles.  A fixed grid strides over all items, the XCDs taking
 // them in chunks of 64, and a slice's tiles run in blocked order, so the tiles resident
 // on one XCD cover a compact part of one image and share their rays through its L2.
@@ -1044,13 +1044,32 @@ fbct_status launch_fp_adjoint(const fbct_plan &p, const DeviceTables &t, const v
     const long long gx = (p.g.nX + kAdjTx - 1) / kAdjTx, gy = (p.g.nY + kAdjTy - 1) / kAdjTy;
     fbct_status st = FBCT_OK;
     if (adj_cells_fit(A.far_x, A.far_y)) {
-        // groups of 16 slices, the rest in groups of the next size up, padded with the last slice
+        // Groups of 16 slices, the rest in groups of the next size up, padded with the last slice
         // (512 x 512: 1, 2, 4, 8, 16 slices take 603, 656, 835, 1117, 1780 us, so that 11 to 15 go
-        // as 16, but 9 and 10 as 8 and the rest)
+        // as 16, but 9 and 10 as 8 and the rest); or all slices in one launch of one group size,
+        // where the costs say so: a launch costs about its group's time on the tiles times (its
+        // workgroups + 800), 800 standing for the time a launch takes that does not fill the chip
+        // (64 x 64 over 90 views, 9 slices: 8 and 1 44 us, pairs 21; 73 x 73 over 102, 41 slices:
+        // 16, 8 and 1 76 us, eights 34; 174 x 174 over 328, 21 slices: 207, eights 174; 256 x 256
+        // over 360, 17 slices: 16 and 1 399, eights 464).
+        static constexpr struct { int s; double time; } kGroups[] = {{1, 603}, {2, 656}, {4, 835}, {8, 1117}, {16, 1780}};
+        const long long tiles = (long long)adj_cell_tiles(A.nX) * adj_cell_tiles(A.nY);
+        auto cost = [&](int S, int groups) {
+            for (const auto &k : kGroups)
+                if (k.s == S) return k.time * ((double)(tiles * groups) + 800.0);
+            return 0.0;
+        };
+        auto rule = [](int left) { return left >= 11 ? 16 : left >= 5 ? 8 : left >= 3 ? 4 : left; };
+        double least = 0.0;
+        for (int left = n; left > 0; left -= rule(left) * std::max(left / rule(left), 1))
+            least += cost(rule(left), std::max(left / rule(left), 1));
+        int all = 0;
+        for (const auto &k : kGroups)
+            if (const double c = cost(k.s, (n + k.s - 1) / k.s); c < least) least = c, all = k.s;
         for (int done = 0; done < n && st == FBCT_OK;) {
             const int left = n - done;
-            const int S = left >= 11 ? 16 : left >= 5 ? 8 : left >= 3 ? 4 : left;
-            const int groups = std::max(left / S, 1);
+            const int S = all ? all : rule(left);
+            const int groups = all ? (left + S - 1) / S : std::max(left / S, 1);
             if (S == 16) st = launch_fpa_t<16>(ti, to, groups, stream, A, done);
             else if (S == 8) st = launch_fpa_t<8>(ti, to, groups, stream, A, done);
             else if (S == 4) st = launch_fpa_t<4>(ti, to, groups, stream, A, done);

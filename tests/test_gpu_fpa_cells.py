@@ -1,6 +1,7 @@
 """GPU: the cell-driven FP^T at its edges, against the FP64 oracle.
 
-Slice counts around the group sizes (1, 2, 4, 8, 16 and their padding), images around the 7 x 7
+Slice counts around the group sizes (1, 2, 4, 8, 16 and their padding, as groups of 16 and the rest
+and as one launch), images around the 7 x 7
 pixel tile, view counts around the quarters, detector windows from a few columns to more than a
 wave's 64 slots (fine detectors, and sources close to the image, where the window of a tile near
 the source covers the detector), both directions of the columns.
@@ -34,6 +35,8 @@ def _scan(side, views, cols, sid, fan, flip=False):
     (32, 20, 200, 80.0, 1.2, 1), (32, 20, 330, 80.0, 1.2, 4),    # 32 and 64 columns a window
     (20, 24, 700, 60.0, 1.2, 1), (20, 24, 500, 60.0, 1.2, 16),   # wider than the slots
     (24, 30, 40, 12.6, 1.0, 1), (24, 30, 400, 12.1, 1.0, 2),     # the source close to the image
+    (211, 5, 90, 500.0, 1.2, 17), (211, 4, 91, 500.0, 1.2, 21), (211, 6, 60, 500.0, 1.2, 11),  # groups of 16 and the rest
+    (120, 5, 90, 300.0, 1.2, 9), (120, 4, 70, 300.0, 1.2, 41), (90, 4, 70, 300.0, 1.2, 7),     # one padded launch
 ])
 @pytest.mark.parametrize("storage", ["f32", "bf16"])
 def test_cells(side, views, cols, sid, fan, slices, storage, oracle_mod):
