@@ -762,7 +762,7 @@ def main(argv=None):
         fpm = "8 flops and 4 taps per FP sample per slice (bilinear)"
         rl_fp = roofline("fp_kernel (two launches: tile classes)", ms["fp_step"], "clinical.fp_step",
                          prof, cal, 8 * samples * S, 8 * samples * S, fpm)
-        rl_adj = roofline("fp_adjoint_cell_staged_kernel", ms["fp_adjoint_step"],
+        rl_adj = roofline("fp_adjoint_cell_kernel", ms["fp_adjoint_step"],
                           "clinical.fp_adjoint_step", prof, cal, 8 * samples * S, 8 * samples * S, fpm)
         out["roofline"] = rl_fp if ms["fp_step"] >= ms["fp_adjoint_step"] else rl_adj
         out["roofline_fp"] = rl_fp
@@ -794,7 +794,7 @@ def main(argv=None):
     if args.workload in ("all", "fdk"):
         out, ctx = bench_fdk(torch, args)
         ms, U = ctx["ms"], ctx["U"]
-        out["roofline"] = roofline("cone_bp_lds_kernel<32-voxel z-chunks, float>", ms["backproject"],
+        out["roofline"] = roofline("cone_bp_tile_kernel<float>", ms["backproject"],
                                    "fdk.backproject", prof, cal, 8 * U, 16 * U,
                                    "8 flops and 4 taps of 4 B (FP32 filtered projections) per voxel-view update")
         rf = roofline("ramp_gemm_kernel<bf16 rows, cosine pre-weight>", ms["filter"], "fdk.filter", prof, cal,

@@ -1079,7 +1079,7 @@ fbct_status launch_bp(const fbct_plan &p, const DeviceTables &t, const float *si
     else if (weighted) launch_bp_nc<true, false>(A, nc, n, stream);
     else launch_bp_nc<false, false>(A, nc, n, stream);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "bp_kernel launch: %s", hipGetErrorString(e));
+    if (e != hipSuccess) return fail(FBCT_ERR_DEVICE, "backprojection launch: %s", hipGetErrorString(e));
     return FBCT_OK;
 }
 
