@@ -413,7 +413,7 @@ __global__ __launch_bounds__(1024, 8) void cone_bp_wave_kernel(ConeArgs A)
 // or over a fan edge in a view take that view's taps from global memory.
 //
 // Bound by VALU issue (10 instructions a voxel) and the LDS reads (two ds_read2_b32).  512 x 512 x 256
-// over 720 views 15.6 -> 14.8 ms, 300 x 300 x 256 over 360 3.09 -> 2.77 (rows through registers before,
+// over 720 views 15.6 -> 14.9 ms, 300 x 300 x 256 over 360 3.09 -> 2.75 (rows through registers before,
 // chunks of 32 voxels at four waves per SIMD); a window of 46 rows holds 16 voxels up to 1.7 rows
 // apart anywhere and most at 2.2 (320 x 320 x 160 over 400 at 1.5 rows 3.15 -> 2.31 ms).  The row
 // stride sets the bank conflicts (512 x 512 x 256: 65: 20.6 ms, 67: 19.6, 69: 17.5, 71: 15.9, 73 to 77:
@@ -431,7 +431,11 @@ __global__ __launch_bounds__(kTx *kTy, 6) void cone_bp_tile_kernel(ConeArgs A)
     __shared__ float stage[2 * kRows * RS];
     unsigned t, gz;
     xcd_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x * gridDim.y, gridDim.z, t, gz);
-    const int tx0 = (int)(t % gridDim.x) * kTx, ty0 = (int)(t / gridDim.x) * kTy;
+    // tiles in blocked order: the footprints of those that run together overlap in an XCD's L2 (512 x
+    // 512 x 256, 720 views: 15.3 -> 14.85 ms)
+    unsigned tbx, tby;
+    blocked_tile(t, gridDim.x, gridDim.y, tbx, tby);
+    const int tx0 = (int)tbx * kTx, ty0 = (int)tby * kTy;
     // each wave takes an 8x8 pixel quarter of the tile: its taps spread over fewer staged
     // rows and columns than a 16x4 strip's (fewer LDS bank conflicts)
     static_assert(kTx == 16 && kTy == 16, "lane layout assumes 16x16 tiles");
