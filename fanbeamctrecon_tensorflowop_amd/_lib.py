@@ -133,6 +133,7 @@ SIGNATURES = [
     ("fbct_cone_geom_from_params", _I, [_F, _I, _I, _I, ctypes.POINTER(ConeGeom)]),
     ("fbct_cone_plan_create", _I, [ctypes.POINTER(ConeGeom), _F, _I, ctypes.POINTER(_P)]),
     ("fbct_cone_plan_destroy", _I, [_P]),
+    ("fbct_cone_plan_windows", _I, [_P, _I, _I, _I, _I, ctypes.POINTER(ctypes.c_int32)]),
     ("fbct_cone_workspace_size", ctypes.c_size_t, [_P, _I]),
     ("fbct_cone_filter", _I, [_P, _P, _I, _P, _I, _P]),
     ("fbct_cone_backproject", _I, [_P, _P, _P, _I, _I, _P]),

@@ -93,6 +93,15 @@ class ConePlan:
         g = self.geom
         return g["nX"] * g["nY"] * g["nZ"] * g["nViews"]
 
+    def windows(self, side: int, i0: int, j0: int, k0: int) -> np.ndarray:
+        """int32 [nViews, 5]: staged, first and last column, first and last row of the detector window of
+        a staged backprojection tile (``fbct_cone_plan_windows``)."""
+        out = np.zeros((self.geom["nViews"], 5), dtype=np.int32)
+        _lib.check(_lib.load().fbct_cone_plan_windows(self._h, int(side), int(i0), int(j0), int(k0),
+                                                      out.ctypes.data_as(ctypes.POINTER(ctypes.c_int32))),
+                   "fbct_cone_plan_windows")
+        return out
+
     def _prep(self, x, shape, what):
         if not isinstance(x, torch.Tensor) or not x.is_cuda:
             raise ValueError("%s: expected a HIP device tensor; this library has no CPU path" % what)

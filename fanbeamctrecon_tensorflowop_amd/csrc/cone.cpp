@@ -140,6 +140,7 @@ void build(fbct_cone_plan &p)
     d.tan_min = std::min(t0, t1);
     d.tan_max = std::max(t0, t1);
     d.atan_nc = 0;
+    d.atan_zmax = 0.0f;
     std::fill(d.atan_c, d.atan_c + kBpAtanMax, 0.0f);
     if (!flat) {
         const double rf = g.rFOV;
@@ -147,6 +148,7 @@ void build(fbct_cone_plan &p)
         for (int nc : {5, 9})
             if (fit_atan(zmax, nc, d.atan_c)) {
                 d.atan_nc = nc;
+                d.atan_zmax = (float)zmax;
                 break;
             }
         if (d.atan_nc == 0) std::fill(d.atan_c, d.atan_c + kBpAtanMax, 0.0f);

@@ -46,11 +46,12 @@ struct ConeArgs {
     int ct_col, rt_row;
     float ct_lo, ct_hi;  // the detector's edges on the relative column axis
     double tan_min, tan_max;
+    float z_fit;  // the polynomial of atan holds for |t/U| <= z_fit, which covers the FOV disk
     float atan_c[kBpAtanMax];
 };
 
 template <int kNc>
-__device__ __forceinline__ float fan_atan(const ConeArgs &A, float z)
+__host__ __device__ __forceinline__ float fan_atan(const ConeArgs &A, float z)
 {
     if constexpr (kNc == 0) {
         return atanf(z);
@@ -72,9 +73,18 @@ __device__ __forceinline__ int cvt_floor(float v)
     return r;
 }
 
-__device__ __forceinline__ int floor_to_int(float v)
+__host__ __device__ __forceinline__ int floor_to_int(float v)
 {
     return (int)floorf(fminf(fmaxf(v, -1.0e6f), 1.0e6f));
+}
+
+__host__ __device__ __forceinline__ float reciprocal(float x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_rcpf(x);
+#else
+    return 1.0f / x;
+#endif
 }
 
 // cos and sin of a uniform view's angle, by a scalar load: a vector load would wait behind the rows in
@@ -94,16 +104,19 @@ struct ColumnView {
     float U;   // distance from the source along the central ray
 };
 
-template <bool kFlat, int kNc>
-__device__ __forceinline__ ColumnView column_view(const ConeArgs &A, float2 cs, float x, float y)
+// kAnywhere: (x, y) may lie outside the FOV disk, where the polynomial of atan turns away from it; t/U
+// is cut to the range it was fitted on.
+template <bool kFlat, int kNc, bool kAnywhere = false>
+__host__ __device__ __forceinline__ ColumnView column_view(const ConeArgs &A, float2 cs, float x, float y)
 {
     const float U = fmaf(-y, cs.y, fmaf(-x, cs.x, A.R));
     const float t = fmaf(x, cs.y, -y * cs.x);
-    const float rU = __builtin_amdgcn_rcpf(U);
-    const float z = t * rU;
+    const float rU = reciprocal(U);
+    float z = t * rU;
+    if constexpr (kAnywhere && !kFlat && kNc > 0) z = fminf(fmaxf(z, -A.z_fit), A.z_fit);
     ColumnView c;
     c.ct = fmaf(kFlat ? z : fan_atan<kNc>(A, z), A.xi_scale, A.ct_offset);
-    c.w = kFlat ? rU * rU : __builtin_amdgcn_rcpf(fmaf(U, U, t * t));
+    c.w = kFlat ? rU * rU : reciprocal(fmaf(U, U, t * t));
     c.a = rU * A.zr_scale;
     c.U = U;
     return c;
@@ -182,46 +195,78 @@ __device__ __forceinline__ void column_staged(const ColumnView &c, float rt0, fl
     }
 }
 
-// Windows of sixteen views, view vg + m's in lane 4m: the first and last column and row (relative to
-// ct_col and rt_row) of a tile's taps, from its corner columns (corner c in lane 4m + c) and the ends
-// of its z-chunk, with a margin of one sample, which absorbs the rounding between corner and voxel.
-// A corner at or behind the source makes the window too wide to be used.
-struct Window {
+// What one corner column of a tile says about a view's window: its column coordinate (least and
+// greatest, apart where the window is not to be used) and its row coordinates at the ends of the
+// z-chunk.  A corner outside the FOV disk is cut to the range of t/U that the disk's voxels keep to,
+// and t/U and 1/U are extremal at a corner, so the corners bound every voxel of the disk in the tile.
+// A corner at or behind the source, or rows beyond +-1e6 (where the window's ends would be cut), put
+// the window off the detector.
+struct Corner {
+    float cn, cm, rn, rx;
+};
+template <bool kFlat, int kNc>
+__host__ __device__ __forceinline__ Corner corner_of(const ConeArgs &A, float2 cs, int i, int j, float z0, float z1)
+{
+    const ColumnView c = column_view<kFlat, kNc, true>(A, cs, fmaf(A.dx, (float)i + 0.5f, A.xmin),
+                                                       fmaf(A.dy, (float)j + 0.5f, A.ymin));
+    const float ra = fmaf(z0, c.a, A.rt_offset), rb = fmaf(z1, c.a, A.rt_offset);
+    const Corner k{c.ct, c.ct, fminf(ra, rb), fmaxf(ra, rb)};
+    const bool usable = c.U > 1.0e-3f * A.R && k.rn > -1.0e6f && k.rx < 1.0e6f;
+    return usable ? k : Corner{-1.0e6f, c.ct, k.rn, k.rx};
+}
+
+// The first and last column and row (relative to ct_col and rt_row) of a tile's taps in a view, from
+// the extremes over its corners, with a margin of one sample, which absorbs the rounding between
+// corner and voxel.
+struct Range {
     int c0, c1, r0, r1;
+};
+__host__ __device__ __forceinline__ Range range_of(const Corner &k)
+{
+    return {floor_to_int(k.cn) - 1, floor_to_int(k.cm) + 2, floor_to_int(k.rn) - 1, floor_to_int(k.rx) + 2};
+}
+// Whether a tile is staged in a view: its window inside the detector's columns and at most `cols` x
+// `rows`.
+__host__ __device__ __forceinline__ bool is_staged(const ConeArgs &A, const Range &r, int cols, int rows)
+{
+    return r.c0 + A.ct_col >= 0 && r.c1 + A.ct_col < A.nCols && r.c1 - r.c0 < cols && r.r1 - r.r0 < rows;
+}
+
+// Windows of sixteen views, view vg + m's in lane 4m, corner c's evaluated by lane 4m + c.
+struct Window {
+    Range w;
     template <bool kFlat, int kNc>
     __device__ __forceinline__ void eval(const ConeArgs &A, int vg, int i0, int i1, int j0, int j1, float z0, float z1)
     {
         const int lane = (int)threadIdx.x & 63;
-        const float cx = fmaf(A.dx, (float)((lane & 1) ? i1 : i0) + 0.5f, A.xmin);
-        const float cy = fmaf(A.dy, (float)((lane & 2) ? j1 : j0) + 0.5f, A.ymin);
         const int v = min(vg + (lane >> 2), A.nViews - 1);
-        const ColumnView c = column_view<kFlat, kNc>(A, A.cs[v], cx, cy);
-        float cn = c.ct, cm = c.ct;
-        if (!(c.U > 1.0e-3f * A.R)) cn = -1.0e6f;
-        const float ra = fmaf(z0, c.a, A.rt_offset), rb = fmaf(z1, c.a, A.rt_offset);
-        float rn = fminf(ra, rb), rx = fmaxf(ra, rb);
+        Corner k = corner_of<kFlat, kNc>(A, A.cs[v], (lane & 1) ? i1 : i0, (lane & 2) ? j1 : j0, z0, z1);
 #pragma unroll
         for (int sh = 1; sh <= 2; sh <<= 1) {
-            cn = fminf(cn, __shfl_xor(cn, sh));
-            cm = fmaxf(cm, __shfl_xor(cm, sh));
-            rn = fminf(rn, __shfl_xor(rn, sh));
-            rx = fmaxf(rx, __shfl_xor(rx, sh));
+            k.cn = fminf(k.cn, __shfl_xor(k.cn, sh));
+            k.cm = fmaxf(k.cm, __shfl_xor(k.cm, sh));
+            k.rn = fminf(k.rn, __shfl_xor(k.rn, sh));
+            k.rx = fmaxf(k.rx, __shfl_xor(k.rx, sh));
         }
-        c0 = floor_to_int(cn) - 1;
-        c1 = floor_to_int(cm) + 2;
-        r0 = floor_to_int(rn) - 1;
-        r1 = floor_to_int(rx) + 2;
+        w = range_of(k);
     }
-    // View vg + m's window, and whether a tile with it is staged: inside the detector's columns and
-    // at most `cols` x `rows`.
+    // View vg + m's window (its first column and row and its rows), and whether the tile is staged.
     __device__ __forceinline__ bool view(const ConeArgs &A, int m, int cols, int rows, int &vc0, int &vr0, int &nrow) const
     {
-        vc0 = __builtin_amdgcn_readlane(c0, 4 * m), vr0 = __builtin_amdgcn_readlane(r0, 4 * m);
-        const int vc1 = __builtin_amdgcn_readlane(c1, 4 * m);
-        nrow = __builtin_amdgcn_readlane(r1, 4 * m) - vr0 + 1;
-        return vc0 + A.ct_col >= 0 && vc1 + A.ct_col < A.nCols && vc1 - vc0 < cols && nrow <= rows;
+        const Range r{__builtin_amdgcn_readlane(w.c0, 4 * m), __builtin_amdgcn_readlane(w.c1, 4 * m),
+                      __builtin_amdgcn_readlane(w.r0, 4 * m), __builtin_amdgcn_readlane(w.r1, 4 * m)};
+        vc0 = r.c0, vr0 = r.r0, nrow = r.r1 - r.r0 + 1;
+        return is_staged(A, r, cols, rows);
     }
 };
+
+// The staged loops' columns: lanes outside the FOV disk evaluate the first column of the wave inside it
+// (their own may lie outside the windows) and are not stored.
+__device__ __forceinline__ float inside_column(float xy, bool active, unsigned long long in)
+{
+    const float first = __shfl(xy, in != 0 ? __builtin_ctzll(in) : 0);
+    return active ? xy : first;
+}
 
 // The views of [vbeg, vend) in which a tile is not staged, from global memory.  (A pass of its own:
 // the staged views' loop then updates its sums in one place, and reads taps well ahead of their use.)
@@ -343,9 +388,11 @@ __global__ __launch_bounds__(1024, 8) void cone_bp_wave_kernel(ConeArgs A)
     const unsigned zg = (unsigned)A.gz0 + gz;
     const int k0 = (int)(zg % A.nzc) * KZ;
     const size_t vi = zg / A.nzc;
-    const float x = fmaf(A.dx, (float)i + 0.5f, A.xmin);
-    const float y = fmaf(A.dy, (float)j + 0.5f, A.ymin);
-    const bool active = x * x + y * y <= A.r2;
+    const float xp = fmaf(A.dx, (float)i + 0.5f, A.xmin);
+    const float yp = fmaf(A.dy, (float)j + 0.5f, A.ymin);
+    const bool active = xp * xp + yp * yp <= A.r2;
+    const unsigned long long in = __ballot(active);
+    const float x = inside_column(xp, active, in), y = inside_column(yp, active, in);
     const float z0 = fmaf(A.dz, (float)k0 + 0.5f, A.zmin);
     const float z1 = fmaf(A.dz, (float)(k0 + KZ - 1) + 0.5f, A.zmin);
     const int nC = A.nCols, nR = A.nRows;
@@ -359,7 +406,7 @@ __global__ __launch_bounds__(1024, 8) void cone_bp_wave_kernel(ConeArgs A)
     for (int k = 0; k < KZ; ++k) acc[k] = 0.0f;
 
     const int vbeg = A.nViews * wave / waves;
-    const int vend = __ballot(active) != 0 ? A.nViews * (wave + 1) / waves : vbeg;
+    const int vend = in != 0 ? A.nViews * (wave + 1) / waves : vbeg;
     Window win;
     // staging of a window, two rows per load and sixteen rows at a time (a wave's LDS accesses
     // complete in order, so it waits for nothing but its own loads)
@@ -449,10 +496,12 @@ __global__ __launch_bounds__(kTx *kTy, 6) void cone_bp_tile_kernel(ConeArgs A)
     const size_t vi = zg / A.nzc;
     const int lane = (int)threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const float x = fmaf(A.dx, (float)i + 0.5f, A.xmin);
-    const float y = fmaf(A.dy, (float)j + 0.5f, A.ymin);
-    const bool active = x * x + y * y <= A.r2;
-    const bool wave_active = __ballot(active) != 0;
+    const float xp = fmaf(A.dx, (float)i + 0.5f, A.xmin);
+    const float yp = fmaf(A.dy, (float)j + 0.5f, A.ymin);
+    const bool active = xp * xp + yp * yp <= A.r2;
+    const unsigned long long in = __ballot(active);
+    const bool wave_active = in != 0;
+    const float x = inside_column(xp, active, in), y = inside_column(yp, active, in);
     // Row coordinate of voxel k: rt_k = rt_0 + k (dz a), rt_0 = z_0 a + rt_offset and
     // a = zr_scale / U -- one fma with k as an immediate.
     const float z0 = fmaf(A.dz, (float)k0 + 0.5f, A.zmin);
@@ -603,15 +652,14 @@ ConeLaunch choose(const fbct_cone_geom &g, double zr_scale)
 
 }  // namespace
 
-fbct_status launch_cone_bp(const fbct_cone_plan &p, const ConeDeviceTables &t, const float *q,
-                           void *vol, fbct_dtype to, int n, hipStream_t stream)
+// The launch's arguments that the plan fixes; `cs` and `csd`: its angles, on the device or (csd unused) on
+// the host.
+static ConeArgs cone_args(const fbct_cone_plan &p, const float2 *cs, const double2 *csd)
 {
     const fbct_cone_geom &g = p.g;
-    ConeArgs A;
-    A.q = q;
-    A.vol = vol;
-    A.cs = t.view_cs;
-    A.csd = t.view_csd;
+    ConeArgs A{};
+    A.cs = cs;
+    A.csd = csd;
     A.nX = g.nX;
     A.nY = g.nY;
     A.nZ = g.nZ;
@@ -636,7 +684,18 @@ fbct_status launch_cone_bp(const fbct_cone_plan &p, const ConeDeviceTables &t, c
     A.ct_hi = (float)(g.nCols - p.d.ct_col) - 0.5f;
     A.tan_min = p.d.tan_min;
     A.tan_max = p.d.tan_max;
+    A.z_fit = p.d.atan_zmax;
     for (int k = 0; k < kBpAtanMax; ++k) A.atan_c[k] = p.d.atan_c[k];
+    return A;
+}
+
+fbct_status launch_cone_bp(const fbct_cone_plan &p, const ConeDeviceTables &t, const float *q,
+                           void *vol, fbct_dtype to, int n, hipStream_t stream)
+{
+    const fbct_cone_geom &g = p.g;
+    ConeArgs A = cone_args(p, t.view_cs, t.view_csd);
+    A.q = q;
+    A.vol = vol;
     const ConeLaunch L = choose(g, p.d.zr_scale);
     const int kz_most = g.nZ >= 32 ? 32 : (g.nZ >= 16 ? 16 : (g.nZ >= 4 ? 4 : 1));
     const long long most = (long long)((g.nZ + kz_most - 1) / kz_most) * n;
@@ -660,3 +719,36 @@ fbct_status launch_cone_bp(const fbct_cone_plan &p, const ConeDeviceTables &t, c
 }
 
 }  // namespace fbct
+
+extern "C" fbct_status fbct_cone_plan_windows(const fbct_cone_plan *plan, int side, int i0, int j0, int k0, int32_t *out)
+{
+    using namespace fbct;
+    if (!plan || !out) return fail(FBCT_ERR_INVALID_ARGUMENT, "fbct_cone_plan_windows: null pointer");
+    const fbct_cone_geom &g = plan->g;
+    if ((side != 8 && side != 16) || i0 < 0 || i0 >= g.nX || j0 < 0 || j0 >= g.nY || k0 < 0 || k0 >= g.nZ)
+        return fail(FBCT_ERR_INVALID_ARGUMENT, "fbct_cone_plan_windows: side 8 or 16 and a voxel of the volume");
+    const ConeArgs A = cone_args(*plan, nullptr, nullptr);
+    const int kz = side == 8 ? kWaveKz : kTileKz;
+    const int cols = side == 8 ? kWaveCols : kTileCols, rows = side == 8 ? kWaveRows : kTileRows;
+    const int i1 = std::min(i0 + side - 1, g.nX - 1), j1 = std::min(j0 + side - 1, g.nY - 1);
+    const float z0 = fmaf(A.dz, (float)k0 + 0.5f, A.zmin), z1 = fmaf(A.dz, (float)(k0 + kz - 1) + 0.5f, A.zmin);
+    const bool flat = g.detector == FBCT_DETECTOR_FLAT;
+    for (int v = 0; v < g.nViews; ++v) {
+        const float2 cs = make_float2(plan->view_cs[2 * v], plan->view_cs[2 * v + 1]);
+        Corner k{};
+        for (int c = 0; c < 4; ++c) {
+            const int i = (c & 1) ? i1 : i0, j = (c & 2) ? j1 : j0;
+            const Corner q = flat                     ? corner_of<true, 0>(A, cs, i, j, z0, z1)
+                             : plan->d.atan_nc == 9 ? corner_of<false, 9>(A, cs, i, j, z0, z1)
+                             : plan->d.atan_nc == 5 ? corner_of<false, 5>(A, cs, i, j, z0, z1)
+                                                    : corner_of<false, 0>(A, cs, i, j, z0, z1);
+            k = c == 0 ? q
+                       : Corner{fminf(k.cn, q.cn), fmaxf(k.cm, q.cm), fminf(k.rn, q.rn), fmaxf(k.rx, q.rx)};
+        }
+        const Range r = range_of(k);
+        int32_t *o = out + 5 * v;
+        o[0] = is_staged(A, r, cols, rows);
+        o[1] = r.c0 + A.ct_col, o[2] = r.c1 + A.ct_col, o[3] = r.r0 + A.rt_row, o[4] = r.r1 + A.rt_row;
+    }
+    return FBCT_OK;
+}

@@ -249,6 +249,7 @@ struct ConeDerived {
     int edge_exact;             // 1: the in-range decision near the edges is retaken in FP64 on t/U
     double tan_min, tan_max;    //    0 < xi < nCols  <=>  tan_min < t/U < tan_max
     int atan_nc;                // curved: coefficients of the atan correction polynomial (0 = atanf)
+    float atan_zmax;            // it is fitted on |t/U| <= atan_zmax, which the FOV disk's columns keep to
     float atan_c[kBpAtanMax];
     int ramp_np, ramp_kp, ramp_lg;
 };

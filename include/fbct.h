@@ -370,6 +370,13 @@ fbct_status fbct_cone_plan_create(const fbct_cone_geom *geom, const float *angle
                                   fbct_cone_plan **out);
 fbct_status fbct_cone_plan_destroy(fbct_cone_plan *plan);
 
+/* The detector windows that the staged backprojection kernels use for the tile of side x side
+ * pixels (8: eight slices a tile, 16: sixteen) at pixel (i0, j0) and slice k0: out[nViews][5] =
+ * staged (0 or 1), first and last column, first and last row (rows may lie beyond the detector; they
+ * repeat its edges).  Where staged, every tap of the tile's voxels inside rFOV lies in the window.  No
+ * counterpart in the reference (a texture fetch per voxel); it lets tests check the windows on the host. */
+fbct_status fbct_cone_plan_windows(const fbct_cone_plan *plan, int side, int i0, int j0, int k0, int32_t *out);
+
 /* Workspace bytes for fbct_cone_fdk on n volumes: the filtered projections as FP32
  * rows, 4 bytes per detector sample. */
 size_t fbct_cone_workspace_size(const fbct_cone_plan *plan, int n);
