@@ -292,6 +292,15 @@ __device__ __forceinline__ void unstaged_views(const ConeArgs &A, int vbeg, int 
     }
 }
 
+// Orders a wave's LDS accesses where its lanes read what others wrote, or write over what others read: the
+// hardware completes them in program order, so nothing waits, but the compiler sees one lane's addresses
+// and must not move them across.
+__device__ __forceinline__ void wave_lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // The wave kernels: a workgroup owns an 8 x 8 pixel tile of KZ voxels; its waves split the
 // views and add their sums at the end (in wave order).  LDS: per wave `wave_floats` floats.
 extern __shared__ float cone_lds[];
@@ -313,6 +322,7 @@ __device__ __forceinline__ void store_columns(const ConeArgs &A, const float (&a
         return;
     }
     float *mine = cone_lds + wave * wave_floats + lane;
+    wave_lds_order();  // the last window's reads
 #pragma unroll
     for (int k = 0; k < KZ; ++k) mine[64 * k] = acc[k];  // its own staging area: no wait for others
     __syncthreads();
@@ -437,9 +447,11 @@ __global__ __launch_bounds__(1024, 8) void cone_bp_wave_kernel(ConeArgs A)
                 for (int u = 0; u < 8; ++u)
                     p[u] = load_at(qv, (unsigned)min(max(gr + k + lrow + 2 * u, 0), nR - 1) * row_bytes + c4);
             }
+            if (k == 0) wave_lds_order();  // the previous window's reads
 #pragma unroll
             for (int u = 0; u < 8; ++u) dst[(k + 2 * u) * P] = p[u];
         }
+        wave_lds_order();
         column_staged<KZ, P>(c, rt0, step, lds0 + 4u * (unsigned)(cvt_floor(c.ct) - c0 - r0 * P), acc);
     }
     if (unstaged)

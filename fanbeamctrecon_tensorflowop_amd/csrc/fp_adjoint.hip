@@ -709,9 +709,15 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
             for (int s = 0; s < S; ++s) pv[s] = sino[s][rb];
         }
     };
+    // the wave's lanes read each other's slots: keep the order, LDS keeps it too
+    auto slots_order = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+    };
     auto store_ray = [&]() {
         float *d = slots + lane * kDw;
         const float n = (float)pn, dd = pg.z * pg.w * (1.0f / 12.0f);
+        slots_order();  // the previous rays' reads
         *reinterpret_cast<float4 *>(d) = pg;
         *reinterpret_cast<float4 *>(d + 4) = make_float4(pi.x, pi.y, -pg.x * pi.x, -pg.y * pi.y);
         if constexpr (S >= 4) {
@@ -723,9 +729,7 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         } else {
             *reinterpret_cast<float4 *>(d + 8) = make_float4(n, dd, widen(pv[0]), widen(pv[S - 1]));
         }
-        // the wave's lanes read each other's slots: keep the order, LDS keeps it too
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+        slots_order();
     };
     struct Ray {
         RayRec rec;
@@ -863,8 +867,6 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                             read_ray(slots + (c - w) * kDw, r);
                             add_ray(std::true_type{}, r);
                         }
-                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                        __builtin_amdgcn_wave_barrier();
                     }
                 }
                 if (kAhead && vn < v_end) {
