@@ -942,8 +942,9 @@ __global__ __launch_bounds__(kAdjThreads, 6) void fp_adjoint_batch_kernel(const 
                                                                        int total, const TI *sino, TO *img)
 {
     __shared__ CellShared<1> sh;
-    const int first = (int)xcd_chunk(blockIdx.x, gridDim.x);
-    for (int item = first; item < total; item += gridDim.x) {
+    const unsigned first = xcd_chunk(blockIdx.x, gridDim.x);
+    for (unsigned at = first; at < (unsigned)total; at += gridDim.x) {  // (total < 2^31, the grid below 2^24)
+        const int item = (int)at;
         int lo = 0, hi = n - 1;  // last slice with prefix[s] <= item
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -1122,9 +1123,10 @@ fbct_status launch_fp_adjoint_batch(const fbct_batch &b, const BatchDevice &bd, 
     if (k == kAdjNumTiles) return fail(FBCT_ERR_INVALID_ARGUMENT, "fbct_batch_fp_adjoint: tile width %d", b.shape.adj_tile_x);
     const int total = b.fpa_prefix[k][n];
     if (total == 0) return FBCT_OK;
-    const long long wgs = b.shape.adj_wgs_per_cu == 0
-                              ? total
-                              : std::min<long long>(total, (long long)b.shape.adj_wgs_per_cu * bd.num_cu);
+    // (a grid holds fewer than 2^32 threads; beyond, its workgroups stride over the items)
+    const long long most = b.shape.adj_wgs_per_cu == 0 ? 0xffffffffLL / kAdjThreads
+                                                       : (long long)b.shape.adj_wgs_per_cu * bd.num_cu;
+    const long long wgs = std::min<long long>(total, most);
     const dim3 grid((unsigned)wgs);
     const int *prefix = bd.fpa_prefix[k];
     switch (b.shape.adj_tile_x) {
