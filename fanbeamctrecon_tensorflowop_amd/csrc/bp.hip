@@ -520,6 +520,7 @@ struct BpaArgs {
     const int2 *fov_row, *fov_col;
     long long img_stride, sino_stride;
     int nX, nY, nViews, nCols, nSlices, win;
+    unsigned cblocks, vgroups;  // workgroups along the columns and the views
     double R, xmin, ymin, dx, dy;
     float rFOV, tanc, icol;  // rFOV, tan|dCol|, 1/dCol
 };
@@ -684,9 +685,10 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
     if (threadIdx.x == 0) put(zero_at, TapT{});
     __shared__ int2 fovc[kBpaChunk];  // FOV ranges of the chunk's lines
     __shared__ int red[2][4];
-    unsigned cb, vg, g;  // blocked, XCD-aware order over (column block, view group, slice group)
-    xcd_blocked_tile(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, gridDim.z,
-                     cb, vg, g);
+    // blocked, XCD-aware order over (column block, view group, slice group); the first two share the grid's
+    // x, since either may exceed what its y holds
+    unsigned cb, vg, g;
+    xcd_blocked_tile(blockIdx.x + gridDim.x * blockIdx.z, A.cblocks, A.vgroups, gridDim.z, cb, vg, g);
     const int lane = (int)threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int c = (int)cb * 64 + lane;
@@ -1123,6 +1125,8 @@ fbct_status launch_bp_adjoint(const fbct_plan &p, const DeviceTables &t, const f
     const double dview = p.g.nViews > 1 ? fabs((double)p.angles[p.g.nViews - 1] - p.angles[0]) / (p.g.nViews - 1) : 0.0;
     const int cblocks = (p.g.nCols + 63) / 64;
     const bool split = (long long)cblocks * ((p.g.nViews + 3) / 4) < 300 || 64.0 * dcol + 4.0 * dview > 0.52;
+    A.cblocks = cblocks;
+    A.vgroups = split ? p.g.nViews : (p.g.nViews + 3) / 4;
     // Staged pixels per line: what 64 columns reach at the far end of the FOV disk on a ray 45
     // degrees off the axis, the views' spread, a chunk's slant and margins; at most the image and
     // kBpaWin (wider windows read global memory)
@@ -1134,7 +1138,7 @@ fbct_status launch_bp_adjoint(const fbct_plan &p, const DeviceTables &t, const f
         int S = left >= 5 ? 8 : left >= 3 ? 4 : left;  // padded with the last slice
         while ((unsigned long long)S * img_bytes >= (1ULL << 32)) S /= 2;
         const int groups = std::max(left / S, 1);
-        const dim3 grid(cblocks, split ? p.g.nViews : (p.g.nViews + 3) / 4, groups);
+        const dim3 grid(A.cblocks * A.vgroups, 1, groups);
         const size_t lds = std::max(sizeof(float) * S * (kBpaChunk * (size_t)A.win + 1), sizeof(double) * 256);
 #define FBCT_BPA(SS)                                                                                            \
     if (split && weighted) hipLaunchKernelGGL((bp_adjoint_staged_kernel<true, SS, true>), grid, dim3(256), lds, stream, A, done); \

@@ -22,3 +22,16 @@ def test_uneven_adjoint_of_many_slices():
     out = batch.fp_adjoint(y.reshape(-1))
     for s in (0, n // 2, n - 2, n - 1):
         assert torch.equal(batch.image(out, s), plan.fp_adjoint(y[s:s + 1])[0]), s
+
+
+@pytest.mark.parametrize("views,dcol", [(70000, 0.02), (270000, 0.006)])  # a view a workgroup, four views
+def test_bp_adjoint_of_many_views(views, dcol, oracle_mod):
+    # more than 65536 view groups, in either split of the work
+    p, a = workloads.scan(nx=4, rfov=2.0, sid=60.0, sdd=120.0, n_cols=8, dcol_rad=dcol, n_views=views)
+    plan, o = FanBeamPlan(p, a), oracle_mod.Oracle(p, a)
+    x = np.random.default_rng(views).normal(size=(2,) + plan.image_shape).astype(np.float32)
+    for fn, weighted in ((plan.bp_adjoint, False), (plan.fbp_weighted_bp_adjoint, True)):
+        got = fn(torch.from_numpy(x).cuda()).double().cpu().numpy()
+        e = rel_l2(got, o.bp_adjoint(x, weighted=True) if weighted else o.bp_adjoint(x))
+        print("%d views: %.2e" % (views, e), flush=True)
+        assert e <= 1e-5
