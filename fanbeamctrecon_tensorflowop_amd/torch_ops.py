@@ -36,12 +36,19 @@ __all__ = ["OPS"]
 _impl = torch.library.Library("fbct", "IMPL")
 
 
+def _device_kernel(fn):
+    """fn as a dispatcher kernel.  Where a compiled function calls an op from a frame that Dynamo leaves
+    to Python, Dynamo would go on into fn (its array conversions and ctypes calls) as into any callee;
+    the kernels that custom_op makes are closed to it, and so is this one (0.5 us a call)."""
+    return torch._disable_dynamo(fn)
+
+
 def _register(fn):
     """The custom op ``fbct::<name of fn>``.  On device tensors the dispatcher calls fn itself: the
     wrapper that custom_op puts around it compares inputs and outputs for aliasing on every call (10
     us), and the outputs here are new tensors."""
     op = torch.library.custom_op("fbct::" + fn.__name__, mutates_args=())(fn)
-    _impl.impl(fn.__name__, fn, "CUDA")
+    _impl.impl(fn.__name__, _device_kernel(fn), "CUDA")
     return op
 
 
