@@ -757,22 +757,11 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         constexpr bool kMixed = decltype(mixed)::value;
         const CellSums c = cell_sums<kMixed>(ray.rec, fci, fcj, kMixed ? fci : ulo, kMixed ? fci + 1.0f : uhi,
                                              kMixed ? fcj : wlo, kMixed ? fcj + 1.0f : whi);
-        if constexpr (S <= 2) {
+        const float r[4] = {c.n, c.n * c.ta, c.n * c.tm, c.n * c.g};
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const float nv = c.n * ray.v[s];
-                acc[0][s] += nv;
-                acc[1][s] = fmaf(c.ta, nv, acc[1][s]);
-                acc[2][s] = fmaf(c.tm, nv, acc[2][s]);
-                acc[3][s] = fmaf(c.g, nv, acc[3][s]);
-            }
-        } else {
-            const float r[4] = {c.n, c.n * c.ta, c.n * c.tm, c.n * c.g};
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int s = 0; s < S; ++s) acc[q][s] = fmaf(r[q], ray.v[s], acc[q][s]);
-        }
+            for (int s = 0; s < S; ++s) acc[q][s] = fmaf(r[q], ray.v[s], acc[q][s]);
     };
     // nit >= 1 adjacent slots from d
     auto add_rays = [&](auto mixed, const float *d, int nit) {
