@@ -507,11 +507,14 @@ __global__ __launch_bounds__(kBpTx *kBpTy *VG) void bp_staged_kernel(BpArgs A, i
 // from global memory.
 //
 // Bound: VALU issue (0.6) and the latency of a chunk (two barriers, the staging loads, the
-// candidates' chains).  512 x 512 pixels, 984 views, 888 columns, against two views per thread with a
-// candidate loop per lane: 1 slice 831 -> 573 us, 4 slices 831 -> 645 us, 16 slices 1.74 -> 1.56 ms;
-// 256 x 256, 360 views, 512 columns, 1 slice 164 -> 107 us.  8 slices with their float4 planes apart (a
-// 32-byte pixel made 16-byte reads conflict two-fold) 1029 -> 996 us, with the window sized by
-// the plan instead of 160 pixels (four workgroups per CU instead of three) 846 us.
+// candidates' chains).  With the distance weight, 512 x 512 pixels, 984 views, 888 columns, against
+// two views per thread with a candidate loop per lane: 1 slice 805 -> 598 us, 4 slices 887 -> 682 us, 16
+// slices 1.94 -> 1.62 ms; 256 x 256, 360 views, 512 columns, 1 slice 172 -> 104 us.  With 8 slices (1.12
+// ms -> 884 us) float4 planes apart gave 3% (a 32-byte pixel made 16-byte reads conflict two-fold), the
+// window sized by the plan instead of 160 pixels (four workgroups per CU instead of three) 15%.
+// Against 64 bits the results are 5 to 18% closer than with a candidate's place from an FP64 crossing
+// rounded to FP32 (RMS of 1 slice as above 5.9e-8 against 6.8e-8); the crossing in single FP32 steps was 4%
+// faster and up to 13% further off than that.
 struct BpaArgs {
     const float *img;
     float *sino;
@@ -522,11 +525,12 @@ struct BpaArgs {
     int nX, nY, nViews, nCols, nSlices, win;
     unsigned cblocks, vgroups;  // workgroups along the columns and the views
     double R, xmin, ymin, dx, dy;
-    float rFOV, tanc, icol;  // rFOV, tan|dCol|, 1/dCol
+    double icol;       // 1/dCol
+    float rFOV, tanc;  // rFOV, tan|dCol|
 };
 
 constexpr int kBpaChunk = 8;                 // lines per staged chunk
-constexpr float kBpaTan = 0.015f;            // tan^4 below an FP32 rounding
+constexpr float kBpaTan = 0.0125f;           // 1.2 tan^4 < 2^-25
 constexpr int kBpaFar = 1 << 24;             // beyond any window
 constexpr int kBpaWin = 160;                 // most staged pixels per line
 
@@ -550,9 +554,10 @@ struct BpaRay {
     int klo, khi;              // lines holding candidates (klo > khi: none)
 };
 
-// The same for the staged chunks: a = a32 + da, and pd, pl times the pixel pitch along the line.
+// The same for the staged chunks: a = a32 + da with a32 a multiple of 2^-23; pd, pl times the pixel
+// pitch along the line; 1/dCol for these.
 struct BpaStep {
-    float a32, da, hpd, hpl;
+    float a32, da, hpd, hpl, icol;
 };
 
 __device__ __forceinline__ void bpa_ray(const BpaArgs &A, double cth, double sth, double Rs, double Rc, bool along_y,
@@ -659,9 +664,10 @@ __device__ __forceinline__ int wave_max(int x)
     return wave_reduce(x, [](int a, int b) { return max(a, b); });
 }
 
-// Slices [slice0 + S*g, +S) of the batch, g = the workgroup's slice group.
+// Slices [slice0 + S*g, +S) of the batch, g = the workgroup's slice group.  The waves per SIMD are what
+// the LDS window leaves room for (one fewer, from 3 registers more: 4 slices 5%).
 template <bool kWeighted, int S, bool kSplit>
-__global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int slice0)
+__global__ __launch_bounds__(256, S == 8 ? 4 : S == 4 ? 6 : S == 2 ? 7 : 8) void bp_adjoint_staged_kernel(BpaArgs A, int slice0)
 {
     constexpr int kLines = kBpaChunk / 4;  // kSplit: lines of a chunk per wave
     constexpr int kBpaViewsWg = kSplit ? 1 : 4;  // views per workgroup
@@ -713,8 +719,8 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
     hh.chi = c == A.nCols - 1 ? 0.0f : 3.0e38f;
     hh.cut_lo = c == 0 ? -0.5f : -1.0f;
     hh.cut_hi = c == A.nCols - 1 ? 0.5f : 1.0f;
-    hh.icol = A.icol;
-    hh.c3 = -A.icol * (1.0f / 3.0f);
+    hh.icol = (float)A.icol;
+    hh.c3 = -hh.icol * (1.0f / 3.0f);
 
     BpaRay r;
     int kmin = INT_MAX, kmax = INT_MIN;
@@ -766,9 +772,12 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
     for (int s = 0; s < S; ++s) accd[s] = 0.0;
 
     BpaStep st;
-    st.a32 = (float)r.a;
+    st.a32 = (float)(rint(r.a * 0x1p23) * 0x1p-23);
     st.da = (float)(r.a - (double)st.a32);
-    st.hpd = h * r.pd, st.hpl = h * r.pl;
+    // (what rounds hpd would be an error of all of the ray's weights: icol takes it back)
+    const double hpd = along_y ? A.dx * sth : -A.dy * cth;
+    st.hpd = (float)hpd, st.hpl = (float)(along_y ? -A.dx * cth : -A.dy * sth);
+    st.icol = (float)(A.icol * hpd / (double)st.hpd);
 
     // chunks at multiples of kBpaChunk lines: a ray's sums do not depend on its workgroup
     for (int k0 = Klo & ~(kBpaChunk - 1); k0 <= Khi; k0 += kBpaChunk) {
@@ -779,7 +788,9 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
         int wlo = INT_MAX, whi = INT_MIN;
         const double m0 = fma(r.a, (double)k0, r.b);
         const double fl = floor(m0);
-        const float fr0 = (float)(m0 - fl);
+        // the crossing's fraction as a multiple of 2^-23 and the rest
+        const float fr0 = (float)(floor((m0 - fl) * 0x1p23) * 0x1p-23);
+        const float fr1 = (float)((m0 - fl) - (double)fr0);
         const int mi0 = (int)fl;
         const int ka = max(k0, r.klo), kb = min(k1, r.khi);
         const bool on = !own && ka <= kb;
@@ -840,7 +851,7 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
         __syncthreads();  // tile ready
         if (!wide) {
             // general: the hat of any column and the weight at any column pitch; else max(1 - |rel|, 0)
-            // and the weight's series
+            // and the series of narrow columns
             auto staged = [&](auto general) {
                 constexpr bool kGen = decltype(general)::value;
                 if (own || r.klo > r.khi) return;
@@ -852,23 +863,29 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
                 const int kka = kSplit ? wave * kLines : 0, kkb = kSplit ? min(kka + kLines, nl) : nl;
                 for (int kk = kka; kk < kkb; ++kk, row += A.win) {
                     const int k = k0 + kk;
-                    // m* = mi0 + mint + mf: the fraction from exact products, so that it is
-                    // accurate to an ulp of 1 although kk a32 is not a fraction
+                    // m* = mi0 + mint + mh + ml: mh is exact (kk a32 - mint and fr0 are multiples of
+                    // 2^-23 below 2), and so are a candidate's dl = j0 + it - mh; ml, below 2^-22,
+                    // enters d alone, which is rounded once, at its own size
                     const float kf = (float)kk;
                     const float mint = floorf(fmaf(kf, st.a32, fr0));
-                    const float mf = fmaf(kf, st.da, fmaf(kf, st.a32, -mint) + fr0);
+                    const float mh = fmaf(kf, st.a32, -mint) + fr0, mld = fmaf(kf, st.da, fr1) * st.hpd;
                     const float Lk = fmaf((float)k, r.Ls, r.L0);
                     const float hw = fmaf(Lk, r.hwc, 1.0e-3f);
-                    const float j0 = ceilf(mf - hw);
+                    const float j0 = ceilf(mh - hw);
                     const int at0 = row + (int)(mint + j0);
                     // candidates beyond hw, and all of a line outside the ray's range, read zeros
                     const float last_dl = (unsigned)(k - r.klo) <= span ? hw : -3.0e38f;
                     // (a candidate that reads zeros may lie at the source: its weight stays finite)
                     auto weight = [&](float dl, bool own_cand) {
-                        const float L = fmaf(dl, st.hpl, Lk), d = dl * st.hpd;
-                        const float iL = own_cand ? __builtin_amdgcn_rcpf(L) : 0.0f;
-                        const float z = d * iL, z2 = z * z;
-                        const float rel = z * fmaf(z2, hh.c3, hh.icol);
+                        const float L = fmaf(dl, st.hpl, Lk), d = fmaf(dl, st.hpd, -mld);
+                        // z = d / L is the tangent of the angle off the column's ray, and rel =
+                        // icol (z - z^3 / 3).  With the distance weight iq = 1 / (L^2 + d^2) the one
+                        // reciprocal serves both: s = d L iq = z / (1 + z^2), rel = icol (s + 2/3 s^3)
+                        // up to 1.2 s^4 of itself, |z| <= tan|dCol| < kBpaTan
+                        constexpr bool kOne = kWeighted && !kGen;
+                        const float iq = own_cand ? __builtin_amdgcn_rcpf(kOne ? fmaf(L, L, d * d) : L) : 0.0f;
+                        const float z = kOne ? d * (L * iq) : d * iq;
+                        const float rel = z * fmaf(z * z, kOne ? -2.0f * hh.c3 : hh.c3, st.icol);
                         float w;
                         if constexpr (kGen) {
                             w = 1.0f - fabsf(fminf(fmaxf(rel, hh.clo), hh.chi));
@@ -876,12 +893,11 @@ __global__ __launch_bounds__(256) void bp_adjoint_staged_kernel(BpaArgs A, int s
                         } else {
                             w = fmaxf(1.0f - fabsf(rel), 0.0f);
                         }
-                        // 1 / (L^2 + d^2) = (1 - z^2) / L^2 up to z^4, |z| <= tan|dCol| < kBpaTan
                         if constexpr (kWeighted && kGen) w = own_cand ? w * __builtin_amdgcn_rcpf(fmaf(L, L, d * d)) : 0.0f;
-                        if constexpr (kWeighted && !kGen) w *= fmaf(-z2, iL * iL, iL * iL);
+                        if constexpr (kOne) w *= iq;
                         return w;
                     };
-                    const float dl0 = j0 - mf;
+                    const float dl0 = j0 - mh;
                     int it = 0;
                     for (; it + 2 <= nit; it += 2) {  // two independent chains
                         const float da = dl0 + (float)it, db = da + 1.0f;
@@ -1108,7 +1124,7 @@ fbct_status launch_bp_adjoint(const fbct_plan &p, const DeviceTables &t, const f
     A.dy = p.g.dy;
     A.rFOV = p.g.rFOV;
     A.tanc = p.d.bpa_tan;
-    A.icol = p.d.bp_xi_scale;
+    A.icol = 1.0 / (double)p.g.dCol;
     A.nSlices = n;
     // a group's images are addressed by 32-bit byte offsets: its S images stay below 4 GiB
     const unsigned long long img_bytes = (unsigned long long)p.g.nX * p.g.nY * sizeof(float);
