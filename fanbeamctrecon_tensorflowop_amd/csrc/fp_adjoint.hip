@@ -714,9 +714,26 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
     };
-    auto store_ray = [&]() {
+    // Cells read rays that have no samples in them, with weights 0, which would spread an infinity or
+    // NaN: such values are staged as zeros and added in a pass of their own (rest: what that pass
+    // stages; returns whether there is any).
+    bool nonfinite = false;
+    auto store_ray = [&](auto rest) {
+        constexpr bool kRest = decltype(rest)::value;
         float *d = slots + lane * kDw;
         const float n = (float)pn, dd = pg.z * pg.w * (1.0f / 12.0f);
+        float val[S], t = 0.0f;
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            val[s] = widen(pv[s]);
+            t = fmaf(val[s], 0.0f, t);
+        }
+        const bool any = __any(t != 0.0f);
+        if (kRest || any) {
+            nonfinite = true;
+#pragma unroll
+            for (int s = 0; s < S; ++s) val[s] = (fabsf(val[s]) <= 3.402823466e38f) != kRest ? val[s] : 0.0f;
+        }
         slots_order();  // the previous rays' reads
         *reinterpret_cast<float4 *>(d) = pg;
         *reinterpret_cast<float4 *>(d + 4) = make_float4(pi.x, pi.y, -pg.x * pi.x, -pg.y * pi.y);
@@ -724,12 +741,12 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
             *reinterpret_cast<float2 *>(d + 8) = make_float2(n, dd);
 #pragma unroll
             for (int s = 0; s < S; s += 4)
-                *reinterpret_cast<float4 *>(d + 12 + s) =
-                    make_float4(widen(pv[s]), widen(pv[s + 1]), widen(pv[s + 2]), widen(pv[s + 3]));
+                *reinterpret_cast<float4 *>(d + 12 + s) = make_float4(val[s], val[s + 1], val[s + 2], val[s + 3]);
         } else {
-            *reinterpret_cast<float4 *>(d + 8) = make_float4(n, dd, widen(pv[0]), widen(pv[S - 1]));
+            *reinterpret_cast<float4 *>(d + 8) = make_float4(n, dd, val[0], val[S - 1]);
         }
         slots_order();
+        return any;
     };
     struct Ray {
         RayRec rec;
@@ -753,10 +770,11 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         }
     };
     float ulo = fci, uhi = fci + 1.0f, wlo = fcj, whi = fcj + 1.0f;  // boundaries in the order of the group's rays
-    auto add_ray = [&](auto mixed, const Ray &ray) {
+    auto add_ray = [&](auto mixed, const Ray &ray, auto rest) {
         constexpr bool kMixed = decltype(mixed)::value;
         const CellSums c = cell_sums<kMixed>(ray.rec, fci, fcj, kMixed ? fci : ulo, kMixed ? fci + 1.0f : uhi,
                                              kMixed ? fcj : wlo, kMixed ? fcj + 1.0f : whi);
+        if (decltype(rest)::value && c.n == 0.0f) return;
         const float r[4] = {c.n, c.n * c.ta, c.n * c.tm, c.n * c.g};
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -770,21 +788,41 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 Ray r0, r1;
                 read_ray(d, r0);
                 read_ray(d + kDw, r1);
-                add_ray(mixed, r0);
-                add_ray(mixed, r1);
+                add_ray(mixed, r0, std::false_type{});
+                add_ray(mixed, r1, std::false_type{});
             }
             if (nit > 0) {
                 Ray r;
                 read_ray(d, r);
-                add_ray(mixed, r);
+                add_ray(mixed, r, std::false_type{});
             }
         } else {
             do {
                 Ray r;
                 read_ray(d, r);
-                add_ray(mixed, r);
+                add_ray(mixed, r, std::false_type{});
                 d += kDw;
             } while (--nit > 0);
+        }
+    };
+
+    // A view whose window is wider than the slots: 64 columns at a time, each cell's range per lane.
+    auto wide_view = [&](int v, auto rest) {
+        const BlockCand b = block_candidates(A, A.cs[v], bx, by, kCellRho, kWvHalf * A.dx);
+        const float cf = fmaf(b.gx, dxl, fmaf(b.gy, dyl, b.cf));
+        const int clo = (int)fmaxf(ceilf(cf - b.hw), 0.0f);
+        const int chi = (int)fminf(floorf(cf + b.hw), (float)(A.nCols - 1));
+        const float ext = kWvHalf * A.dx * (fabsf(b.gx) + fabsf(b.gy)) + b.hw + 0.01f;
+        const int first = __builtin_amdgcn_readfirstlane((int)fmaxf(ceilf(b.cf - ext), 0.0f));
+        const int last = __builtin_amdgcn_readfirstlane((int)fminf(floorf(b.cf + ext), (float)(A.nCols - 1)));
+        for (int w = first; w <= last; w += kWvSlots) {
+            load_ray(w + lane < A.nCols, v, w + lane);
+            if (!store_ray(rest) && decltype(rest)::value) continue;
+            for (int c = max(clo, w); c <= min(chi, w + kWvSlots - 1); ++c) {
+                Ray r;
+                read_ray(slots + (c - w) * kDw, r);
+                add_ray(std::true_type{}, r, rest);
+            }
         }
     };
 
@@ -817,7 +855,7 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 auto group = [&](auto mixed) {
                     for (int v0 = vb; v0 < gend; v0 += cnv) {
                         if (!kAhead) load_batch(vb, v0, gend);
-                        store_ray();
+                        store_ray(std::false_type{});
                         if constexpr (kAhead) {
                             if (v0 + cnv < gend) {
                                 load_batch(vb, v0 + cnv, gend);
@@ -839,25 +877,7 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 if (S < 16 && (cdirs & 3) && (cdirs & 12)) group(std::false_type{});
                 else group(std::true_type{});
             } else {
-                // windows wider than the slots: 64 columns at a time, each cell's range per lane
-                for (int v = vb; v < gend; ++v) {
-                    const BlockCand b = block_candidates(A, A.cs[v], bx, by, kCellRho, kWvHalf * A.dx);
-                    const float cf = fmaf(b.gx, dxl, fmaf(b.gy, dyl, b.cf));
-                    const int clo = (int)fmaxf(ceilf(cf - b.hw), 0.0f);
-                    const int chi = (int)fminf(floorf(cf + b.hw), (float)(A.nCols - 1));
-                    const float ext = kWvHalf * A.dx * (fabsf(b.gx) + fabsf(b.gy)) + b.hw + 0.01f;
-                    const int wlo = __builtin_amdgcn_readfirstlane((int)fmaxf(ceilf(b.cf - ext), 0.0f));
-                    const int whi = __builtin_amdgcn_readfirstlane((int)fminf(floorf(b.cf + ext), (float)(A.nCols - 1)));
-                    for (int w = wlo; w <= whi; w += kWvSlots) {
-                        load_ray(w + lane < A.nCols, v, w + lane);
-                        store_ray();
-                        for (int c = max(clo, w); c <= min(chi, w + kWvSlots - 1); ++c) {
-                            Ray r;
-                            read_ray(slots + (c - w) * kDw, r);
-                            add_ray(std::true_type{}, r);
-                        }
-                    }
-                }
+                for (int v = vb; v < gend; ++v) wide_view(v, std::false_type{});
                 if (kAhead && vn < v_end) {
                     need = models(vn, v_end, M, dirs);
                     set_window();
@@ -869,6 +889,8 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 set_window();
             }
         }
+        if (nonfinite)
+            for (int v = v_begin; v < v_end; ++v) wide_view(v, std::true_type{});
     };
 
 #pragma unroll
