@@ -238,6 +238,13 @@ def _time(fn, reps: int) -> float:
     return e0.elapsed_time(e1) / reps
 
 
+def _tune_key(batch: UnevenBatch, images: torch.Tensor, sinos: torch.Tensor) -> str:
+    # the library's digest: a shape is the best one for the kernels that were timed
+    with open(_lib.LIB_PATH, "rb") as f:
+        lib = hashlib.sha1(f.read()).hexdigest()[:16]
+    return "%s|%s|%s|%s|%s" % (torch.cuda.get_device_name(images.device), lib, batch.signature(), images.dtype, sinos.dtype)
+
+
 def autotune(batch: UnevenBatch, images: torch.Tensor, sinos: torch.Tensor, reps: int = 2,
              use_cache: bool = True, verbose: bool = False) -> dict:
     """Pick the batch's launch shape by timing every candidate, then set it.
@@ -246,10 +253,10 @@ def autotune(batch: UnevenBatch, images: torch.Tensor, sinos: torch.Tensor, reps
     FP^T: pixel tile width in ``ADJ_TILE_X`` x workgroups per CU (the tile width shapes the
     gather tiles only).  The two operators are tuned independently on the given
     packed buffers (their storage types are part of the key).  Results are cached in ``$FBCT_TUNE_CACHE`` (default
-    ``~/.cache/fbct_amd/batch_shapes.json``) by device name and geometry signature.
+    ``~/.cache/fbct_amd/batch_shapes.json``) by device name, library build and geometry signature.
     Returns ``{"shape": ..., "fp_ms": ..., "adj_ms": ..., "cached": bool}``."""
     dev = images.device
-    key = "%s|%s|%s|%s" % (torch.cuda.get_device_name(dev), batch.signature(), images.dtype, sinos.dtype)
+    key = _tune_key(batch, images, sinos)
     path = _cache_path()
     if use_cache:
         hit = _load_cache(path).get(key)
@@ -276,9 +283,9 @@ def autotune(batch: UnevenBatch, images: torch.Tensor, sinos: torch.Tensor, reps
             if verbose:
                 print("autotune adj tile=%dx%d wgs/cu=%d: %.3f ms" % (tx, 256 // tx, w, t), flush=True)
             if best_adj is None or t < best_adj[0]:
-                best_adj = (t, tx, w, 0)
+                best_adj = (t, tx, w)
     shape = dict(fp_rays=best_fp[1], fp_wgs_per_cu=best_fp[2], adj_tile_x=best_adj[1], adj_wgs_per_cu=best_adj[2],
-                 adj_stage_views=best_adj[3])
+                 adj_stage_views=0)
     batch.set_shape(**shape)
     result = {"shape": shape, "fp_ms": best_fp[0], "adj_ms": best_adj[0]}
     if use_cache:
