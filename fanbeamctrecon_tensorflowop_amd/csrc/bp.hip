@@ -238,23 +238,16 @@ __global__ __launch_bounds__(64 * W) void bp_direct_kernel(BpArgs A, int slice0)
         for (int v = v0; v < min(v0 + kBpChunk, A.nViews); ++v) update(v);
     }
 
-    if constexpr (W == 1) {
-        if (valid) {
+    __shared__ float part[W][S][64];
 #pragma unroll
-            for (int s = 0; s < S; ++s) A.img[(sl + s) * A.img_stride + (size_t)j * A.nX + i] = acc[s];
-        }
-    } else {
-        __shared__ float part[W][S][64];
+    for (int s = 0; s < S; ++s) part[wave][s][lane] = acc[s];
+    __syncthreads();
+    // slice s of the block is summed by wave s mod W
+    for (int s = wave; s < S; s += W) {
+        double sum = 0.0;
 #pragma unroll
-        for (int s = 0; s < S; ++s) part[wave][s][lane] = acc[s];
-        __syncthreads();
-        // slice s of the block is summed by wave s mod W
-        for (int s = wave; s < S; s += W) {
-            double sum = 0.0;
-#pragma unroll
-            for (int w = 0; w < W; ++w) sum += (double)part[w][s][lane];
-            if (valid) A.img[(sl + s) * A.img_stride + (size_t)j * A.nX + i] = (float)sum;
-        }
+        for (int w = 0; w < W; ++w) sum += (double)part[w][s][lane];
+        if (valid) A.img[(sl + s) * A.img_stride + (size_t)j * A.nX + i] = (float)sum;
     }
 }
 
@@ -608,10 +601,8 @@ struct BpaHat {
 };
 
 // Calls fn(m, w) for the candidates m of line k (FOV range fr) of ray r, w the hat weight
-// (times 1/L^2 for the weighted form); n_minor bounds the candidate range.  kEdge: the
-// column may be the first or the last (clamped taps, cut at half a column); for every
-// other column the hat with its cut at |rel| = 1 is max(1 - |rel|, 0), the same value.
-template <bool kWeighted, bool kEdge = true, typename Fn>
+// (times 1/L^2 for the weighted form); n_minor bounds the candidate range.
+template <bool kWeighted, typename Fn>
 __device__ __forceinline__ void bpa_line(const BpaRay &r, const BpaHat &hh, float h, int k, int2 fr, int n_minor, Fn &&fn)
 {
     const double ms = fma(r.a, (double)k, r.b);
@@ -628,13 +619,8 @@ __device__ __forceinline__ void bpa_line(const BpaRay &r, const BpaHat &hh, floa
         const float L = fmaf(dl, r.pl, Lk);
         const float z = d * __builtin_amdgcn_rcpf(L);
         const float rel = z * fmaf(z * z, hh.c3, hh.icol);
-        float w;
-        if constexpr (kEdge) {
-            w = 1.0f - fabsf(fminf(fmaxf(rel, hh.clo), hh.chi));
-            w = (rel > hh.cut_lo && rel < hh.cut_hi) ? w : 0.0f;
-        } else {
-            w = fmaxf(1.0f - fabsf(rel), 0.0f);
-        }
+        float w = 1.0f - fabsf(fminf(fmaxf(rel, hh.clo), hh.chi));
+        w = (rel > hh.cut_lo && rel < hh.cut_hi) ? w : 0.0f;
         if constexpr (kWeighted) w *= __builtin_amdgcn_rcpf(fmaf(L, L, d * d));
         fn(m, w);
     }

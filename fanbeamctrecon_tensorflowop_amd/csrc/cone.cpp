@@ -136,7 +136,6 @@ void build(fbct_cone_plan &p)
     const double e0 = (double)g.colLeft - (double)g.dShift * dc;
     const double e1 = (double)g.colLeft + ((double)nC - g.dShift) * dc;
     double t0 = flat ? e0 / D : std::tan(e0), t1 = flat ? e1 / D : std::tan(e1);
-    d.edge_exact = 1;
     d.tan_min = std::min(t0, t1);
     d.tan_max = std::max(t0, t1);
     d.atan_nc = 0;

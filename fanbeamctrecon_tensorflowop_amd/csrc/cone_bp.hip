@@ -316,11 +316,6 @@ __device__ __forceinline__ void store_columns(const ConeArgs &A, const float (&a
         const int i = i0 + (lane & 7), j = j0 + (lane >> 3);
         if (i < A.nX && j < A.nY && k0 + k < A.nZ) store_f(out, ((size_t)(k0 + k) * A.nY + j) * A.nX + i, v);
     };
-    if (waves == 1) {
-#pragma unroll
-        for (int k = 0; k < KZ; ++k) put(k, acc[k]);
-        return;
-    }
     float *mine = cone_lds + wave * wave_floats + lane;
     wave_lds_order();  // the last window's reads
 #pragma unroll
@@ -591,7 +586,7 @@ void launch_tile(dim3 grid, hipStream_t st, const ConeArgs &A, fbct_dtype to)
 template <bool kFlat, int kNc, int KZ, bool kPair = true>
 void launch_direct(dim3 grid, int waves, hipStream_t st, const ConeArgs &A, fbct_dtype to)
 {
-    const size_t lds = waves > 1 ? (size_t)waves * KZ * 64 * sizeof(float) : 0;
+    const size_t lds = (size_t)waves * KZ * 64 * sizeof(float);
     if (to == FBCT_BF16)
         hipLaunchKernelGGL((cone_bp_direct_kernel<kFlat, kNc, KZ, kPair, bf16_t>), grid, dim3(64 * waves), lds, st, A);
     else
@@ -709,9 +704,10 @@ fbct_status launch_cone_bp(const fbct_cone_plan &p, const ConeDeviceTables &t, c
     A.q = q;
     A.vol = vol;
     const ConeLaunch L = choose(g, p.d.zr_scale);
+    // the most z-chunks (of 32, 16, 4 or one slice) that a call may hold, whatever chunks its kernel takes
     const int kz_most = g.nZ >= 32 ? 32 : (g.nZ >= 16 ? 16 : (g.nZ >= 4 ? 4 : 1));
     const long long most = (long long)((g.nZ + kz_most - 1) / kz_most) * n;
-    if (most > 65535) return fail(FBCT_ERR_UNSUPPORTED, "cone backprojection: %lld z-groups exceed the grid", most);
+    if (most > 65535) return fail(FBCT_ERR_UNSUPPORTED, "cone backprojection: %lld z-chunks, at most 65535 a call", most);
     A.nzc = (g.nZ + L.kz - 1) / L.kz;
     const long long gz = (long long)A.nzc * n;
     if ((unsigned long long)g.nRows * (unsigned long long)g.nCols * 4ull >= (1ull << 32))

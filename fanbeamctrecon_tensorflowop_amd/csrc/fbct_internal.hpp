@@ -246,8 +246,7 @@ struct ConeDerived {
     float zr_scale, rt_offset;
     int ct_col, rt_row;
     float r2;                   // rFOV^2 (float)
-    int edge_exact;             // 1: the in-range decision near the edges is retaken in FP64 on t/U
-    double tan_min, tan_max;    //    0 < xi < nCols  <=>  tan_min < t/U < tan_max
+    double tan_min, tan_max;    // 0 < xi < nCols  <=>  tan_min < t/U < tan_max (decided so near the edges, in FP64)
     int atan_nc;                // curved: coefficients of the atan correction polynomial (0 = atanf)
     float atan_zmax;            // it is fitted on |t/U| <= atan_zmax, which the FOV disk's columns keep to
     float atan_c[kBpAtanMax];
