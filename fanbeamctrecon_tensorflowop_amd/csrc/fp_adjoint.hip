@@ -714,26 +714,9 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
     };
-    // Cells read rays that have no samples in them, with weights 0, which would spread an infinity or
-    // NaN: such values are staged as zeros and added in a pass of their own (rest: what that pass
-    // stages; returns whether there is any).
-    bool nonfinite = false;
-    auto store_ray = [&](auto rest) {
-        constexpr bool kRest = decltype(rest)::value;
+    auto store_ray = [&]() {
         float *d = slots + lane * kDw;
         const float n = (float)pn, dd = pg.z * pg.w * (1.0f / 12.0f);
-        float val[S], t = 0.0f;
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            val[s] = widen(pv[s]);
-            t = fmaf(val[s], 0.0f, t);
-        }
-        const bool any = __any(t != 0.0f);
-        if (kRest || any) {
-            nonfinite = true;
-#pragma unroll
-            for (int s = 0; s < S; ++s) val[s] = (fabsf(val[s]) <= 3.402823466e38f) != kRest ? val[s] : 0.0f;
-        }
         slots_order();  // the previous rays' reads
         *reinterpret_cast<float4 *>(d) = pg;
         *reinterpret_cast<float4 *>(d + 4) = make_float4(pi.x, pi.y, -pg.x * pi.x, -pg.y * pi.y);
@@ -741,12 +724,12 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
             *reinterpret_cast<float2 *>(d + 8) = make_float2(n, dd);
 #pragma unroll
             for (int s = 0; s < S; s += 4)
-                *reinterpret_cast<float4 *>(d + 12 + s) = make_float4(val[s], val[s + 1], val[s + 2], val[s + 3]);
+                *reinterpret_cast<float4 *>(d + 12 + s) =
+                    make_float4(widen(pv[s]), widen(pv[s + 1]), widen(pv[s + 2]), widen(pv[s + 3]));
         } else {
-            *reinterpret_cast<float4 *>(d + 8) = make_float4(n, dd, val[0], val[S - 1]);
+            *reinterpret_cast<float4 *>(d + 8) = make_float4(n, dd, widen(pv[0]), widen(pv[S - 1]));
         }
         slots_order();
-        return any;
     };
     struct Ray {
         RayRec rec;
@@ -770,11 +753,11 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         }
     };
     float ulo = fci, uhi = fci + 1.0f, wlo = fcj, whi = fcj + 1.0f;  // boundaries in the order of the group's rays
-    auto add_ray = [&](auto mixed, const Ray &ray, auto rest) {
+    auto add_ray = [&](auto mixed, const Ray &ray, auto skip_empty) {
         constexpr bool kMixed = decltype(mixed)::value;
         const CellSums c = cell_sums<kMixed>(ray.rec, fci, fcj, kMixed ? fci : ulo, kMixed ? fci + 1.0f : uhi,
                                              kMixed ? fcj : wlo, kMixed ? fcj + 1.0f : whi);
-        if (decltype(rest)::value && c.n == 0.0f) return;
+        if (decltype(skip_empty)::value && c.n == 0.0f) return;
         const float r[4] = {c.n, c.n * c.ta, c.n * c.tm, c.n * c.g};
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -807,7 +790,8 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
     };
 
     // A view whose window is wider than the slots: 64 columns at a time, each cell's range per lane.
-    auto wide_view = [&](int v, auto rest) {
+    // Rays without samples in the cell add nothing, whatever their value.
+    auto wide_view = [&](int v) {
         const BlockCand b = block_candidates(A, A.cs[v], bx, by, kCellRho, kWvHalf * A.dx);
         const float cf = fmaf(b.gx, dxl, fmaf(b.gy, dyl, b.cf));
         const int clo = (int)fmaxf(ceilf(cf - b.hw), 0.0f);
@@ -817,11 +801,11 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         const int last = __builtin_amdgcn_readfirstlane((int)fminf(floorf(b.cf + ext), (float)(A.nCols - 1)));
         for (int w = first; w <= last; w += kWvSlots) {
             load_ray(w + lane < A.nCols, v, w + lane);
-            if (!store_ray(rest) && decltype(rest)::value) continue;
+            store_ray();
             for (int c = max(clo, w); c <= min(chi, w + kWvSlots - 1); ++c) {
                 Ray r;
                 read_ray(slots + (c - w) * kDw, r);
-                add_ray(std::true_type{}, r, rest);
+                add_ray(std::true_type{}, r, std::true_type{});
             }
         }
     };
@@ -855,7 +839,7 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 auto group = [&](auto mixed) {
                     for (int v0 = vb; v0 < gend; v0 += cnv) {
                         if (!kAhead) load_batch(vb, v0, gend);
-                        store_ray(std::false_type{});
+                        store_ray();
                         if constexpr (kAhead) {
                             if (v0 + cnv < gend) {
                                 load_batch(vb, v0 + cnv, gend);
@@ -877,7 +861,7 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 if (S < 16 && (cdirs & 3) && (cdirs & 12)) group(std::false_type{});
                 else group(std::true_type{});
             } else {
-                for (int v = vb; v < gend; ++v) wide_view(v, std::false_type{});
+                for (int v = vb; v < gend; ++v) wide_view(v);
                 if (kAhead && vn < v_end) {
                     need = models(vn, v_end, M, dirs);
                     set_window();
@@ -889,18 +873,30 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 set_window();
             }
         }
-        if (nonfinite)
-            for (int v = v_begin; v < v_end; ++v) wide_view(v, std::true_type{});
     };
 
+    auto clear = [&]() {
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int s = 0; s < S; ++s) acc[q][s] = 0.0f;
+            for (int s = 0; s < S; ++s) acc[q][s] = 0.0f;
+    };
+    clear();
     // cells outside the FOV disk hold no samples; a tile without any other cell skips the views
     if (__any(ci <= A.nX - 1 && cj <= A.nY - 1 && cell_in_fov(A, fci, fcj))) {
         const int v0 = view_quarter(A.nViews, wave), v1 = view_quarter(A.nViews, wave + 1);
-        if (v0 < v1) run(v0, v1);
+        if (v0 < v1) {
+            run(v0, v1);
+            // Cells add the rays that have no samples in them with weights 0, which spreads an infinity
+            // or NaN: where there is one, the sums are formed again without them (the same sums otherwise)
+            float t = 0.0f;
+#pragma unroll
+            for (int s = 0; s < S; ++s) t = fmaf(acc[0][s], 0.0f, t);
+            if (__any(t != 0.0f)) {
+                clear();
+                for (int v = v0; v < v1; ++v) wide_view(v);
+            }
+        }
     }
     __syncthreads();  // the staging space turns into partial sums
     constexpr int kC = CellShared<S>::kC;

@@ -166,9 +166,10 @@ fbct_status fbct_fp_residual(fbct_plan *plan, const void *image, int image_dtype
                              void *residual, int residual_dtype, int n_slices, void *stream);
 
 /* Exact matched adjoint of fbct_fp (transpose of the same interpolation weights).
- * sino -> image.  No reference counterpart (the reference has no gradient).  The
- * sinogram must be finite: a NaN or infinity spreads to every pixel whose candidate
- * rays include it, not only to the pixels the ray touches. */
+ * sino -> image.  No reference counterpart (the reference has no gradient).  A NaN or
+ * infinity reaches the pixels that its ray's samples touch; where samples lie outside
+ * the cells between pixel centres -1 and n (2 rFOV/dx - n + 1/2 >= 1) or nX != nY it
+ * may reach pixels beside the ray too. */
 fbct_status fbct_fp_adjoint(fbct_plan *plan, const float *sino, float *image, int n_slices,
                             void *stream);
 
