@@ -557,7 +557,10 @@ template <int S>
 union CellShared {
     static constexpr int kC = S < kCombineS ? S : kCombineS;
     WvStage<S> stage[kWvSplit];
-    float part[(kWvSplit - 1) * 4 * kC * kCells];
+    struct {
+        float part[kWvSplit][4][kC][kCells];  // the waves' sums
+        float corner[kC][4][kCells];
+    } sum;
 };
 
 // Cell (lx, ly) of this lane in the tile: each 16 lanes a 4 x 4 block, whose candidate columns
@@ -569,59 +572,71 @@ __device__ __forceinline__ void tile_cell(int &lx, int &ly)
     ly = 4 * (lane >> 5) + ((lane >> 2) & 3);
 }
 
-// Combines the cell sums acc[4][S] (n, Su, Sw, Suw, each times the ray values) of the
-// tile's cells, as corner partials, into its 7 x 7 pixels of slices [s0, s0 + S),
-// kCombineS slices per pass through part (4 x kCombineS x kCells floats of LDS, free when
-// called).  Pixel (px, py) collects corner dx of cell px - dx (dx = 0, 1), and, on the borders,
-// the clamped outer corner of cell -1 (pixel 0) or of cell n-1 (pixel n-1).  Every thread of
-// the workgroup calls it; those with own = false only keep the barriers.
-template <int S, typename TO>
-__device__ __forceinline__ void cell_combine(const FpaArgs &A, float *part, const float (&acc)[4][S], int tx, int ty,
-                                             int s0, bool own)
+// LDS accesses of a wave complete in order; this keeps the compiler from moving them across each
+// other where lanes read what other lanes of their wave wrote.
+__device__ __forceinline__ void wave_lds_order()
 {
-    int lx, ly;
-    tile_cell(lx, ly);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Adds the waves' cell sums acc[4][S] (n, Su, Sw, Suw, each times the ray values; FP32, in pairs) and
+// combines them, as corner partials, into the tile's 7 x 7 pixels of slices [s0, s0 + S), kCombineS
+// slices per pass, a wave each (one wave for all of them took 340 of the 890 us of 64 slices of 512 x
+// 512 over 90 views).  Pixel (px, py) collects corner dx of cell px - dx (dx = 0, 1), and, on the
+// borders, the clamped outer corner of cell -1 (pixel 0) or of cell n-1 (pixel n-1).  sh is free when
+// called; every thread of the workgroup calls it.
+template <int S, typename TO>
+__device__ __forceinline__ void cell_combine(const FpaArgs &A, CellShared<S> &sh, const float (&acc)[4][S], int tx,
+                                             int ty, int s0)
+{
+    constexpr int kC = CellShared<S>::kC;
+    int lane = (int)threadIdx.x;
+    asm volatile("" : "+v"(lane));  // nothing of this is kept in registers while the views are summed
+    const int wave = __builtin_amdgcn_readfirstlane(lane >> 6);
+    lane &= 63;
+    const int lx = 4 * ((lane >> 4) & 1) + (lane & 3), ly = 4 * (lane >> 5) + ((lane >> 2) & 3);
     const int cid = ly * kCellTile + lx;
     const int px = tx * kCellOut + lx, py = ty * kCellOut + ly;
-    const bool out = own && lx < kCellOut && ly < kCellOut && px < A.nX && py < A.nY;
-    int xc[4], xd[4], yc[4], yd[4];  // local cell column and corner of each x (y) term (4: a side of one pixel)
-    int nxt = 0, nyt = 0;
-    xc[nxt] = lx + 1, xd[nxt++] = 0;
-    xc[nxt] = lx, xd[nxt++] = 1;
-    if (px == 0) xc[nxt] = lx, xd[nxt++] = 0;
-    if (px == A.nX - 1) xc[nxt] = lx + 1, xd[nxt++] = 1;
-    yc[nyt] = ly + 1, yd[nyt++] = 0;
-    yc[nyt] = ly, yd[nyt++] = 1;
-    if (py == 0) yc[nyt] = ly, yd[nyt++] = 0;
-    if (py == A.nY - 1) yc[nyt] = ly + 1, yd[nyt++] = 1;
+    const bool out = lx < kCellOut && ly < kCellOut && px < A.nX && py < A.nY;
 #pragma unroll
     for (int sb = 0; sb < S; sb += kCombineS) {
-        constexpr int kC = S < kCombineS ? S : kCombineS;
-        if (own) {
+        if (sb > 0) __syncthreads();  // the previous pass's reads
 #pragma unroll
-            for (int k = 0; k < kC; ++k) {  // corner weights from the sums (n, Su, Sw, Suw)
-                const float sn = acc[0][sb + k], su = acc[1][sb + k], sw = acc[2][sb + k], suw = acc[3][sb + k];
-                const float c01 = sw - suw;
-                part[(0 * kC + k) * kCells + cid] = (sn - su) - c01;
-                part[(1 * kC + k) * kCells + cid] = su - suw;
-                part[(2 * kC + k) * kCells + cid] = c01;
-                part[(3 * kC + k) * kCells + cid] = suw;
-            }
-        }
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int k = 0; k < kC; ++k) sh.sum.part[wave][q][k][lane] = acc[q][sb + k];
         __syncthreads();
-        if (out) {
+        if (wave >= kC || s0 + sb + wave >= A.nSlices) continue;
+        float r[4];  // corner weights from the sums (n, Su, Sw, Suw)
 #pragma unroll
-            for (int k = 0; k < kC; ++k) {
-                double sum = 0.0;
-                for (int a = 0; a < nyt; ++a)
-                    for (int b = 0; b < nxt; ++b)
-                        sum += (double)part[((yd[a] * 2 + xd[b]) * kC + k) * kCells + yc[a] * kCellTile + xc[b]];
-                if (s0 + sb + k < A.nSlices)
-                    store_f(static_cast<TO *>(A.img), (size_t)(s0 + sb + k) * A.img_stride + (size_t)py * A.nX + px,
-                            (float)(sum * (double)A.scale));
-            }
+        for (int q = 0; q < 4; ++q)
+            r[q] = (sh.sum.part[0][q][wave][lane] + sh.sum.part[1][q][wave][lane]) +
+                   (sh.sum.part[2][q][wave][lane] + sh.sum.part[3][q][wave][lane]);
+        float(&corner)[4][kCells] = sh.sum.corner[wave];
+        const float c01 = r[2] - r[3];
+        wave_lds_order();  // the previous pass's corners are read
+        corner[0][cid] = (r[0] - r[1]) - c01;
+        corner[1][cid] = r[1] - r[3];
+        corner[2][cid] = c01;
+        corner[3][cid] = r[3];
+        wave_lds_order();
+        if (out) {
+            double sum = 0.0;
+            auto row = [&](int cy, int dy) {
+                const float *c0 = &corner[2 * dy][cy * kCellTile + lx], *c1 = c0 + kCells;
+                sum += (double)c0[1];
+                sum += (double)c1[0];
+                if (px == 0) sum += (double)c0[0];
+                if (px == A.nX - 1) sum += (double)c1[1];
+            };
+            row(ly + 1, 0);
+            row(ly, 1);
+            if (py == 0) row(ly, 0);
+            if (py == A.nY - 1) row(ly + 1, 1);
+            store_f(static_cast<TO *>(A.img), (size_t)(s0 + sb + wave) * A.img_stride + (size_t)py * A.nX + px,
+                    (float)(sum * (double)A.scale));
         }
-        __syncthreads();  // part is free again
     }
 }
 
@@ -709,15 +724,10 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
             for (int s = 0; s < S; ++s) pv[s] = sino[s][rb];
         }
     };
-    // the wave's lanes read each other's slots: keep the order, LDS keeps it too
-    auto slots_order = [&]() {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-    };
     auto store_ray = [&]() {
         float *d = slots + lane * kDw;
         const float n = (float)pn, dd = pg.z * pg.w * (1.0f / 12.0f);
-        slots_order();  // the previous rays' reads
+        wave_lds_order();  // the previous rays' reads
         *reinterpret_cast<float4 *>(d) = pg;
         *reinterpret_cast<float4 *>(d + 4) = make_float4(pi.x, pi.y, -pg.x * pi.x, -pg.y * pi.y);
         if constexpr (S >= 4) {
@@ -729,7 +739,7 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         } else {
             *reinterpret_cast<float4 *>(d + 8) = make_float4(n, dd, widen(pv[0]), widen(pv[S - 1]));
         }
-        slots_order();
+        wave_lds_order();
     };
     struct Ray {
         RayRec rec;
@@ -789,8 +799,8 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         }
     };
 
-    // A view whose window is wider than the slots: 64 columns at a time, each cell's range per lane.
-    // Rays without samples in the cell add nothing, whatever their value.
+    // A view by itself: 64 columns at a time, each cell's range per lane, without the rays that have no
+    // samples in the cell.  Where windows are wider than the slots.
     auto wide_view = [&](int v) {
         const BlockCand b = block_candidates(A, A.cs[v], bx, by, kCellRho, kWvHalf * A.dx);
         const float cf = fmaf(b.gx, dxl, fmaf(b.gy, dyl, b.cf));
@@ -808,6 +818,23 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 add_ray(std::true_type{}, r, std::true_type{});
             }
         }
+    };
+
+    // Cells add rays that have no samples in them with weights 0, which would spread an infinity or NaN:
+    // where there is one, the rest of its group of views (16 slices: all of the wave's views, found from
+    // the sums) is taken view by view without such rays; the other sums come out the same.  (Looking at
+    // the staged values costs 16 slices 1.5%, looking at the sums 8 slices 5%, in registers.)
+    auto nonfinite = [&](auto &&value) {
+        float most = fabsf(value(0));
+#pragma unroll
+        for (int s = 1; s < S; ++s) most = __builtin_elementwise_maximum(most, fabsf(value(s)));  // keeps NaN
+        return __any(!(most < __builtin_inff())) != 0;
+    };
+    auto clear = [&]() {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int s = 0; s < S; ++s) acc[q][s] = 0.0f;
     };
 
     // Sums of the views [v_begin, v_end) into acc.
@@ -829,10 +856,13 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
         };
         set_window();
         if (kAhead && need <= kWvSlots) load_batch(v_begin, v_begin, min(v_begin + kWvGroup, v_end));
+        bool one_by_one = false;
         for (int vb = v_begin; vb < v_end; vb += kWvGroup) {
             const int gend = min(vb + kWvGroup, v_end), vn = gend;
             const Model C = M;
-            if (need <= kWvSlots) {
+            int left = vb;  // first view that is taken by itself
+            if (need <= kWvSlots && !one_by_one) {
+                left = gend;
                 const int cwd = wd, cnv = nv, cdirs = dirs;
                 ulo = cdirs & 2 ? fci + 1.0f : fci, uhi = cdirs & 2 ? fci : fci + 1.0f;
                 wlo = cdirs & 8 ? fcj + 1.0f : fcj, whi = cdirs & 8 ? fcj : fcj + 1.0f;
@@ -840,6 +870,10 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                     for (int v0 = vb; v0 < gend; v0 += cnv) {
                         if (!kAhead) load_batch(vb, v0, gend);
                         store_ray();
+                        if (!kAhead && nonfinite([&](int s) { return widen(pv[s]); })) {
+                            left = v0;
+                            break;
+                        }
                         if constexpr (kAhead) {
                             if (v0 + cnv < gend) {
                                 load_batch(vb, v0 + cnv, gend);
@@ -860,8 +894,9 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 // (one copy of the loop for 16 slices: the other costs a wave per SIMD)
                 if (S < 16 && (cdirs & 3) && (cdirs & 12)) group(std::false_type{});
                 else group(std::true_type{});
-            } else {
-                for (int v = vb; v < gend; ++v) wide_view(v);
+            }
+            if (left < gend) {
+                for (int v = left; v < gend; ++v) wide_view(v);
                 if (kAhead && vn < v_end) {
                     need = models(vn, v_end, M, dirs);
                     set_window();
@@ -872,57 +907,22 @@ __device__ __forceinline__ void cell_tile(const FpaArgs &A, CellShared<S> &sh, i
                 need = models(vn, v_end, M, dirs);
                 set_window();
             }
+            if (kAhead && vn == v_end && !one_by_one && nonfinite([&](int s) { return acc[0][s]; })) {
+                one_by_one = true;
+                clear();
+                vb = v_begin - kWvGroup;
+            }
         }
     };
 
-    auto clear = [&]() {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int s = 0; s < S; ++s) acc[q][s] = 0.0f;
-    };
     clear();
     // cells outside the FOV disk hold no samples; a tile without any other cell skips the views
     if (__any(ci <= A.nX - 1 && cj <= A.nY - 1 && cell_in_fov(A, fci, fcj))) {
         const int v0 = view_quarter(A.nViews, wave), v1 = view_quarter(A.nViews, wave + 1);
-        if (v0 < v1) {
-            run(v0, v1);
-            // Cells add the rays that have no samples in them with weights 0, which spreads an infinity
-            // or NaN: where there is one, the sums are formed again without them (the same sums otherwise)
-            float t = 0.0f;
-#pragma unroll
-            for (int s = 0; s < S; ++s) t = fmaf(acc[0][s], 0.0f, t);
-            if (__any(t != 0.0f)) {
-                clear();
-                for (int v = v0; v < v1; ++v) wide_view(v);
-            }
-        }
+        if (v0 < v1) run(v0, v1);
     }
     __syncthreads();  // the staging space turns into partial sums
-    constexpr int kC = CellShared<S>::kC;
-#pragma unroll
-    for (int sb = 0; sb < S; sb += kCombineS) {
-        if (wave > 0) {
-            float *mine = sh.part + (wave - 1) * 4 * kC * kCells + lane;
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int k = 0; k < kC; ++k) mine[(q * kC + k) * kCells] = acc[q][sb + k];
-        }
-        __syncthreads();
-        if (wave == 0) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int k = 0; k < kC; ++k) {
-                    const float *p = sh.part + (q * kC + k) * kCells + lane;
-                    constexpr int kG = 4 * kC * kCells;
-                    acc[q][sb + k] = (acc[q][sb + k] + p[0]) + (p[kG] + p[2 * kG]);
-                }
-        }
-        __syncthreads();
-    }
-    cell_combine<S, TO>(A, sh.part, acc, tx, ty, s0, wave == 0);
+    cell_combine<S, TO>(A, sh, acc, tx, ty, s0);
 }
 
 // Waves per SIMD that the registers are held to: one slice 667, 662, 668 us at 5, 6, 8; four 878,
@@ -989,6 +989,7 @@ __global__ __launch_bounds__(kAdjThreads, 6) void fp_adjoint_batch_kernel(const 
         if (adj_cells_fit(A.far_x, A.far_y)) {  // same test as the single-slice launch
             blocked_tile(local, adj_cell_tiles(A.nX), adj_cell_tiles(A.nY), tx, ty);
             cell_tile<1, TI, TO>(A, sh, (int)tx, (int)ty, 0);
+            __syncthreads();  // sh is free again
         } else {
             blocked_tile(local, (A.nX + TX - 1) / TX, (A.nY + 256 / TX - 1) / (256 / TX), tx, ty);
             adjoint_tile<1, TX, TI, TO>(A, (int)tx, (int)ty, 0);
