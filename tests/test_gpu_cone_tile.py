@@ -39,6 +39,33 @@ CASES = {
 }
 
 
+def _check(plan, g, a, seed, what, oracle_mod):
+    cols, rows, views, nz, dx = (g[k] for k in ("nCols", "nRows", "nViews", "nZ", "dx"))
+    ells = workloads.random_ellipsoids(6, seed=seed, rfov=g["rFOV"], zhalf=0.5 * nz * dx)
+    P = workloads.ellipsoid_projections(ells, g, a).numpy()
+    P = (P + np.random.default_rng(nz).normal(0, 1e-3, size=P.shape)).astype(np.float32)
+    q = plan.filter(torch.from_numpy(P[None]).cuda())
+    got = plan.backproject(q)[0].double().cpu().numpy()
+    q, o = q.double().cpu().numpy(), oracle_mod.ConeOracle(g, a)
+    ref, eps = o.backproject(q)[0], 2.0 ** -24
+
+    def steps(axis):  # the larger of a sample's differences to its neighbours
+        d = np.abs(np.diff(q, axis=axis))
+        pad = [(0, 0)] * q.ndim
+        pad[axis] = (0, 1)
+        low = np.pad(d, pad)
+        pad[axis] = (1, 0)
+        return np.maximum(low, np.pad(d, pad))
+
+    bound = (8.0 * eps * cols * o.backproject(steps(3))[0] + 6.0 * eps * rows * o.backproject(steps(2))[0]
+             + (20 + views) * eps * o.backproject(np.abs(q))[0])
+    err = np.abs(got - ref)
+    worst = float((err / np.maximum(bound, 1e-30)).max())
+    print("%s, rel_l2 %.2e, worst voxel %.2f of its bound" % (what, rel_l2(got, ref), worst), flush=True)
+    assert worst <= 1.0
+    assert np.count_nonzero(bound) > 0.7 * bound.size
+
+
 @pytest.mark.parametrize("detector", ["flat", "curved"])
 @pytest.mark.parametrize("name", sorted(CASES))
 def test_staged_and_not(name, detector, oracle_mod):
@@ -62,27 +89,19 @@ def test_staged_and_not(name, detector, oracle_mod):
               + min(abs(c - 0.5 * nx) for c in (j + 0.5, min(j + side, nx) - 0.5)) ** 2 < (0.5 * nx) ** 2]
     share = float(np.mean(staged))
     assert share > 0.98 if whole else 0.1 < share < 0.95
-    ells = workloads.random_ellipsoids(6, seed=nx + nz, rfov=rfov, zhalf=0.5 * nz * dx)
-    P = workloads.ellipsoid_projections(ells, g, a).numpy()
-    P = (P + np.random.default_rng(nz).normal(0, 1e-3, size=P.shape)).astype(np.float32)
-    q = plan.filter(torch.from_numpy(P[None]).cuda())
-    got = plan.backproject(q)[0].double().cpu().numpy()
-    q, o = q.double().cpu().numpy(), oracle_mod.ConeOracle(g, a)
-    ref, eps = o.backproject(q)[0], 2.0 ** -24
+    _check(plan, g, a, nx + nz, "%s %s: %.2f staged" % (name, detector, share), oracle_mod)
 
-    def steps(axis):  # the larger of a sample's differences to its neighbours
-        d = np.abs(np.diff(q, axis=axis))
-        pad = [(0, 0)] * q.ndim
-        pad[axis] = (0, 1)
-        low = np.pad(d, pad)
-        pad[axis] = (1, 0)
-        return np.maximum(low, np.pad(d, pad))
 
-    bound = (8.0 * eps * cols * o.backproject(steps(3))[0] + 6.0 * eps * rows * o.backproject(steps(2))[0]
-             + (20 + views) * eps * o.backproject(np.abs(q))[0])
-    err = np.abs(got - ref)
-    worst = float((err / np.maximum(bound, 1e-30)).max())
-    print("%s %s: %.2f staged, rel_l2 %.2e, worst voxel %.2f of its bound" % (name, detector, share, rel_l2(got, ref), worst),
-          flush=True)
-    assert worst <= 1.0
-    assert np.count_nonzero(bound) > 0.7 * bound.size
+# few views: 16, 8 and 4 waves a tile (sums over the waves), of 8 slices (8 x 8 pixel tiles times chunks of 8 from
+# 700 and 1500 on) and from global memory
+@pytest.mark.parametrize("nx,nz,d_row,views", [
+    (60, 56, 1.5, 9), (80, 56, 1.5, 9), (80, 56, 1.5, 40), (80, 56, 1.5, 64), (100, 72, 1.5, 1), (100, 72, 1.5, 9),
+    (100, 72, 1.5, 57), (240, 4, 1.5, 3), (240, 4, 1.5, 33), (60, 4, 1.5, 17),
+])
+def test_few_views(nx, nz, d_row, views, oracle_mod):
+    half = 1.1 * math.asin(0.5 * nx / R)
+    cols, rows = int(2.0 * D * math.tan(half) / 1.4), int(1.3 * nz * D / R / d_row)
+    g = cone_geom(R=R, D=D, n_views=views, d_angle=2.0 * math.pi / views, detector="flat", n_cols=cols, n_rows=rows,
+                  d_col=1.4, d_row=d_row, nx=nx, nz=nz, dx=1.0, dz=1.0)
+    a = (np.arange(views) * (2.0 * math.pi / views) + 0.1).astype(np.float32)
+    _check(ConePlan(g, a), g, a, nx + nz, "%d x %d, %d views" % (nx, nz, views), oracle_mod)
