@@ -641,11 +641,11 @@ void launch_nc(const ConeLaunch &L, dim3 grid, hipStream_t st, const ConeArgs &A
 // Waves per tile: sixteen for wave (400 x 400 x 64 over 500: 2.8 ms, eight 3.4, four 3.7) and where
 // there are fewer than 512 tiles (direct, 64 x 64 x 16 over 120 views: 15 us, eight 18), else eight.
 // With few views each wave's share gets short beside its windows' evaluation and the sum over the
-// waves: from 1500 tiles on wave takes eight below 500 views (180 x 180 x 86: 90 views 119 us, sixteen
-// 143; 250: 294, 328; 500: 602, 625; 720: 1037, 952) and four below 56 (24 views: 40 us, eight 46,
-// sixteen 68; 64: 85, 89, 110), from 700 on eight below 64 (128 x 128 x 32, 40 views: 23 us, sixteen 26;
-// 90: 43, 45; 180: 92, 81) and four below 32; direct four below 32 (200 x 200 x 64, 12 views: 30 us,
-// eight 36; 24: 53, 53).
+// waves: from 1500 tiles on wave takes eight below a twelfth of the tiles (180 x 180 x 86, 5819 tiles: 90
+// views 119 us, sixteen 143; 250: 294, 328; 500: 602, 625; 720: 1037, 952; curved 128 x 128 x 64, 2048
+// tiles: 90 views 71, 75; 180: 146, 145) and four below 56 (24 views: 40 us, eight 46, sixteen 68; 64: 85,
+// 89, 110), from 700 on eight below 64 (128 x 128 x 32, 40 views: 23 us, sixteen 26; 90: 43, 45; 180: 92,
+// 81) and four below 32; direct four below 32 (200 x 200 x 64, 12 views: 30 us, eight 36; 24: 53, 53).
 ConeLaunch choose(const fbct_cone_geom &g, double zr_scale)
 {
     auto chunks = [&](int kz) { return (long long)((g.nZ + kz - 1) / kz); };
@@ -663,7 +663,7 @@ ConeLaunch choose(const fbct_cone_geom &g, double zr_scale)
     const int few = g.nViews < 32 ? 4 : 8;
     int waves = 16;
     if (!wave && wgs >= 512) waves = few;
-    else if (wave && wgs >= 1500 && g.nViews < 500) waves = g.nViews < 56 ? 4 : 8;
+    else if (wave && wgs >= 1500 && 12LL * g.nViews < wgs) waves = g.nViews < 56 ? 4 : 8;
     else if (wave && wgs >= 700 && g.nViews < 64) waves = few;
     return {wave ? ConeLaunch::kWave : ConeLaunch::kDirect, kz, waves};
 }
