@@ -8,9 +8,9 @@
 // Here one launch covers every view and a group of slices: a thread owns a pixel of S
 // slices, loops over its views with the per-view (cos, sin) read as uniform scalars, computes the
 // column coordinate, in-range decision, taps and weight once per (pixel, view) and
-// applies them to the S slices, accumulates in registers and stores once.  The detector
-// row is read with two gathers per update; the 1-D texture's clamp-to-edge linear
-// filter is reproduced with exact FP32 weights.
+// applies them to the S slices, accumulates in registers and stores once.  Both taps of an
+// update come in one load from global memory (few slices) or from columns staged in LDS; the
+// 1-D texture's clamp-to-edge linear filter is reproduced with exact FP32 weights.
 //
 // atan(t/U) is evaluated as z + z^3 R(z^2) with a correction polynomial R fitted per
 // plan over the range FOV pixels reach, |t/U| <= rFOV/sqrt(R^2 - rFOV^2) (relative error
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(64 * W) void bp_direct_kernel(BpArgs A, int slice0)
 // fill the chip.
 //
 // Bound: VALU issue and the LDS reads, about even.  64 slices of 512 x 512 pixels, 984 views:
-// 3.29 -> 2.12 ms by giving each wave an 8 x 8 block (its 16-byte reads stop conflicting: a
+// 3.29 -> 2.33 ms by giving each wave an 8 x 8 block (its 16-byte reads stop conflicting: a
 // 16 x 4 strip spans more columns than the 16 that fall in distinct bank groups) and by the
 // batch path (4 independent chains instead of one).
 constexpr int kBpStageCols = 64;

@@ -110,17 +110,17 @@ __device__ __forceinline__ void candidate_rays(const FpaArgs &A, float2 cs, floa
     chi = (int)fminf(floorf(cf + hw), (float)(A.nCols - 1));
 }
 
-// Candidate rays of the cells of one 4 x 4 block in one view, from a linear model of the
+// Candidate rays of the cells of one square block in one view, from a linear model of the
 // column coordinate about the block centre (xc, yc) (mm): cf(p) = c_scale atan(t/U) +
 // c_off is c_scale times the polar angle of p about the source, whose Hessian has norm
-// 1/r^2 (r the distance to the source).  Over the block's cell centres, within h = 1.5 dx
-// of the centre along each axis, the linear model is therefore off by at most
+// 1/r^2 (r the distance to the source).  Over the block's cell centres, within h of the
+// centre along each axis (3.5 dx for a tile of 8 x 8 cells), the linear model is therefore off by at most
 // |c_scale| h^2 / Rmin^2, Rmin the least r over the block.  A ray at fan-angle offset g
 // from a cell centre passes r sin|g| from it, so the rays that meet the cell lie within
 // asin(rs dx / Rmin) <= z (1 + z^2), z = rs dx / Rmin, of its fan angle (rs the cell's
 // support radius, below); the half-width adds the model's error and the atan bound to
 // that, so every cell's range holds every column whose ray meets the cell.  One lane
-// evaluates a view's model; the 16 lanes of the block read it with shuffles.
+// evaluates a view's model for all of the tile's cells.
 struct BlockCand {
     float cf, gx, gy, hw;  // centre column, d cf / dx, d cf / dy (per mm), half-width
     float dx, dy, spread;  // ray direction at the centre; a bound on how far any candidate's differs
@@ -439,8 +439,8 @@ __global__ __launch_bounds__(kAdjThreads) void fp_adjoint_kernel(FpaArgs A)
 // ci..ci+1 and cj..cj+1 (samples inside it interpolate between those four pixels).  Per
 // view and candidate ray (lines within half a cell diagonal of the cell centre) it finds
 // the ray's samples inside the cell: along each axis the samples before boundary b number
-// ceil((b - u0) / du) (du > 0; floor + 1 for du < 0), evaluated by the same expression in
-// both cells that share b, so the cells partition every ray's samples exactly.  The sums
+// ceil((b - u0) / du) in either direction, evaluated by the same expression in both cells
+// that share b, so the cells partition every ray's samples exactly.  The sums
 // over those n samples of 1, the u- and w-fractions and their products (fractions
 // ta + j du, tm + j dw) are closed-form, as in the forward kernel's cell walk, and
 // accumulate (FP32) times the ray's value per slice; at the end they give the four corner
@@ -518,7 +518,7 @@ __device__ __forceinline__ bool cell_in_fov(const FpaArgs &A, float fci, float f
 }
 
 // A workgroup owns a tile of 8 x 8 cells, one per lane, and its four waves a quarter of the views
-// each (their sums meet in LDS at the end), so that small images fill the chip too.  A wave runs
+// each (their sums meet in LDS at the end, see cell_combine), so that small images fill the chip too.  A wave runs
 // without workgroup barriers: the columns around its candidate rays are staged by the wave, for
 // itself, in 64 LDS slots (the windows of 4, 3, 2 or 1 views, 16, 21, 32 or 64 columns wide, as
 // the tile's geometry in the current group of views needs), each slot holding a ray's record and
@@ -534,9 +534,9 @@ __device__ __forceinline__ bool cell_in_fov(const FpaArgs &A, float fci, float f
 // Bound: VALU issue (0.7 of it, a third of the instructions issued in pairs): per wave and view
 // about 2.15 candidates (1.55 rays meet a cell at 512 x 512 / 888 columns) of 25 instructions and
 // 4 S multiply-adds, and 30 for the model, the staging and the loop.  Measured on 512 x 512 pixels, 984
-// views, 888 columns: 1 slice 940 -> 603 us, 4 slices 1.30 ms -> 835 us (with the rays read by every
-// cell from global memory, and staged per workgroup between barriers); 16 slices 2.0 -> 1.78 ms;
-// 256 x 256, 360 views, 512 columns: 1 slice 162 -> 115 us, 4 slices 614 -> 145 us; 104 x 104, 147
+// views, 888 columns: 1 slice 940 -> 630 us, 4 slices 1.30 ms -> 829 us (with the rays read by every
+// cell from global memory, and staged per workgroup between barriers); 16 slices 2.0 -> 1.75 ms;
+// 256 x 256, 360 views, 512 columns: 1 slice 162 -> 117 us, 4 slices 614 -> 151 us; 104 x 104, 147
 // views: 81 -> 19 us.  Tiles of 16 x 16 cells (four waves side by side) have less overlap (1.14
 // against 1.31 cells per pixel) and measured the same within 5% at 512 x 512 (596 us for 1 slice) and
 // slower on smaller images (156 us at 256 x 256).
@@ -1056,8 +1056,8 @@ fbct_status launch_fp_adjoint(const fbct_plan &p, const DeviceTables &t, const v
     fbct_status st = FBCT_OK;
     if (adj_cells_fit(A.far_x, A.far_y)) {
         // Groups of 16 slices, the rest in groups of the next size up, padded with the last slice
-        // (512 x 512: 1, 2, 4, 8, 16 slices take 603, 656, 835, 1117, 1780 us, so that 11 to 15 go
-        // as 16, but 9 and 10 as 8 and the rest); or all slices in one launch of one group size,
+        // (512 x 512: 1, 2, 4, 8, 16 slices take 630, 671, 829, 1139, 1747 us, and 603, 656, 835, 1117,
+        // 1780 when the costs below were taken, so that 11 to 15 go as 16, but 9 and 10 as 8 and the rest); or all slices in one launch of one group size,
         // where the costs say so: a launch costs about its group's time on the tiles times (its
         // workgroups + 800), 800 standing for the time a launch takes that does not fill the chip
         // (64 x 64 over 90 views, 9 slices: 8 and 1 44 us, pairs 21; 73 x 73 over 102, 41 slices:

@@ -26,6 +26,11 @@
  * must not overlap: kernels read one while other workgroups write the other, so an
  * overlap is refused with FBCT_ERR_INVALID_ARGUMENT before any device work.
  *
+ * A slice's (volume's) result has the same bits whatever others share the call in
+ * fbct_fp_adjoint, fbct_bp_adjoint, fbct_fbp_backproject_adjoint, the batch's operators
+ * and the cone operators.  In fbct_fp, fbct_bp, fbct_fbp and fbct_fbp_backproject the
+ * order of its sums goes with the number of slices, so bits may differ at rounding level.
+ *
  * Errors are returned as fbct_status; nothing ever exits the process (the reference
  * exits through checkCudaErrors, FP/transform.cu:4).  fbct_last_error() gives a
  * thread-local message for the last failing call on the calling thread.
@@ -167,9 +172,9 @@ fbct_status fbct_fp_residual(fbct_plan *plan, const void *image, int image_dtype
 
 /* Exact matched adjoint of fbct_fp (transpose of the same interpolation weights).
  * sino -> image.  No reference counterpart (the reference has no gradient).  A NaN or
- * infinity reaches the pixels that its ray's samples touch; where samples lie outside
- * the cells between pixel centres -1 and n (2 rFOV/dx - n + 1/2 >= 1) or nX != nY it
- * may reach pixels beside the ray too. */
+ * infinity reaches the pixels that its ray's samples touch; where samples lie beyond the
+ * last cells (2 rFOV/dx - n + 1/2 >= 1 for n = nX or nY) it spreads to every pixel whose
+ * candidate rays include it. */
 fbct_status fbct_fp_adjoint(fbct_plan *plan, const float *sino, float *image, int n_slices,
                             void *stream);
 
