@@ -27,3 +27,14 @@ def test_fp_adjoint(side, views, cols, slices, storage):
         got = plan.fp_adjoint(y[:n])
         for s in range(min(n, slices)):
             assert torch.equal(got[s], plan.fp_adjoint(y[s:s + 1])[0]), (n, s)
+
+
+# images of fewer rows than columns: per-pixel gathers, in groups of 1, 2, 4, 8 and 16 slices
+@pytest.mark.parametrize("side,ny,views,cols,slices", [
+    (60, 47, 30, 80, 3), (260, 200, 21, 300, 10), (400, 300, 18, 350, 12), (512, 400, 9, 300, 11), (512, 400, 9, 300, 18)])
+def test_fp_adjoint_gather(side, ny, views, cols, slices):
+    plan = _plan(side, views, cols, ny=ny)
+    y = torch.randn((slices,) + plan.sino_shape, generator=torch.Generator().manual_seed(side)).cuda()
+    got = plan.fp_adjoint(y)
+    for s in sorted({0, slices // 2, slices - 1}):
+        assert torch.equal(got[s], plan.fp_adjoint(y[s:s + 1])[0]), s
